@@ -1,11 +1,9 @@
-// Batched dense decompositions of the block matrices of a block-sparse
-// tensor, in FP64 and complex128: SVD by one-sided block Jacobi, QR by
-// Householder reflections.  They replace MatSVD (framework/hp_numeric/
-// lapack.h:41-82 gesvd, GPU :811-1011) and MatQR (lapack.h:332-487 geqrf +
-// orgqr/ungqr) called once per block matrix by DataBlkDecompSVD /
-// DataBlkDecompQR (qltensor/blk_spar_data_ten/data_blk_operations.h:630-663,
-// 1028-1046); here every block matrix of the tensor is decomposed in one
-// batched launch sequence.
+// Batched SVD of the block matrices of a block-sparse tensor, in FP64 and
+// complex128, by one-sided block Jacobi.  It replaces MatSVD (framework/
+// hp_numeric/lapack.h:41-82 gesvd, GPU :811-1011) called once per block matrix
+// by DataBlkDecompSVD (qltensor/blk_spar_data_ten/data_blk_operations.h:
+// 630-663); here every block matrix of the tensor is decomposed in one batched
+// launch sequence.
 //
 // SVD.  The working matrix X is A (rows >= cols) or A^H (rows < cols), stored
 // column-major so that columns are contiguous; V starts as the identity.  The
@@ -26,71 +24,16 @@
 // whose sweep rotates nothing has converged; then sigma_j = |X_j|,
 // U_j = X_j / sigma_j (zero when sigma_j = 0) and A = U diag(sigma) V^H,
 // sorted by decreasing sigma (ties by column).
-//
-// QR.  One workgroup per matrix runs the unblocked Householder QR with
-// LAPACK's reflector convention (xLARFG: beta = -sign(Re alpha) * |(alpha, x)|,
-// tau = (beta - alpha) / beta, v = x / (alpha - beta); no reflection when x = 0
-// and alpha is real), so R has the same diagonal signs as geqrf, then forms
-// Q = H_0 ... H_{k-1} I[:, :k] as orgqr / ungqr do.
 
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
-#include "qlt_internal.h"
+#include "block_dense.h"
+
+using namespace qlt::dense;
 
 namespace {
-
-struct cplx {
-  double x, y;
-};
-
-__device__ __forceinline__ double re_(double a) { return a; }
-__device__ __forceinline__ double re_(cplx a) { return a.x; }
-__device__ __forceinline__ double conj_(double a) { return a; }
-__device__ __forceinline__ cplx conj_(cplx a) { return {a.x, -a.y}; }
-__device__ __forceinline__ double mul_(double a, double b) { return a * b; }
-__device__ __forceinline__ cplx mul_(cplx a, cplx b) { return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-// conj(a) * b
-__device__ __forceinline__ double cmul_(double a, double b) { return a * b; }
-__device__ __forceinline__ cplx cmul_(cplx a, cplx b) { return {a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x}; }
-__device__ __forceinline__ double add_(double a, double b) { return a + b; }
-__device__ __forceinline__ cplx add_(cplx a, cplx b) { return {a.x + b.x, a.y + b.y}; }
-__device__ __forceinline__ double sub_(double a, double b) { return a - b; }
-__device__ __forceinline__ cplx sub_(cplx a, cplx b) { return {a.x - b.x, a.y - b.y}; }
-__device__ __forceinline__ double scl_(double s, double a) { return s * a; }
-__device__ __forceinline__ cplx scl_(double s, cplx a) { return {s * a.x, s * a.y}; }
-__device__ __forceinline__ double abs2_(double a) { return a * a; }
-__device__ __forceinline__ double abs2_(cplx a) { return a.x * a.x + a.y * a.y; }
-template <typename T> __device__ __forceinline__ T zero_();
-template <> __device__ __forceinline__ double zero_<double>() { return 0.0; }
-template <> __device__ __forceinline__ cplx zero_<cplx>() { return {0.0, 0.0}; }
-template <typename T> __device__ __forceinline__ T one_();
-template <> __device__ __forceinline__ double one_<double>() { return 1.0; }
-template <> __device__ __forceinline__ cplx one_<cplx>() { return {1.0, 0.0}; }
-// unit phase of g (|g| > 0), conjugated: e^{-i arg g}, from 1 / |g|
-__device__ __forceinline__ double uphase_conj_inv(double g, double inv) { return g * inv; }
-__device__ __forceinline__ cplx uphase_conj_inv(cplx g, double inv) { return {g.x * inv, -g.y * inv}; }
-// complex reciprocal
-__device__ __forceinline__ double recip_(double a) { return 1.0 / a; }
-__device__ __forceinline__ cplx recip_(cplx a) {
-  const double d = a.x * a.x + a.y * a.y;
-  return {a.x / d, -a.y / d};
-}
-
-template <bool C> struct ElemOf { using T = double; };
-template <> struct ElemOf<true> { using T = cplx; };
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ double shfl_(double v, int src) { return __shfl(v, src); }
-__device__ __forceinline__ cplx shfl_(cplx v, int src) { return {__shfl(v.x, src), __shfl(v.y, src)}; }
-__device__ __forceinline__ double wave_max(double v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-  return v;
-}
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
@@ -610,154 +553,6 @@ __global__ void __launch_bounds__(kThreads) k_svd_finish(const SvdMat *mats, con
   }
 }
 
-// ---- QR ----
-
-struct QrMat {
-  int64_t m, n, k;
-  int64_t w_off;      // W: column-major m x n (becomes R and the reflectors)
-  int64_t q_off_ws;   // Qw: column-major m x k
-  int64_t t_off;      // tau (k elements)
-  int64_t a_off, q_off, r_off;
-};
-
-template <typename T>
-__device__ __forceinline__ double block_sum(double v, double *red) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  const double s = red[0] + red[1] + red[2] + red[3];
-  __syncthreads();
-  return s;
-}
-
-template <bool C>
-__global__ void __launch_bounds__(kThreads) k_qr(const QrMat *mats, const void *a_, void *ws_, void *q_, void *r_) {
-  using T = typename ElemOf<C>::T;
-  __shared__ double sRed[kWaves];
-  __shared__ T sTau, sScale;
-  const QrMat mt = mats[blockIdx.x];
-  const T *A = static_cast<const T *>(a_) + mt.a_off;
-  T *Wm = static_cast<T *>(ws_) + mt.w_off;
-  T *Qw = static_cast<T *>(ws_) + mt.q_off_ws;
-  T *tau = static_cast<T *>(ws_) + mt.t_off;
-  const int64_t m = mt.m, n = mt.n, k = mt.k;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t e = threadIdx.x; e < m * n; e += kThreads) {
-    const int64_t j = e / m, i = e - j * m;
-    Wm[e] = A[i * n + j];
-  }
-  __syncthreads();
-  for (int64_t j = 0; j < k; ++j) {
-    T *col = Wm + j * m;
-    double part = 0.0;
-    for (int64_t i = j + 1 + threadIdx.x; i < m; i += kThreads) part += abs2_(col[i]);
-    const double xn2 = block_sum<T>(part, sRed);
-    if (threadIdx.x == 0) {
-      const T alpha = col[j];
-      T t = zero_<T>(), sc = zero_<T>();
-      const double ai = C ? (abs2_(alpha) - re_(alpha) * re_(alpha)) : 0.0;   // (Im alpha)^2
-      if (!(xn2 == 0.0 && ai == 0.0)) {
-        const double nrm = sqrt(abs2_(alpha) + xn2);
-        const double beta = re_(alpha) >= 0.0 ? -nrm : nrm;
-        T bt = zero_<T>();
-        bt = add_(bt, scl_(beta, one_<T>()));
-        t = scl_(1.0 / beta, sub_(bt, alpha));
-        sc = recip_(sub_(alpha, bt));
-        col[j] = bt;
-      }
-      sTau = t;
-      sScale = sc;
-      tau[j] = t;
-    }
-    __syncthreads();
-    const T t = sTau;
-    if (abs2_(t) == 0.0) continue;
-    const T sc = sScale;
-    for (int64_t i = j + 1 + threadIdx.x; i < m; i += kThreads) col[i] = mul_(sc, col[i]);
-    __syncthreads();
-    // trailing columns: x <- H^H x = x - conj(tau) v (v^H x)
-    const T ct = conj_(t);
-    for (int64_t c = j + 1 + wave; c < n; c += kWaves) {
-      T *x = Wm + c * m;
-      T d = zero_<T>();
-      for (int64_t i = j + lane; i < m; i += 64) {
-        const T vi = (i == j) ? one_<T>() : col[i];
-        d = add_(d, cmul_(vi, x[i]));
-      }
-      if constexpr (C) {
-        d.x = wave_sum(d.x);
-        d.y = wave_sum(d.y);
-      } else {
-        d = wave_sum(d);
-      }
-      const T f = mul_(ct, d);
-      for (int64_t i = j + lane; i < m; i += 64) {
-        const T vi = (i == j) ? one_<T>() : col[i];
-        x[i] = sub_(x[i], mul_(vi, f));
-      }
-    }
-    __syncthreads();
-  }
-  // R (k x n), upper triangle of W
-  T *R = static_cast<T *>(r_) + mt.r_off;
-  for (int64_t e = threadIdx.x; e < k * n; e += kThreads) {
-    const int64_t i = e / n, c = e - i * n;
-    R[e] = c >= i ? Wm[c * m + i] : zero_<T>();
-  }
-  // Q = H_0 ... H_{k-1} I[:, :k]
-  for (int64_t e = threadIdx.x; e < m * k; e += kThreads) {
-    const int64_t c = e / m, i = e - c * m;
-    Qw[e] = (i == c) ? one_<T>() : zero_<T>();
-  }
-  __syncthreads();
-  for (int64_t j = k - 1; j >= 0; --j) {
-    const T t = tau[j];
-    if (abs2_(t) == 0.0) continue;
-    const T *v = Wm + j * m;
-    for (int64_t c = j + wave; c < k; c += kWaves) {
-      T *x = Qw + c * m;
-      T d = zero_<T>();
-      for (int64_t i = j + lane; i < m; i += 64) {
-        const T vi = (i == j) ? one_<T>() : v[i];
-        d = add_(d, cmul_(vi, x[i]));
-      }
-      if constexpr (C) {
-        d.x = wave_sum(d.x);
-        d.y = wave_sum(d.y);
-      } else {
-        d = wave_sum(d);
-      }
-      const T f = mul_(t, d);
-      for (int64_t i = j + lane; i < m; i += 64) {
-        const T vi = (i == j) ? one_<T>() : v[i];
-        x[i] = sub_(x[i], mul_(vi, f));
-      }
-    }
-    __syncthreads();
-  }
-  T *Q = static_cast<T *>(q_) + mt.q_off;
-  for (int64_t e = threadIdx.x; e < m * k; e += kThreads) {
-    const int64_t i = e / k, c = e - i * k;
-    Q[e] = Qw[c * m + i];
-  }
-}
-
-struct DevBuf {
-  void *p = nullptr;
-  ~DevBuf() {
-    if (p != nullptr) (void)hipFree(p);
-  }
-};
-
-qlt_status check_shapes(const char *who, int64_t n_mats, const int64_t *rows, const int64_t *cols) {
-  QLT_CHECK_ARG(n_mats >= 0, std::string(who) + ": negative matrix count");
-  QLT_CHECK_ARG(n_mats == 0 || (rows != nullptr && cols != nullptr), std::string(who) + ": null shape array");
-  QLT_CHECK_ARG(n_mats < (int64_t(1) << 31), std::string(who) + ": too many matrices");
-  for (int64_t i = 0; i < n_mats; ++i)
-    QLT_CHECK_ARG(rows[i] >= 1 && cols[i] >= 1, std::string(who) + ": matrix " + std::to_string(i) + " is empty");
-  return QLT_OK;
-}
-
 template <bool C>
 qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, const void *a, const int64_t *a_offsets,
                     void *u, const int64_t *u_offsets, double *s, const int64_t *s_offsets, void *vt,
@@ -890,54 +685,6 @@ qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, co
   return QLT_OK;
 }
 
-template <bool C>
-qlt_status qr_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, const void *a, const int64_t *a_offsets,
-                   void *q, const int64_t *q_offsets, void *r, const int64_t *r_offsets, hipStream_t st) {
-  const size_t esz = C ? 16 : 8;
-  std::vector<QrMat> mats(static_cast<size_t>(n_mats));
-  int64_t ws = 0;
-  for (int64_t i = 0; i < n_mats; ++i) {
-    QrMat &mt = mats[static_cast<size_t>(i)];
-    mt.m = rows[i];
-    mt.n = cols[i];
-    mt.k = std::min(rows[i], cols[i]);
-    mt.w_off = ws;
-    ws += mt.m * mt.n;
-    mt.q_off_ws = ws;
-    ws += mt.m * mt.k;
-    mt.t_off = ws;
-    ws += mt.k;
-    mt.a_off = a_offsets[i];
-    mt.q_off = q_offsets[i];
-    mt.r_off = r_offsets[i];
-  }
-  DevBuf d_ws, d_mats;
-  QLT_HIP(hipMalloc(&d_ws.p, std::max<size_t>(1, static_cast<size_t>(ws) * esz)));
-  QLT_HIP(hipMalloc(&d_mats.p, sizeof(QrMat) * mats.size()));
-  QLT_HIP(hipMemcpyAsync(d_mats.p, mats.data(), sizeof(QrMat) * mats.size(), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_qr<C>, dim3(static_cast<unsigned>(n_mats)), dim3(kThreads), 0, st,
-                     static_cast<const QrMat *>(d_mats.p), a, d_ws.p, q, r);
-  QLT_HIP(hipGetLastError());
-  QLT_HIP(hipStreamSynchronize(st));
-  return QLT_OK;
-}
-
-// Single-precision element types: the block matrices are widened to FP64
-// (complex128) device buffers, decomposed there, and the factors rounded
-// back; `ext` is the extent (elements) of a buffer addressed by offsets.
-int64_t extent(int64_t n, const int64_t *offs, const int64_t *r, const int64_t *c) {
-  int64_t e = 0;
-  for (int64_t i = 0; i < n; ++i) e = std::max(e, offs[i] + r[i] * c[i]);
-  return e;
-}
-
-struct DevTmp {
-  void *p = nullptr;
-  ~DevTmp() {
-    if (p != nullptr) (void)hipFree(p);
-  }
-};
-
 }  // namespace
 
 extern "C" {
@@ -963,7 +710,7 @@ qlt_status qlt_block_svd(int32_t dtype, int64_t n_mats, const int64_t *rows, con
     const int64_t na = extent(n_mats, a_offsets, rows, cols);
     const int64_t nu = extent(n_mats, u_offsets, rows, kk.data());
     const int64_t nv = extent(n_mats, vt_offsets, kk.data(), cols);
-    DevTmp wa, wu, wv;
+    DevBuf wa, wu, wv;
     QLT_HIP(hipMalloc(&wa.p, std::max<int64_t>(1, na) * esz));
     QLT_HIP(hipMalloc(&wu.p, std::max<int64_t>(1, nu) * esz));
     QLT_HIP(hipMalloc(&wv.p, std::max<int64_t>(1, nv) * esz));
@@ -980,41 +727,6 @@ qlt_status qlt_block_svd(int32_t dtype, int64_t n_mats, const int64_t *rows, con
                            qlt::as_stream(stream));
   return svd_impl<true>(n_mats, rows, cols, a, a_offsets, u, u_offsets, s, s_offsets, vt, vt_offsets, sweeps,
                         qlt::as_stream(stream));
-}
-
-qlt_status qlt_block_qr(int32_t dtype, int64_t n_mats, const int64_t *rows, const int64_t *cols, const void *a,
-                        const int64_t *a_offsets, void *q, const int64_t *q_offsets, void *r,
-                        const int64_t *r_offsets, void *stream) {
-  QLT_REQUIRE_INIT();
-  QLT_CHECK_ARG(qlt::valid_dtype(dtype), "qlt_block_qr: bad dtype");
-  QLT_TRY(check_shapes("qlt_block_qr", n_mats, rows, cols));
-  if (n_mats == 0) return QLT_OK;
-  QLT_CHECK_ARG(a != nullptr && q != nullptr && r != nullptr, "qlt_block_qr: null data pointer");
-  QLT_CHECK_ARG(a_offsets != nullptr && q_offsets != nullptr && r_offsets != nullptr,
-                "qlt_block_qr: null offset array");
-  QLT_CHECK_ARG(!qlt::stream_capturing(qlt::as_stream(stream)), "qlt_block_qr: not capturable (allocates)");
-  if (qlt::dtype_is_single(dtype)) {
-    const int32_t wide = dtype == QLT_F32 ? QLT_F64 : QLT_C128;
-    const int64_t esz = qlt::dtype_bytes(wide);
-    std::vector<int64_t> kk(static_cast<size_t>(n_mats));
-    for (int64_t i = 0; i < n_mats; ++i) kk[i] = std::min(rows[i], cols[i]);
-    const int64_t na = extent(n_mats, a_offsets, rows, cols);
-    const int64_t nq = extent(n_mats, q_offsets, rows, kk.data());
-    const int64_t nr = extent(n_mats, r_offsets, kk.data(), cols);
-    DevTmp wa, wq, wr;
-    QLT_HIP(hipMalloc(&wa.p, std::max<int64_t>(1, na) * esz));
-    QLT_HIP(hipMalloc(&wq.p, std::max<int64_t>(1, nq) * esz));
-    QLT_HIP(hipMalloc(&wr.p, std::max<int64_t>(1, nr) * esz));
-    QLT_TRY(qlt_convert(dtype, wide, na, a, wa.p, stream));
-    QLT_TRY(qlt_block_qr(wide, n_mats, rows, cols, wa.p, a_offsets, wq.p, q_offsets, wr.p, r_offsets, stream));
-    QLT_TRY(qlt_convert(wide, dtype, nq, wq.p, q, stream));
-    QLT_TRY(qlt_convert(wide, dtype, nr, wr.p, r, stream));
-    QLT_HIP(hipStreamSynchronize(qlt::as_stream(stream)));
-    return QLT_OK;
-  }
-  if (dtype == QLT_F64)
-    return qr_impl<false>(n_mats, rows, cols, a, a_offsets, q, q_offsets, r, r_offsets, qlt::as_stream(stream));
-  return qr_impl<true>(n_mats, rows, cols, a, a_offsets, q, q_offsets, r, r_offsets, qlt::as_stream(stream));
 }
 
 }  // extern "C"
