@@ -7,15 +7,17 @@
 // and then issues one BLAS call C_blk = A'(m x k) B'(k x n) + beta C_blk
 // (hp_numeric::MatMultiply, framework/hp_numeric/blas_level3.h:35-56,798-856).
 // Here one launch per tile class covers the whole plan.  Each workgroup owns
-// one TM x TN tile (64 or 32 each way) of one output block, or one k-slice of
-// it, and walks every task of that block, so the per-block beta chain (0 for
-// the first task, 1 after) becomes a single write of the finished tile (or of
-// its slices' sum).  Narrow outputs (n <= 16) go to a row-streaming kernel.  The transposes are never materialised: the
-// prologue gathers A'(i, p) = A[a_off + row_off(i) + col_off(p)] straight
+// one TM x TN tile (64 or 32 each way; 32 x 16 for n <= 16) of one output
+// block, or one k-slice of it, and walks every task of that block, so the
+// per-block beta chain (0 for the first task, 1 after) becomes a single write
+// of the finished tile (or of its slices' sum).  Outputs of n <= 4 go to a
+// row-streaming path, or to row panels.  The transposes are never
+// materialised: the prologue gathers A'(i, p) = A[a_off + row_off(i) + col_off(p)] straight
 // from the original block layout through per-tile offset tables, staging the
 // k-chunk in LDS, with the thread mapping chosen so that the block's
 // innermost memory axis is read contiguously.
 
+#include <algorithm>
 #include <cstdio>
 #include <memory>
 #include <type_traits>
@@ -160,7 +162,6 @@ __device__ __forceinline__ void tile_epilogue(const Seg &seg, int r0, int c0, co
 
 constexpr int KC = kKChunk;   // plan step: k-chunk of 16
 constexpr double kPanelStreamBytes = 256.0 * 1024 * 1024;   // the MI355X last-level (Infinity) cache
-constexpr int kRealUnits = 1; // plan steps staged per pipeline step (FP64); 2 halves the occupancy and measured slower
 
 // Tile order for the XCDs: workgroups are dispatched to the 8 XCDs round
 // robin, so workgroup b runs on XCD b % 8.  Mapping b to logical tile
@@ -186,24 +187,25 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 //      otherwise    -> r = tid % TM, cols tid / TM + (256 / TM) q;
 //   B' n-contiguous -> c = tid % TN, rows tid / TN + (256 / TN) q;
 //      otherwise    -> p = tid & 15, cols (tid >> 4) + 16 q.
-template <bool CPLX, int TMv, int TNv, typename E = double>
-__global__ __launch_bounds__(256) void k_grouped_gemm_f64(
-    const Tile *__restrict__ tiles, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
-    const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout L,
+template <bool CPLX, int TMv, int TNv>
+struct GroupedShared {
+  static constexpr int P = CPLX ? 2 : 1, KCv = KC;
+  double As[2][P][KCv][TMv + 1];
+  double Bs[2][P][KCv][TNv + 1];
+};
+template <bool CPLX, int TMv, int TNv, typename E>
+__device__ __forceinline__ void grouped_tile(
+    char *smem, const Tile tile, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
+    const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout &L,
     const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part,
     double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
-  // k extent per pipeline step: U plan steps of 16 (FP64 stages 32 k per
-  // step; complex128, whose LDS tiles are twice as large, stages 16)
-  constexpr int U = CPLX ? 1 : kRealUnits;
-  constexpr int KCv = KC * U;
-  constexpr int QA0 = TMv / 16, QB0 = TNv / 16;        // elements per thread per 16 k
-  constexpr int QA = QA0 * U, QB = QB0 * U;            // elements per thread per step
+  constexpr int KCv = KC;                              // k extent per pipeline step
+  constexpr int QA = TMv / 16, QB = TNv / 16;          // elements per thread per step
   constexpr int BM = TMv / 32, BN = TNv / 32;          // MFMA blocks per wave
-  __shared__ double As[2][P][KCv][TMv + 1];
-  __shared__ double Bs[2][P][KCv][TNv + 1];
+  auto &As = reinterpret_cast<GroupedShared<CPLX, TMv, TNv> *>(smem)->As;
+  auto &Bs = reinterpret_cast<GroupedShared<CPLX, TMv, TNv> *>(smem)->Bs;
 
-  const Tile tile = tiles[xcd_tile(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   const Seg seg = segs[tile.seg];
   const int i0 = tile.tm * TMv, j0 = tile.tn * TNv;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -223,10 +225,10 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
       acc_s[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
     }
 
-  auto a_r = [&](int q) { return akf ? (tid >> 4) + 16 * (q % QA0) : tid % TMv; };
-  auto a_p = [&](int q) { return akf ? (tid & 15) + 16 * (q / QA0) : tid / TMv + (256 / TMv) * q; };
-  auto b_c = [&](int q) { return bnf ? tid % TNv : (tid >> 4) + 16 * (q % QB0); };
-  auto b_p = [&](int q) { return bnf ? tid / TNv + (256 / TNv) * q : (tid & 15) + 16 * (q / QB0); };
+  auto a_r = [&](int q) { return akf ? (tid >> 4) + 16 * q : tid % TMv; };
+  auto a_p = [&](int q) { return akf ? tid & 15 : tid / TMv + (256 / TMv) * q; };
+  auto b_c = [&](int q) { return bnf ? tid % TNv : (tid >> 4) + 16 * q; };
+  auto b_p = [&](int q) { return bnf ? tid / TNv + (256 / TNv) * q : tid & 15; };
 
   // Per task: the row offsets of the A' elements and column offsets of the
   // B' elements this thread loads.  A block whose permuted view is plain
@@ -334,14 +336,10 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
   };
 
   // ---- pipeline over this tile's steps of the (task, k-chunk) sequence ----
-  // A step stages up to U plan steps of 16 k, never crossing a task or the
-  // end of the tile's slice; k beyond the step's end loads as zero.
-  auto span_of = [&](const ExecTask &e, int kk_, int left_) {
-    return min(U, min((e.k - kk_ + KC - 1) / KC, left_));
-  };
-
+  // A step stages 16 k, never crossing a task; k beyond the task's end loads
+  // as zero.
   const bool seg_affine = (seg.flags & (kSegAColAffine | kSegBRowAffine)) == (kSegAColAffine | kSegBRowAffine);
-  if (seg_affine && U == 1) {
+  if (seg_affine) {
     // Output block whose every task reads A and B blocks that are affine in
     // k: A' element (r, p) at a_off + roff(r) + p * cs, B' element (p, c) at
     // b_off + p * rs + coff(c) (plain blocks: roff = r*k, cs = 1, rs = n,
@@ -448,37 +446,33 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
     int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks;
     ExecTask et = exec[t];
     task_rows(ga[et.a_blk], gb[et.b_blk], et);
-    int sp = span_of(et, kk, left);
-    fetch(et, ga[et.a_blk], gb[et.b_blk], kk, min(et.k, kk + KC * sp));
+    fetch(et, ga[et.a_blk], gb[et.b_blk], kk, min(et.k, kk + KC));
     stage(0);
     __syncthreads();
     int buf = 0;
     while (left > 0) {
-      const int left2 = left - sp;
-      int t2 = t, kk2 = kk + KC * sp;
+      const int left2 = left - 1;
+      int t2 = t, kk2 = kk + KC;
       if (kk2 >= et.k) {
         t2 = t + 1;
         kk2 = 0;
       }
       const bool has_next = left2 > 0;
       ExecTask et2 = et;
-      int sp2 = 0;
       if (has_next) {
         if (t2 != t) {
           et2 = exec[t2];
           task_rows(ga[et2.a_blk], gb[et2.b_blk], et2);
         }
-        sp2 = span_of(et2, kk2, left2);
-        fetch(et2, ga[et2.a_blk], gb[et2.b_blk], kk2, min(et2.k, kk2 + KC * sp2));
+        fetch(et2, ga[et2.a_blk], gb[et2.b_blk], kk2, min(et2.k, kk2 + KC));
       }
-      compute(buf, min(et.k - kk, KC * sp));
+      compute(buf, min(et.k - kk, KC));
       if (has_next) stage(buf ^ 1);
       __syncthreads();
       t = t2;
       kk = kk2;
       et = et2;
       left = left2;
-      sp = sp2;
       buf ^= 1;
     }
   }
@@ -495,7 +489,7 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
       }
   }
 
-  // ---- a k-slice stores its unscaled partial sum, in the thread's own order ----
+  // ---- a k-slice stores its unscaled partial sum, row-major over the tile ----
   if (tile.part >= 0) {
     double *pp = part + static_cast<int64_t>(tile.part) * (TMv * TNv * P);
 #pragma unroll
@@ -504,7 +498,7 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
       for (int nt = 0; nt < BN; ++nt)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int e = ((mt * BN + nt) * 4 + v) * 256 + tid;
+          const int e = (wm + 16 * mt + 4 * v + lk) * TNv + wn + 16 * nt + lr;
           pp[e] = acc[mt][nt][v];
           if (CPLX) pp[TMv * TNv + e] = acc_i[mt][nt][v];
         }
@@ -516,47 +510,314 @@ __global__ __launch_bounds__(256) void k_grouped_gemm_f64(
   tile_epilogue<CPLX, BM, BN, E>(seg, i0 + wm + lk, j0 + wn + lr, acc, acc_i, C, alpha_r, alpha_i, beta_r, beta_i);
 }
 
-// Sum of the k-slices of one output tile, in slice order, then the usual
-// epilogue.  The thread-to-element map is the MFMA kernel's, so thread tid
-// reads exactly the partial elements it would have held.
-template <bool CPLX, int TMv, int TNv, typename E = double>
-__global__ __launch_bounds__(256) void k_reduce_slices(const ReduceItem *__restrict__ items,
-                                                       const Seg *__restrict__ segs,
-                                                       const double *__restrict__ part, E *__restrict__ C,
-                                                       double alpha_r, double alpha_i, double beta_r, double beta_i) {
+// Narrow outputs (4 < n <= 16): one workgroup per 32 x 16 tile (two MFMA
+// blocks of 16 x 16) or k-slice of it, its four waves taking every fourth
+// 16-k chunk of the tile's (task, chunk) sequence and meeting in LDS at the
+// end (sums in wave order).  The operand fragments are loaded from global
+// memory straight into the registers the MFMA reads (lane lr = lane % 16 holds
+// A' row / B' column lr, lk = lane / 16 the contracted index), so no wave waits
+// for another inside the loop, and the loads of one stage are issued before
+// the MFMAs of the previous one (two register sets).
+//   What bounds it is latency: few tiles, each a long chain of chunks.  A row
+// kernel with one thread per row and an LDS chunk of B' per step walked the
+// chain alone, about 1 us per 16 k: a complex64 contraction onto n <= 16
+// outputs 143 -> 27 us, the n <= 16 tiles of a lognormal FP64 matvec 46 -> 15 us
+// per contraction.  The same unstaged form for n > 16 is slower than the LDS
+// tiles (D = 4096 complex128 matvec 1.23 -> 1.41 ms): there the fragments'
+// uncoalesced lines bound it, so it stays with this class.
+//   Full stages of the types of at most 8 bytes per element give lane (lr, lk)
+// the KS consecutive contracted indices KS lk .. KS lk + KS - 1, so that an
+// operand contiguous in k is read in 16-byte pieces; complex128 and a task's
+// last partial stage use 4 s + lk.  The order of the contracted indices is
+// free as long as both operands follow it.
+//   Rows and columns past the block read the block's first row or column and
+// their results are not stored; contracted indices past the task count zero
+// on both sides.
+constexpr int kNarrowM = 32, kNarrowN = 16, kNarrowWaves = 4;
+
+template <bool CPLX>
+struct NarrowShared {
+  double acc[kNarrowWaves][CPLX ? 2 : 1][2][4][64];
+};
+
+// KS consecutive elements of an operand contiguous in k: 16-byte loads with
+// the element's alignment only.
+template <typename E, bool CPLX, int KS>
+__device__ __forceinline__ void ld_run(const E *p, raw_t<E, CPLX> (&x)[KS]) {
+  static_assert(sizeof(raw_t<E, CPLX>) <= 8, "runs are for elements of at most 8 bytes");
+  typedef E vec __attribute__((ext_vector_type(16 / sizeof(E)), aligned(sizeof(E))));
+  constexpr int PER = 16 / sizeof(raw_t<E, CPLX>);   // elements per load
+  static_assert(KS % PER == 0, "whole 16-byte pieces");
+#pragma unroll
+  for (int i = 0; i < KS / PER; ++i) {
+    const vec v = reinterpret_cast<const vec *>(p)[i];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      if constexpr (CPLX) x[i * PER + j] = raw_t<E, CPLX>{v[2 * j], v[2 * j + 1]};
+      else x[i * PER + j] = v[j];
+    }
+  }
+}
+
+template <bool CPLX, typename E>
+__device__ __forceinline__ void narrow_tile(
+    char *smem, const Tile tile, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
+    const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout &L,
+    const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part,
+    double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
-  constexpr int BM = TMv / 32, BN = TNv / 32;
-  const ReduceItem it = items[blockIdx.x];
-  const Seg seg = segs[it.seg];
-  const int i0 = it.tm * TMv, j0 = it.tn * TNv;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = (w >> 1) * (TMv / 2), wn = (w & 1) * (TNv / 2);
-  const int lr = lane & 15, lk = lane >> 4;
-  // slices outer, elements inner: every slice's loads are independent
-  double sr[BM][BN][4], si[BM][BN][4];
+  constexpr int KW = kNarrowWaves, BM = kNarrowM / 16;
+  constexpr int KS = (CPLX && sizeof(E) == 8) ? 2 : 4;   // k-steps of 4 per stage
+  constexpr int SK = 4 * KS;
+  constexpr bool kLaneRuns = sizeof(E) * P <= 8;
+  using R = raw_t<E, CPLX>;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const Seg seg = segs[tile.seg];
+  const int i0 = tile.tm * kNarrowM;
+  const bool m1_ok = i0 + 16 < seg.m;
+  v4d acc[P][BM];
 #pragma unroll
-  for (int mt = 0; mt < BM; ++mt)
+  for (int q = 0; q < P; ++q)
 #pragma unroll
-    for (int nt = 0; nt < BN; ++nt)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        sr[mt][nt][v] = 0.0;
-        si[mt][nt][v] = 0.0;
+    for (int mt = 0; mt < BM; ++mt) acc[q][mt] = v4d{0.0, 0.0, 0.0, 0.0};
+  R a[2][BM][KS], b[2][KS];
+
+  // position: task t (k extent tk), contracted index kk, chunks left
+  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks - w;
+  int tk = 0;
+  // moves n chunks forward from chunk start kk (which may equal or pass tk)
+  auto skip = [&](int n) {
+    for (;;) {
+      if (kk >= tk) {
+        ++t;
+        tk = exec[t].k;
+        kk = 0;
       }
-  for (int s = 0; s < it.n_parts; ++s) {
-    const double *pp = part + static_cast<int64_t>(it.part0 + s) * (TMv * TNv * P);
+      if (n == 0) break;
+      const int here = (tk - kk + KC - 1) / KC;
+      if (n < here) {
+        kk += KC * n;
+        break;
+      }
+      n -= here;
+      kk = tk;
+    }
+  };
+
+  // per task: element pointers of this lane's rows and column at k = 0, and
+  // how an index k moves them
+  const E *ap[BM], *bp = nullptr;
+  const BlkGather *gA = nullptr, *gB = nullptr;
+  bool a_aff = false, b_aff = false;
+  int cs = 1, rs = 1, cur = -1;
+  auto setup = [&]() {
+    cur = t;
+    const ExecTask et = exec[t];
+    gA = ga + et.a_blk;
+    gB = gb + et.b_blk;
+    const bool a_plain = (seg.flags & kSegAPlain) || gA->plain != 0;
+    const bool b_plain = (seg.flags & kSegBPlain) || gB->plain != 0;
+    a_aff = (seg.flags & kSegAColAffine) || a_plain || gA->caff != 0;
+    b_aff = (seg.flags & kSegBRowAffine) || b_plain || gB->raff != 0;
+    cs = a_plain ? 1 : gA->cstep;
+    rs = b_plain ? seg.n : gB->rstep;
+#pragma unroll
+    for (int mt = 0; mt < BM; ++mt) {
+      int r = i0 + 16 * mt + lr;
+      r = r < seg.m ? r : 0;
+      const int64_t off = a_plain ? static_cast<int64_t>(r) * et.k
+                                  : split_offset(r, gA->rdim, gA->rstr, gA->rmag, gA->rsh, L.a_nr);
+      ap[mt] = A + (et.a_off + off) * P;
+    }
+    const int c = lr < seg.n ? lr : 0;
+    const int64_t off = b_plain ? c : split_offset(c, gB->cdim, gB->cstr, gB->cmag, gB->csh, L.b_nc);
+    bp = B + (et.b_off + off) * P;
+  };
+  auto a_off = [&](int k) -> int64_t {
+    return a_aff ? static_cast<int64_t>(k) * cs : split_offset(k, gA->cdim, gA->cstr, gA->cmag, gA->csh, L.a_nc);
+  };
+  auto b_off = [&](int k) -> int64_t {
+    return b_aff ? static_cast<int64_t>(k) * rs : split_offset(k, gB->rdim, gB->rstr, gB->rmag, gB->rsh, L.b_nr);
+  };
+  // the stage at (t, kk) into register set `s`; returns its valid extent
+  auto load = [&](int s) {
+    if (t != cur) setup();
+    const int kv = tk - kk < SK ? tk - kk : SK;
+    if (kv == SK) {
+      bool a_run = false, b_run = false;
+      if constexpr (kLaneRuns) {
+        a_run = a_aff && cs == 1;
+        b_run = b_aff && rs == 1;
+        if (a_run) {
+          ld_run<E, CPLX, KS>(ap[0] + (kk + KS * lk) * P, a[s][0]);
+          if (m1_ok) ld_run<E, CPLX, KS>(ap[1] + (kk + KS * lk) * P, a[s][1]);
+        }
+        if (b_run) ld_run<E, CPLX, KS>(bp + (kk + KS * lk) * P, b[s]);
+      }
+      if (!a_run) {
+#pragma unroll
+        for (int q = 0; q < KS; ++q) {
+          const int64_t off = a_off(kk + (kLaneRuns ? KS * lk + q : 4 * q + lk)) * P;
+          a[s][0][q] = ld_raw<E, CPLX>(ap[0] + off);
+          if (m1_ok) a[s][1][q] = ld_raw<E, CPLX>(ap[1] + off);
+        }
+      }
+      if (!b_run) {
+#pragma unroll
+        for (int q = 0; q < KS; ++q)
+          b[s][q] = ld_raw<E, CPLX>(bp + b_off(kk + (kLaneRuns ? KS * lk + q : 4 * q + lk)) * P);
+      }
+    } else {
+      // a task's last stage: k = kk + 4 q + lk, the steps beyond it skipped
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        if (4 * q >= kv) continue;
+        const bool ok = 4 * q + lk < kv;
+        const int k = ok ? kk + 4 * q + lk : kk;
+        const int64_t ao = a_off(k) * P;
+        const R x = ld_raw<E, CPLX>(ap[0] + ao), z = ld_raw<E, CPLX>(bp + b_off(k) * P);
+        a[s][0][q] = ok ? x : R{};
+        b[s][q] = ok ? z : R{};
+        if (m1_ok) {
+          const R y = ld_raw<E, CPLX>(ap[1] + ao);
+          a[s][1][q] = ok ? y : R{};
+        }
+      }
+    }
+    return kv;
+  };
+  auto compute = [&](int s, int kv) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
+      if (kv < SK && 4 * q >= kv) continue;
+      const double br = re_of(b[s][q]), bi = im_of(b[s][q]);
+#pragma unroll
+      for (int mt = 0; mt < BM; ++mt) {
+        if (mt == 1 && !m1_ok) continue;
+        const double ar = re_of(a[s][mt][q]);
+        v4d &x = acc[0][mt];
+        x = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, x, 0, 0, 0);
+        if constexpr (CPLX) {
+          // four real products: this class is not bound by them
+          const double ai = im_of(a[s][mt][q]);
+          v4d &y = acc[P - 1][mt];
+          x = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, x, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, y, 0, 0, 0);
+          y = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, y, 0, 0, 0);
+        }
+      }
+    }
+  };
+  // past the stage of extent kv; false when this wave's chunks are done
+  auto advance = [&](int kv) {
+    kk += kv;
+    if (kk < tk && (kk & (KC - 1)) != 0) return true;   // inside a chunk
+    left -= KW;
+    if (left <= 0) return false;
+    skip(KW - 1);
+    return true;
+  };
+  if (left > 0) {
+    tk = exec[t].k;
+    skip(w);
+    int kv0 = load(0);
+    for (;;) {
+      bool more = advance(kv0);
+      int kv1 = 0;
+      if (more) kv1 = load(1);
+      compute(0, kv0);
+      if (!more) break;
+      more = advance(kv1);
+      if (more) kv0 = load(0);
+      compute(1, kv1);
+      if (!more) break;
+    }
+  }
+
+  // wave w takes the accumulator element v = w of every lane, from all waves
+  auto &sAcc = reinterpret_cast<NarrowShared<CPLX> *>(smem)->acc;
+#pragma unroll
+  for (int q = 0; q < P; ++q)
 #pragma unroll
     for (int mt = 0; mt < BM; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < BN; ++nt)
+      for (int v = 0; v < 4; ++v) sAcc[w][q][mt][v][lane] = acc[q][mt][v];
+  __syncthreads();
+  double *pp = tile.part >= 0 ? part + static_cast<int64_t>(tile.part) * (kNarrowM * kNarrowN * P) : nullptr;
+  const bool use_beta = pp == nullptr && (beta_r != 0.0 || beta_i != 0.0);
+  double xr[BM], xi[BM];
+  R old[BM];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int e = ((mt * BN + nt) * 4 + v) * 256 + tid;
-          sr[mt][nt][v] += pp[e];
-          if (CPLX) si[mt][nt][v] += pp[TMv * TNv + e];
-        }
+  for (int mt = 0; mt < BM; ++mt) {
+    xr[mt] = 0.0;
+    xi[mt] = 0.0;
+#pragma unroll
+    for (int g = 0; g < KW; ++g) {
+      xr[mt] += sAcc[g][0][mt][w][lane];
+      if (CPLX) xi[mt] += sAcc[g][P - 1][mt][w][lane];
+    }
+    old[mt] = R{};
+    if (use_beta) {
+      const int row = i0 + 16 * mt + 4 * w + lk;
+      const bool ok = row < seg.m && lr < seg.n;
+      old[mt] = ld_raw<E, CPLX>(C + P * (seg.c_off + (ok ? static_cast<int64_t>(row) * seg.n + lr : 0)));
+    }
   }
-  tile_epilogue<CPLX, BM, BN, E>(seg, i0 + wm + lk, j0 + wn + lr, sr, si, C, alpha_r, alpha_i, beta_r, beta_i);
+#pragma unroll
+  for (int mt = 0; mt < BM; ++mt) {
+    const int lrow = 16 * mt + 4 * w + lk;
+    if (pp != nullptr) {
+      // a k-slice stores its unscaled partial sum, row-major over the tile
+      pp[lrow * kNarrowN + lr] = xr[mt];
+      if (CPLX) pp[kNarrowM * kNarrowN + lrow * kNarrowN + lr] = xi[mt];
+    } else if (i0 + lrow < seg.m && lr < seg.n) {
+      st_scaled<E, CPLX>(C + P * (seg.c_off + static_cast<int64_t>(i0 + lrow) * seg.n + lr), xr[mt], xi[mt], old[mt],
+                         use_beta, alpha_r, alpha_i, beta_r, beta_i);
+    }
+  }
+}
+
+// Sum of the k-slices of one output tile, in slice order, then the usual
+// epilogue: element e of the tile (row-major) in thread e % 256.
+template <bool CPLX, int TMv, int TNv, typename E>
+__device__ __forceinline__ void reduce_slices(const ReduceItem it, const Seg &seg, const double *__restrict__ part,
+                                              E *__restrict__ C, double alpha_r, double alpha_i, double beta_r,
+                                              double beta_i) {
+  constexpr int P = CPLX ? 2 : 1;
+  constexpr int NE = TMv * TNv / 256;
+  const int tid = threadIdx.x;
+  double sr[NE], si[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    sr[u] = 0.0;
+    si[u] = 0.0;
+  }
+  // slices outer, elements inner: every slice's loads are independent
+  for (int s = 0; s < it.n_parts; ++s) {
+    const double *pp = part + static_cast<int64_t>(it.part0 + s) * (TMv * TNv * P);
+#pragma unroll
+    for (int u = 0; u < NE; ++u) {
+      sr[u] += pp[tid + 256 * u];
+      if (CPLX) si[u] += pp[TMv * TNv + tid + 256 * u];
+    }
+  }
+  const bool use_beta = beta_r != 0.0 || beta_i != 0.0;
+  raw_t<E, CPLX> old[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = tid + 256 * u, row = it.tm * TMv + e / TNv, col = it.tn * TNv + e % TNv;
+    const bool ok = row < seg.m && col < seg.n;
+    old[u] = raw_t<E, CPLX>{};
+    if (use_beta) old[u] = ld_raw<E, CPLX>(C + P * (seg.c_off + (ok ? static_cast<int64_t>(row) * seg.n + col : 0)));
+  }
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = tid + 256 * u, row = it.tm * TMv + e / TNv, col = it.tn * TNv + e % TNv;
+    if (row < seg.m && col < seg.n)
+      st_scaled<E, CPLX>(C + P * (seg.c_off + static_cast<int64_t>(row) * seg.n + col), sr[u], si[u], old[u], use_beta,
+                         alpha_r, alpha_i, beta_r, beta_i);
+  }
 }
 
 // Row-streaming kernel for narrow outputs (n <= NMAX): one thread per output
@@ -611,19 +872,25 @@ __device__ __forceinline__ void rows_epilogue(const Seg &seg, int r0, int tid, c
   }
 }
 
-template <bool CPLX, int NMAX, int RPT, typename E = double>
-__global__ __launch_bounds__(256) void k_rows_f64(
-    const Tile *__restrict__ tiles, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
-    const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout L,
+template <bool CPLX, int NMAX>
+struct RowsShared {
+  double Bs[CPLX ? 2 : 1][RK][NMAX];
+  int32_t acol[RK], brow[RK], bcol[NMAX];
+};
+template <bool CPLX, int NMAX, int RPT, typename E>
+__device__ __forceinline__ void rows_tile(
+    char *smem, const Tile tile, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
+    const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout &L,
     const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part,
     double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
   static_assert(RK * NMAX <= 256, "one B' element per thread");
   static_assert(RK == kKChunk, "row kernel steps are the plan's k-chunks");
-  __shared__ double Bs[P][RK][NMAX];
-  __shared__ int32_t s_acol[RK], s_brow[RK], s_bcol[NMAX];
+  auto &Bs = reinterpret_cast<RowsShared<CPLX, NMAX> *>(smem)->Bs;
+  auto &s_acol = reinterpret_cast<RowsShared<CPLX, NMAX> *>(smem)->acol;
+  auto &s_brow = reinterpret_cast<RowsShared<CPLX, NMAX> *>(smem)->brow;
+  auto &s_bcol = reinterpret_cast<RowsShared<CPLX, NMAX> *>(smem)->bcol;
 
-  const Tile tile = tiles[xcd_tile(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   const Seg seg = segs[tile.seg];
   const int tid = threadIdx.x;
   const int r0 = tile.tm * (256 * RPT);
@@ -751,15 +1018,12 @@ __global__ __launch_bounds__(256) void k_rows_f64(
 }
 
 // Sum of the k-slices of one row tile, in slice order, then the epilogue.
-template <bool CPLX, int NMAX, int RPT, typename E = double>
-__global__ __launch_bounds__(256) void k_reduce_rows(const ReduceItem *__restrict__ items,
-                                                     const Seg *__restrict__ segs, const double *__restrict__ part,
-                                                     E *__restrict__ C, double alpha_r, double alpha_i,
-                                                     double beta_r, double beta_i) {
+template <bool CPLX, int NMAX, int RPT, typename E>
+__device__ __forceinline__ void reduce_rows(const ReduceItem it, const Seg &seg, const double *__restrict__ part,
+                                            E *__restrict__ C, double alpha_r, double alpha_i, double beta_r,
+                                            double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
   constexpr int SZ = 256 * RPT * NMAX * P;
-  const ReduceItem it = items[blockIdx.x];
-  const Seg seg = segs[it.seg];
   const int tid = threadIdx.x;
   double acc[RPT][NMAX], acc_i[RPT][NMAX];
 #pragma unroll
@@ -798,23 +1062,29 @@ __global__ __launch_bounds__(256) void k_reduce_rows(const ReduceItem *__restric
 // summed from registers in the row kernel's order and stored with its alpha
 // / beta epilogue.  Replaces, for these blocks, the per-task loop of
 // global_operations.h:919-978 (one BLAS call per task).
-template <bool CPLX, bool STREAM, typename E = double>
-__global__ __launch_bounds__(256) void k_panel_rows(const PanelTile *__restrict__ tiles,
-                                                    const PanelOut *__restrict__ outs,
-                                                    const PanelTerm *__restrict__ terms, const Seg *__restrict__ segs,
-                                                    const E *__restrict__ A, const E *__restrict__ B,
-                                                    E *__restrict__ C, double alpha_r, double alpha_i,
-                                                    double beta_r, double beta_i) {
+template <bool CPLX>
+struct PanelShared {
+  double br[kPanelMaxTerms], bi[kPanelMaxTerms];
+  double pa[2][kPanelRows], pai[CPLX ? 2 : 1][kPanelRows];
+  int64_t ocoff[kPanelMaxOuts];
+  int32_t on[kPanelMaxOuts], ot0[kPanelMaxOuts], omask[kPanelMaxOuts];
+};
+template <bool CPLX, bool STREAM, typename E>
+__device__ __forceinline__ void panel_tile(char *smem, const PanelTile &pt, const PanelOut *__restrict__ outs,
+                                           const PanelTerm *__restrict__ terms, const Seg *__restrict__ segs,
+                                           const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C,
+                                           double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
   constexpr int RPT = kPanelRpt;
   static_assert(kPanelRows == 512 && RPT == 2, "pair staging: 4 loads per thread");
-  __shared__ double s_br[kPanelMaxTerms], s_bi[kPanelMaxTerms];
-  __shared__ double s_pa[2][kPanelRows], s_pai[CPLX ? 2 : 1][kPanelRows];
-  __shared__ int64_t s_ocoff[kPanelMaxOuts];
-  __shared__ int32_t s_on[kPanelMaxOuts], s_ot0[kPanelMaxOuts], s_omask[kPanelMaxOuts];
+  auto *sh = reinterpret_cast<PanelShared<CPLX> *>(smem);
+  auto &s_br = sh->br, &s_bi = sh->bi;
+  auto &s_pa = sh->pa;
+  auto &s_pai = sh->pai;
+  auto &s_ocoff = sh->ocoff;
+  auto &s_on = sh->on, &s_ot0 = sh->ot0, &s_omask = sh->omask;
   static_assert(kPanelMaxTerms <= 128 && kPanelMaxOuts <= 128, "one staging thread per term and per output");
 
-  const PanelTile &pt = tiles[blockIdx.x];
   const int tid = threadIdx.x;
   const int n_cols = pt.n_cols, n_outs = pt.n_outs, n_terms = pt.n_terms;
 
@@ -959,21 +1229,110 @@ __global__ __launch_bounds__(256) void k_panel_rows(const PanelTile *__restrict_
   else out_loop(std::false_type{});
 }
 
+// ---- kernels: one tile class, or all classes of a contraction ----
+
+// What every kernel of a contraction reads; tiles and reduction items are
+// stored class-major, and each class has its own region of `part`.
+template <typename E>
+struct ExecArgs {
+  const Tile *tiles;
+  const ReduceItem *red;
+  const Seg *segs;
+  const ExecTask *exec;
+  const BlkGather *ga, *gb;
+  const PanelTile *ptiles;
+  const PanelOut *pouts;
+  const PanelTerm *pterms;
+  const E *A, *B;
+  E *C;
+  double *part;
+  double ar, ai, br, bi;
+  GatherLayout L;
+  int64_t part_off[kNumTileClasses];
+  int32_t tile0[kNumTileClasses];     // first tile of the class
+  int32_t count[kNumTileClasses];     // its tiles
+};
+
+// Workgroup `b` of `n` of class CLS.
+template <bool CPLX, int CLS, typename E>
+__device__ __forceinline__ void class_block(char *smem, const ExecArgs<E> &x, int b, int n) {
+  const Tile *tiles = x.tiles + x.tile0[CLS];
+  double *part = x.part + x.part_off[CLS];
+  if constexpr (CLS == kTileRows4)
+    rows_tile<CPLX, 4, 4, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar,
+                             x.ai, x.br, x.bi);
+  else if constexpr (CLS == kTileRows16)
+    narrow_tile<CPLX, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar, x.ai,
+                         x.br, x.bi);
+  else
+    grouped_tile<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS), E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C,
+                                          part, x.ar, x.ai, x.br, x.bi);
+}
+template <bool CPLX, int CLS>
+constexpr size_t class_shared() {
+  if constexpr (CLS == kTileRows4) return sizeof(RowsShared<CPLX, 4>);
+  else if constexpr (CLS == kTileRows16) return sizeof(NarrowShared<CPLX>);
+  else return sizeof(GroupedShared<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS)>);
+}
+
+template <bool CPLX, int CLS, typename E>
+__global__ __launch_bounds__(256) void k_class(const ExecArgs<E> x) {
+  __shared__ __align__(16) char smem[class_shared<CPLX, CLS>()];
+  class_block<CPLX, CLS, E>(smem, x, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+}
+template <bool CPLX, bool STREAM, typename E>
+__global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
+  __shared__ __align__(16) char smem[sizeof(PanelShared<CPLX>)];
+  panel_tile<CPLX, STREAM, E>(smem, x.ptiles[blockIdx.x], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai, x.br,
+                              x.bi);
+}
+// The k-slice sums of reduction items first, first + 1, ...
+template <bool CPLX, typename E>
+__global__ __launch_bounds__(256) void k_reduce(const ExecArgs<E> x, int first) {
+  const ReduceItem it = x.red[first + static_cast<int>(blockIdx.x)];
+  const Seg seg = x.segs[it.seg];
+  const double *part = x.part + x.part_off[it.cls];
+  switch (it.cls) {
+    case 0: reduce_slices<CPLX, 64, 64, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    case 1: reduce_slices<CPLX, 32, 64, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    case 2: reduce_slices<CPLX, 64, 32, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    case 3: reduce_slices<CPLX, 32, 32, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    case kTileRows4: reduce_rows<CPLX, 4, 4, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    default: reduce_slices<CPLX, kNarrowM, kNarrowN, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+  }
+}
+
 }  // namespace
 
 namespace qlt {
 
-// Native grouped execution of a plan: MFMA tiles for the first tile class,
-// the row-streaming kernel for the second.  `mfma_class` = false skips the
-// MFMA class (the split path runs it on its own kernel).
+// Native grouped execution of a plan.  `mfma_class` = false leaves out the
+// MFMA classes with n > 16 (the split path runs them on its own kernel).
 qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void *a, const void *b, void *c,
                                  const double *alpha, const double *beta, hipStream_t st, bool mfma_class,
                                  bool probe, ClassStreams *shared) {
   const bool cplx = dtype_is_complex(dtype);
-  // classes with work run on the class streams when there are two or more
+  constexpr int32_t kPanelId = kNumTileClasses;
+  // the classes this call runs, the panels last
+  auto runs = [&](int32_t cls) {
+    if (cls == kPanelId) return plan->n_ptiles > 0;
+    return plan->cls_tiles[cls] > 0 && (mfma_class || !is_mfma_class(cls));
+  };
   int n_cls = 0;
-  for (int32_t cls = mfma_class ? 0 : kNumMfmaClasses; cls < kNumTileClasses; ++cls)
-    n_cls += plan->cls_tiles[cls] > 0 || (cls == kTileRows4 && plan->n_ptiles > 0);
+  for (int32_t cls = 0; cls <= kPanelId; ++cls) n_cls += runs(cls);
+  if (n_cls == 0) return QLT_OK;
+  // the class with the most algorithmic work is the one a kernel probe times,
+  // in a launch of its own
+  int32_t dom = -1;
+  if (probe && probe_armed(st)) {
+    double best = 0.0;
+    for (int32_t cls = 0; cls < kNumTileClasses; ++cls)
+      if (runs(cls) && plan->cls_mkn[cls] > best) {
+        best = plan->cls_mkn[cls];
+        dom = cls;
+      }
+    if (runs(kPanelId) && plan->panel_mkn > best) dom = kPanelId;
+  }
   std::unique_ptr<ClassStreams> own;
   ClassStreams *cs = shared;
   if (cs == nullptr && n_cls >= 2) {
@@ -981,28 +1340,16 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     cs = own.get();
   }
   auto stream_of = [&](int32_t cls) {
-    if (cls == kNumTileClasses) cls = kTileRows4;   // the row panels
+    if (cls == kPanelId) cls = kTileRows4;
     return cs != nullptr ? cs->get(cls) : st;
   };
-  // the class with the most algorithmic work is the one a kernel probe times
-  // (kPanelId: the row panels, on the stream of the n <= 4 row class)
-  constexpr int32_t kPanelId = kNumTileClasses;
-  int32_t dom = -1;
-  if (probe && probe_armed(st)) {
-    double best = 0.0;
-    for (int32_t cls = mfma_class ? 0 : kNumMfmaClasses; cls < kNumTileClasses; ++cls)
-      if (plan->cls_tiles[cls] > 0 && plan->cls_mkn[cls] > best) {
-        best = plan->cls_mkn[cls];
-        dom = cls;
-      }
-    if (plan->n_ptiles > 0 && plan->panel_mkn > best) dom = kPanelId;
-  }
   auto probe_in = [&](int32_t cls) {
     if (cls == dom) probe_begin(stream_of(cls));
   };
   auto probe_out = [&](int32_t cls) {
     if (cls != dom) return;
     const hipStream_t ps = stream_of(cls);
+    // the n <= 16 class keeps the name of the row class it is
     static const char *const kNames[kNumTileClasses + 1] = {
         "k_grouped_gemm_f64<64x64>", "k_grouped_gemm_f64<32x64>", "k_grouped_gemm_f64<64x32>",
         "k_grouped_gemm_f64<32x32>", "k_rows_f64<n<=4>",          "k_rows_f64<n<=16>",
@@ -1014,91 +1361,71 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     const double elems = cls == kPanelId ? plan->panel_elems : plan->cls_elems[cls];
     probe_end(ps, name, (cplx ? 8.0 : 2.0) * mkn, static_cast<double>(dtype_bytes(dtype)) * elems);
   };
-  const double ar = alpha[0], ai = cplx ? alpha[1] : 0.0;
-  const double br = beta[0], bi = cplx ? beta[1] : 0.0;
   const dim3 block(256);
+  auto grid_of = [](int64_t n) { return dim3(static_cast<unsigned>(n)); };
   // every kernel instance of one element storage type E (double, or float
   // for the single-precision element types) and complexity
   auto run = [&](auto e_tag, auto cplx_tag) {
     using E = decltype(e_tag);
     constexpr bool CX = decltype(cplx_tag)::value;
-    const auto *A = static_cast<const E *>(a);
-    const auto *B = static_cast<const E *>(b);
-    auto *Cp = static_cast<E *>(c);
-    // MFMA classes: 64x64, 32x64, 64x32, 32x32 (tiles stored class-major)
+    ExecArgs<E> x{};
+    x.tiles = plan->d_tiles;
+    x.red = plan->d_red;
+    x.segs = plan->d_segs;
+    x.exec = plan->d_exec;
+    x.ga = plan->d_ga;
+    x.gb = plan->d_gb;
+    x.ptiles = plan->d_ptiles;
+    x.pouts = plan->d_pouts;
+    x.pterms = plan->d_pterms;
+    x.A = static_cast<const E *>(a);
+    x.B = static_cast<const E *>(b);
+    x.C = static_cast<E *>(c);
+    x.part = plan->d_part;
+    x.ar = alpha[0];
+    x.ai = CX ? alpha[1] : 0.0;
+    x.br = beta[0];
+    x.bi = CX ? beta[1] : 0.0;
+    x.L = plan->layout;
     int64_t base = 0, red_base = 0;
-    for (int cls = 0; cls < kNumMfmaClasses; ++cls) {
-      const int64_t cnt = plan->cls_tiles[cls];
-      const int64_t n_red = plan->cls_red[cls];
-      const Tile *tp = plan->d_tiles + base;
-      const ReduceItem *rp = plan->d_red + red_base;
-      base += cnt;
-      red_base += n_red;
-      if (!mfma_class || cnt == 0) continue;
-      const dim3 grid(static_cast<unsigned>(cnt));
-      const hipStream_t ls = stream_of(cls);
-      // this class's region of the k-slice partial sums
-      double *const cls_part = plan->d_part != nullptr ? plan->d_part + plan->cls_part_off[cls] : nullptr;
-      // k-sliced tiles: the slices write partial sums, then one reduction
-      // workgroup per sliced tile adds them and applies alpha / beta
-      auto mfma = [&](auto tm_tag, auto tn_tag) {
-        constexpr int TMV = decltype(tm_tag)::value, TNV = decltype(tn_tag)::value;
-        probe_in(cls);
-        hipLaunchKernelGGL((k_grouped_gemm_f64<CX, TMV, TNV, E>), grid, block, 0, ls, tp, plan->d_segs, plan->d_exec,
-                           plan->d_ga, plan->d_gb, plan->layout, A, B, Cp, cls_part, ar, ai, br, bi);
-        probe_out(cls);
-        if (n_red > 0)
-          hipLaunchKernelGGL((k_reduce_slices<CX, TMV, TNV, E>), dim3(static_cast<unsigned>(n_red)), block, 0, ls, rp,
-                             plan->d_segs, cls_part, Cp, ar, ai, br, bi);
-      };
-      using I32 = std::integral_constant<int, 32>;
-      using I64 = std::integral_constant<int, 64>;
-      if (cls == 0) mfma(I64{}, I64{});
-      else if (cls == 1) mfma(I32{}, I64{});
-      else if (cls == 2) mfma(I64{}, I32{});
-      else mfma(I32{}, I32{});
+    int32_t red0[kNumTileClasses];
+    for (int32_t cls = 0; cls < kNumTileClasses; ++cls) {
+      x.part_off[cls] = plan->cls_part_off[cls];
+      x.tile0[cls] = static_cast<int32_t>(base);
+      x.count[cls] = static_cast<int32_t>(plan->cls_tiles[cls]);
+      red0[cls] = static_cast<int32_t>(red_base);
+      base += plan->cls_tiles[cls];
+      red_base += plan->cls_red[cls];
     }
-    // row classes (n <= 4, n <= 16), each followed by its k-slice reduction
-    for (int32_t cls = kTileRows4; cls <= kTileRows16; ++cls) {
-      const int64_t cnt = plan->cls_tiles[cls];
-      const int64_t n_red = plan->cls_red[cls];
-      const Tile *tp = plan->d_tiles + base;
-      const ReduceItem *rp = plan->d_red + red_base;
-      base += cnt;
-      red_base += n_red;
-      if (cnt == 0) continue;
-      const dim3 grid(static_cast<unsigned>(cnt)), rgrid(static_cast<unsigned>(n_red > 0 ? n_red : 1));
-      const hipStream_t ls = stream_of(cls);
-      // this class's region of the k-slice partial sums
-      double *const cls_part = plan->d_part != nullptr ? plan->d_part + plan->cls_part_off[cls] : nullptr;
-      auto rows = [&](auto nmax_tag, auto rpt_tag) {
-        constexpr int NMAXV = decltype(nmax_tag)::value, RPTV = decltype(rpt_tag)::value;
-        probe_in(cls);
-        hipLaunchKernelGGL((k_rows_f64<CX, NMAXV, RPTV, E>), grid, block, 0, ls, tp, plan->d_segs, plan->d_exec,
-                           plan->d_ga, plan->d_gb, plan->layout, A, B, Cp, cls_part, ar, ai, br, bi);
-        probe_out(cls);
-        if (n_red > 0)
-          hipLaunchKernelGGL((k_reduce_rows<CX, NMAXV, RPTV, E>), rgrid, block, 0, ls, rp, plan->d_segs, cls_part, Cp,
-                             ar, ai, br, bi);
-      };
-      if (cls == kTileRows4) rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
-      else rows(std::integral_constant<int, 16>{}, std::integral_constant<int, 1>{});
-    }
+    // non-temporal A' loads only when the panels' A' and C exceed the
+    // last-level cache: smaller ones are served from it (measured: a
+    // 0.83 GB W contraction 0.169 -> 0.148 ms with the hint, a small one
+    // 0.028 -> 0.032 ms)
+    const bool stream_a = plan->panel_elems * static_cast<double>(sizeof(E) * (CX ? 2 : 1)) > kPanelStreamBytes;
+    auto one = [&](auto cls_tag) {
+      constexpr int CLS = decltype(cls_tag)::value;
+      if (!runs(CLS)) return;
+      const hipStream_t ls = stream_of(CLS);
+      probe_in(CLS);
+      hipLaunchKernelGGL((k_class<CX, CLS, E>), grid_of(plan->cls_tiles[CLS]), block, 0, ls, x);
+      probe_out(CLS);
+      // k-sliced tiles: the slices wrote partial sums; one workgroup per sliced
+      // tile adds them and applies alpha / beta
+      if (plan->cls_red[CLS] > 0)
+        hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(plan->cls_red[CLS]), block, 0, ls, x, red0[CLS]);
+    };
+    one(std::integral_constant<int, 0>{});
+    one(std::integral_constant<int, 1>{});
+    one(std::integral_constant<int, 2>{});
+    one(std::integral_constant<int, 3>{});
+    one(std::integral_constant<int, 4>{});
+    one(std::integral_constant<int, 5>{});
     // row panels, after the n <= 4 row class on its stream
-    if (plan->n_ptiles > 0) {
+    if (runs(kPanelId)) {
       const hipStream_t ls = stream_of(kPanelId);
       probe_in(kPanelId);
-      // non-temporal A' loads only when the panels' A' and C exceed the
-      // last-level cache: smaller ones are served from it (measured: a
-      // 0.83 GB W contraction 0.169 -> 0.148 ms with the hint, a small one
-      // 0.028 -> 0.032 ms)
-      const bool stream_a = plan->panel_elems * static_cast<double>(sizeof(E) * (CX ? 2 : 1)) > kPanelStreamBytes;
-      if (stream_a)
-        hipLaunchKernelGGL((k_panel_rows<CX, true, E>), dim3(static_cast<unsigned>(plan->n_ptiles)), block, 0, ls,
-                           plan->d_ptiles, plan->d_pouts, plan->d_pterms, plan->d_segs, A, B, Cp, ar, ai, br, bi);
-      else
-        hipLaunchKernelGGL((k_panel_rows<CX, false, E>), dim3(static_cast<unsigned>(plan->n_ptiles)), block, 0, ls,
-                           plan->d_ptiles, plan->d_pouts, plan->d_pterms, plan->d_segs, A, B, Cp, ar, ai, br, bi);
+      if (stream_a) hipLaunchKernelGGL((k_panel_rows<CX, true, E>), grid_of(plan->n_ptiles), block, 0, ls, x);
+      else hipLaunchKernelGGL((k_panel_rows<CX, false, E>), grid_of(plan->n_ptiles), block, 0, ls, x);
       probe_out(kPanelId);
     }
   };

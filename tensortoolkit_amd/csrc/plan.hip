@@ -700,6 +700,9 @@ constexpr int64_t kSliceTargetWGs = 2048;
 // traffic) measured faster on every matvec chain here than 2048.
 constexpr int64_t kSliceTargetWGsMfma = 512;
 constexpr int64_t kMinSliceChunks = 8;
+// The n <= 16 class spreads a tile's chunks over four waves by itself: slices
+// as short as the MFMA classes' would leave two chunks to a wave.
+constexpr int64_t kMinSliceChunksNarrow = 32;
 constexpr int64_t kMaxSlices = 64;
 
 qlt_status slice_long_tiles(qlt_plan *plan) {
@@ -731,7 +734,7 @@ qlt_status slice_long_tiles(qlt_plan *plan) {
     const bool unsliced = plan->slice_target[cls] < 0;
     const int64_t target = plan->slice_target[cls] > 0 ? plan->slice_target[cls]
                                                        : (is_mfma_class(cls) ? kSliceTargetWGsMfma : kSliceTargetWGs);
-    const int64_t q = std::max(kMinSliceChunks, (total + target - 1) / target);
+    const int64_t q = std::max(cls == kTileRows16 ? kMinSliceChunksNarrow : kMinSliceChunks, (total + target - 1) / target);
     std::vector<Tile> cl;
     int64_t parts = 0, n_red = 0;
     for (int64_t i = base; i < base + cnt; ++i) {

@@ -132,9 +132,9 @@ __host__ __device__ inline void magic_of(uint32_t d, uint64_t &mag, int32_t &sh)
 
 // Tile classes.  Classes 0..3: MFMA output tiles of 64x64, 32x64, 64x32 and
 // 32x32 (rows x cols), chosen per output block to limit padding.
-// kTileRows4 / kTileRows16: narrow outputs (n <= 4 / n <= 16) on a
-// row-streaming kernel (bandwidth-bound work), 1024 / 256 output rows per
-// workgroup (4 / 1 rows per thread).
+// kTileRows4: narrow outputs (n <= 4) on a row-streaming path, 1024 output
+// rows per workgroup (4 per thread).  kTileRows16: n <= 16, MFMA tiles of 32
+// rows with the contracted extent spread over the workgroup's waves.
 constexpr int32_t kTileMfma = 0;       // 64 x 64 (first MFMA class)
 constexpr int32_t kNumMfmaClasses = 4;
 constexpr int32_t kTileRows4 = 4;
@@ -179,7 +179,7 @@ __host__ __device__ inline int32_t tuned_tile_class(int64_t m, int64_t n,
   const int8_t t = table[bm - 1][bn - 1];
   return (t >= 0 && t < kNumMfmaClasses) ? t : c;
 }
-__host__ __device__ constexpr int32_t rows_per_tile(int32_t cls) { return cls == kTileRows4 ? 1024 : 256; }
+__host__ __device__ constexpr int32_t rows_per_tile(int32_t cls) { return cls == kTileRows4 ? 1024 : 32; }
 __host__ __device__ constexpr int64_t tiles_of(int32_t cls, int64_t m, int64_t n) {
   return is_mfma_class(cls)
              ? ((m + mfma_tile_m(cls) - 1) / mfma_tile_m(cls)) * ((n + mfma_tile_n(cls) - 1) / mfma_tile_n(cls))
