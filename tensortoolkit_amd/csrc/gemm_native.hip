@@ -6,7 +6,7 @@
 // (hp_numeric::TensorTranspose, framework/hp_numeric/ten_trans.h:56-114,245-349)
 // and then issues one BLAS call C_blk = A'(m x k) B'(k x n) + beta C_blk
 // (hp_numeric::MatMultiply, framework/hp_numeric/blas_level3.h:35-56,798-856).
-// Here one launch per tile class covers the whole plan.  Each workgroup owns
+// Here one launch covers the whole plan (k_all_classes).  Each workgroup owns
 // one TM x TN tile (64 or 32 each way; 32 x 16 for n <= 16) of one output
 // block, or one k-slice of it, and walks every task of that block, so the
 // per-block beta chain (0 for the first task, 1 after) becomes a single write
@@ -1251,7 +1251,12 @@ struct ExecArgs {
   int64_t part_off[kNumTileClasses];
   int32_t tile0[kNumTileClasses];     // first tile of the class
   int32_t count[kNumTileClasses];     // its tiles
+  int32_t block0[kNumTileClasses + 1];  // k_all_classes: first workgroup of the class, and of the panels
 };
+
+// Order of the classes in k_all_classes: the few narrow-output tiles, whose
+// chains of contracted indices are the longest, start first.
+constexpr int32_t kLaunchOrder[kNumTileClasses - 1] = {kTileRows16, kTileRows4, 1, 3, kNumTileClasses};
 
 // Workgroup `b` of `n` of class CLS.
 template <bool CPLX, int CLS, typename E>
@@ -1285,6 +1290,28 @@ __global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
   __shared__ __align__(16) char smem[sizeof(PanelShared<CPLX>)];
   panel_tile<CPLX, STREAM, E>(smem, x.ptiles[blockIdx.x], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai, x.br,
                               x.bi);
+}
+// Every class of a contraction in one launch (the 64-row MFMA classes, which
+// only a tuning table selects, excepted).  With a launch per class on streams
+// forked from the caller's and joined back, the forks and the gaps between
+// dependent launches were most of a small contraction and a tenth of a large
+// one: U(1) FP64 matvec at D = 96 103 -> 32 us, D = 700 164 -> 43 us, lognormal
+// 184 -> 117 us, U(1)xU(1) complex128 D = 1500 252 -> 156 us, D = 4096 1.22 ->
+// 1.18 ms.  The register bound keeps the occupancy of the widest class alone
+// (complex: three workgroups per CU; unbounded, two, and D = 4096 took 1.35 ms).
+template <bool CPLX, bool STREAM, typename E>
+__global__ __launch_bounds__(256, CPLX ? 3 : 4) void k_all_classes(const ExecArgs<E> x) {
+  constexpr size_t kBytes = std::max({class_shared<CPLX, 1>(), class_shared<CPLX, 3>(), class_shared<CPLX, 4>(),
+                                      class_shared<CPLX, 5>(), sizeof(PanelShared<CPLX>)});
+  __shared__ __align__(16) char smem[kBytes];
+  const int b = static_cast<int>(blockIdx.x);
+  if (b < x.block0[4]) class_block<CPLX, 5, E>(smem, x, b - x.block0[5], x.count[5]);
+  else if (b < x.block0[1]) class_block<CPLX, 4, E>(smem, x, b - x.block0[4], x.count[4]);
+  else if (b < x.block0[3]) class_block<CPLX, 1, E>(smem, x, b - x.block0[1], x.count[1]);
+  else if (b < x.block0[6]) class_block<CPLX, 3, E>(smem, x, b - x.block0[3], x.count[3]);
+  else
+    panel_tile<CPLX, STREAM, E>(smem, x.ptiles[b - x.block0[6]], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai,
+                                x.br, x.bi);
 }
 // The k-slice sums of reduction items first, first + 1, ...
 template <bool CPLX, typename E>
@@ -1333,9 +1360,13 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
       }
     if (runs(kPanelId) && plan->panel_mkn > best) dom = kPanelId;
   }
+  // one launch for all classes; a probed class, and the 64-row classes that
+  // k_all_classes leaves out, take a launch per class on the class streams
+  const bool fused = dom < 0 && n_cls >= 2 && !runs(0) && !runs(2) &&
+                     plan->n_tiles + plan->n_ptiles < (int64_t(1) << 31);
   std::unique_ptr<ClassStreams> own;
   ClassStreams *cs = shared;
-  if (cs == nullptr && n_cls >= 2) {
+  if (cs == nullptr && n_cls >= 2 && !fused) {
     own = std::make_unique<ClassStreams>(st);
     cs = own.get();
   }
@@ -1389,19 +1420,37 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     x.L = plan->layout;
     int64_t base = 0, red_base = 0;
     int32_t red0[kNumTileClasses];
+    int64_t first_red = -1, n_red = 0;
     for (int32_t cls = 0; cls < kNumTileClasses; ++cls) {
       x.part_off[cls] = plan->cls_part_off[cls];
       x.tile0[cls] = static_cast<int32_t>(base);
       x.count[cls] = static_cast<int32_t>(plan->cls_tiles[cls]);
       red0[cls] = static_cast<int32_t>(red_base);
+      if (runs(cls) && plan->cls_red[cls] > 0) {
+        if (first_red < 0) first_red = red_base;
+        n_red = red_base + plan->cls_red[cls] - first_red;   // the classes that run are the last ones: contiguous
+      }
       base += plan->cls_tiles[cls];
       red_base += plan->cls_red[cls];
+    }
+    int64_t blocks = 0;
+    for (const int32_t cls : kLaunchOrder) {
+      x.block0[cls] = static_cast<int32_t>(blocks);
+      if (cls == kPanelId) blocks += plan->n_ptiles;
+      else if (runs(cls)) blocks += plan->cls_tiles[cls];
     }
     // non-temporal A' loads only when the panels' A' and C exceed the
     // last-level cache: smaller ones are served from it (measured: a
     // 0.83 GB W contraction 0.169 -> 0.148 ms with the hint, a small one
     // 0.028 -> 0.032 ms)
     const bool stream_a = plan->panel_elems * static_cast<double>(sizeof(E) * (CX ? 2 : 1)) > kPanelStreamBytes;
+    if (fused) {
+      const hipStream_t ls = stream_of(kTileRows4);
+      if (stream_a) hipLaunchKernelGGL((k_all_classes<CX, true, E>), grid_of(blocks), block, 0, ls, x);
+      else hipLaunchKernelGGL((k_all_classes<CX, false, E>), grid_of(blocks), block, 0, ls, x);
+      if (n_red > 0) hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(n_red), block, 0, ls, x, static_cast<int>(first_red));
+      return;
+    }
     auto one = [&](auto cls_tag) {
       constexpr int CLS = decltype(cls_tag)::value;
       if (!runs(CLS)) return;
