@@ -50,6 +50,32 @@ inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s);
 // True when `s` is currently being captured into a graph.
 bool stream_capturing(hipStream_t s);
 
+// Page-locked host memory for one copy to or from the device, taken from a
+// small library-wide pool (at most kPinnedKept buffers of at most
+// kPinnedKeptBytes are kept, and freed by qlt_finalize) and handed back when
+// the object ends, after the stream has finished with it.
+constexpr size_t kPinnedKept = 8, kPinnedKeptBytes = size_t(8) << 20;
+class PinnedStaging {
+ public:
+  explicit PinnedStaging(hipStream_t st) : st_(st) {}
+  ~PinnedStaging() { release(); }
+  PinnedStaging(const PinnedStaging &) = delete;
+  PinnedStaging &operator=(const PinnedStaging &) = delete;
+  // At least `bytes`; what was in it is lost when it has to grow (the stream
+  // must be done with it then, and is waited for).
+  qlt_status reserve(size_t bytes);
+  template <typename T>
+  T *at(size_t off) const {
+    return reinterpret_cast<T *>(static_cast<char *>(p_) + off);
+  }
+
+ private:
+  void release();
+  hipStream_t st_;
+  void *p_ = nullptr;
+  size_t bytes_ = 0;
+};
+
 // ---- device work-list records -------------------------------------------
 
 // Gather descriptor of one input block: the block permuted to
@@ -332,7 +358,8 @@ struct qlt_plan {
   int64_t max_blk_elems_b = 0;
   int64_t a_raw_extent = 0;             // max over A blocks of offset + size
   int64_t b_raw_extent = 0;
-  // ---- device work list ----
+  // ---- device work list: arrays of one allocation ----
+  void *d_store = nullptr;
   qlt::GatherLayout layout{};
   int64_t n_exec = 0;                   // == tasks.size()
   int64_t n_segs = 0;
@@ -346,9 +373,6 @@ struct qlt_plan {
   qlt::BlkGather *d_gb = nullptr;
   std::vector<qlt::Seg> h_segs;         // host mirror (used to rebuild offsets)
   std::vector<qlt::ExecTask> h_exec;    // host mirror of the execution list
-  // tile-size class table chosen at build time
-  int32_t tile_m = 64;
-  int32_t tile_n = 64;
   // k-slicing workgroup target per tile class in effect at build time
   // (0: the built-in target, -1: unsliced)
   int32_t slice_target[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};
@@ -387,10 +411,7 @@ struct qlt_plan {
   qlt_plan(const qlt_plan &) = delete;
   qlt_plan &operator=(const qlt_plan &) = delete;
   ~qlt_plan() {
-    for (void *p : {static_cast<void *>(d_exec), static_cast<void *>(d_segs), static_cast<void *>(d_tiles),
-                    static_cast<void *>(d_ga), static_cast<void *>(d_gb), d_work, static_cast<void *>(d_red),
-                    static_cast<void *>(d_part), static_cast<void *>(d_ptiles), static_cast<void *>(d_pouts),
-                    static_cast<void *>(d_pterms)})
+    for (void *p : {d_store, d_work, static_cast<void *>(d_part)})
       if (p != nullptr) (void)hipFree(p);
   }
 };

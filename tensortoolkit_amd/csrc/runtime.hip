@@ -10,6 +10,7 @@
 #include <mutex>
 #include <type_traits>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "qlt_internal.h"
@@ -119,6 +120,59 @@ ClassStreams::~ClassStreams() {
       (void)hipStreamWaitEvent(st_, g_cls_join[c], 0);
     }
   g_cls_mutex.unlock();
+}
+
+// ---- page-locked staging ----
+namespace {
+std::mutex g_pinned_mutex;
+std::vector<std::pair<void *, size_t>> g_pinned;   // free buffers
+
+void pinned_free_all() {
+  std::lock_guard<std::mutex> lock(g_pinned_mutex);
+  for (auto &b : g_pinned) (void)hipHostFree(b.first);
+  g_pinned.clear();
+}
+}  // namespace
+
+qlt_status PinnedStaging::reserve(size_t bytes) {
+  if (bytes <= bytes_) return QLT_OK;
+  release();
+  {
+    // the smallest free buffer that fits
+    std::lock_guard<std::mutex> lock(g_pinned_mutex);
+    size_t best = g_pinned.size();
+    for (size_t i = 0; i < g_pinned.size(); ++i)
+      if (g_pinned[i].second >= bytes && (best == g_pinned.size() || g_pinned[i].second < g_pinned[best].second))
+        best = i;
+    if (best < g_pinned.size()) {
+      p_ = g_pinned[best].first;
+      bytes_ = g_pinned[best].second;
+      g_pinned.erase(g_pinned.begin() + static_cast<std::ptrdiff_t>(best));
+      return QLT_OK;
+    }
+  }
+  size_t n = size_t(64) << 10;
+  while (n < bytes) n *= 2;
+  // portable: usable from whichever device the thread has current
+  QLT_HIP(hipHostMalloc(&p_, n, hipHostMallocPortable));
+  bytes_ = n;
+  return QLT_OK;
+}
+
+void PinnedStaging::release() {
+  if (p_ == nullptr) return;
+  (void)hipStreamSynchronize(st_);
+  bool kept = false;
+  if (bytes_ <= kPinnedKeptBytes) {
+    std::lock_guard<std::mutex> lock(g_pinned_mutex);
+    if (g_pinned.size() < kPinnedKept) {
+      g_pinned.emplace_back(p_, bytes_);
+      kept = true;
+    }
+  }
+  if (!kept) (void)hipHostFree(p_);
+  p_ = nullptr;
+  bytes_ = 0;
 }
 
 // ---- kernel probe ----
@@ -409,6 +463,7 @@ qlt_status qlt_finalize(void) {
     std::lock_guard<std::mutex> cl(g_cls_mutex);
     class_streams_destroy();
   }
+  pinned_free_all();
   g_initialized = false;
   return QLT_OK;
 }
