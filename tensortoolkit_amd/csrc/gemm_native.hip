@@ -81,6 +81,15 @@ __device__ __forceinline__ double im_of(float2 v) { return static_cast<double>(v
 __device__ __forceinline__ double im_of(double) { return 0.0; }
 __device__ __forceinline__ double im_of(float) { return 0.0; }
 template <typename E, bool CPLX>
+__device__ __forceinline__ void zero_unless(raw_t<E, CPLX> &v, bool ok) {
+  if constexpr (CPLX) {
+    v.x = ok ? v.x : E(0);
+    v.y = ok ? v.y : E(0);
+  } else {
+    v = ok ? v : E(0);
+  }
+}
+template <typename E, bool CPLX>
 __device__ __forceinline__ void st_elem(E *p, double re, double im) {
   if constexpr (CPLX) {
     if constexpr (sizeof(E) == 8) *reinterpret_cast<double2 *>(p) = double2{re, im};
@@ -182,16 +191,27 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 // Grouped MFMA kernel, one 256-thread workgroup per TM x TN output tile
 // (TM, TN in {32, 64}); the four waves split the tile 2 x 2, each wave
 // computing (TM/2) x (TN/2) as BM x BN blocks of v_mfma_f64_16x16x4f64.
-// Per-thread gather of the A' (TM x 16) and B' (16 x TN) k-chunk:
-//   A' k-contiguous -> p = tid & 15, rows (tid >> 4) + 16 q;
-//      otherwise    -> r = tid % TM, cols tid / TM + (256 / TM) q;
-//   B' n-contiguous -> c = tid % TN, rows tid / TN + (256 / TN) q;
-//      otherwise    -> p = tid & 15, cols (tid >> 4) + 16 q.
+//   What bounds it: the MFMAs are busy about half of the time (64 cycles each;
+// 45 us of a 100 us D = 2048 FP64 launch), the rest is the chain of a step --
+// loads, LDS, barrier -- that three to five workgroups per CU only partly
+// cover.  Measured without gain: loads issued two steps ahead (249 us either
+// way at D = 2048 FP64), 8-deep complex steps at four workgroups per CU (1.14
+// ms either way at D = 4096), B' fragments loaded past LDS (249 -> 308 us), and
+// 64 x 64 tiles (303 -> 376 us).
+// The staged chunk, double-buffered, real and imaginary planes: A' by rows (18
+// doubles apart), B' by k (TN + 4 doubles apart), contracted index p at place
+// k_place(p).  Lane (lr, lk) finds the indices lk, 4 + lk, 8 + lk, 12 + lk of the four
+// MFMA steps at places 4 lk .. 4 lk + 3: A' is read in 16-byte pieces, and both
+// strides keep a wave's reads and the k-contiguous / n-contiguous writes free
+// of bank conflicts (with both operands by k and rows one double more than a
+// power of two apart, every read took two passes: D = 2048 FP64 matvec 308 ->
+// 277 us).
+__device__ __forceinline__ int k_place(int p) { return ((p & 3) << 2) | (p >> 2); }
 template <bool CPLX, int TMv, int TNv>
 struct GroupedShared {
-  static constexpr int P = CPLX ? 2 : 1, KCv = KC;
-  double As[2][P][KCv][TMv + 1];
-  double Bs[2][P][KCv][TNv + 1];
+  static constexpr int P = CPLX ? 2 : 1;
+  double As[2][P][TMv][KC + 2];
+  double Bs[2][P][KC][TNv + 4];
 };
 template <bool CPLX, int TMv, int TNv, typename E>
 __device__ __forceinline__ void grouped_tile(
@@ -200,20 +220,17 @@ __device__ __forceinline__ void grouped_tile(
     const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part,
     double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
-  constexpr int KCv = KC;                              // k extent per pipeline step
-  constexpr int QA = TMv / 16, QB = TNv / 16;          // elements per thread per step
+  constexpr int QA = TMv / 16, QB = TNv / 16;          // elements per thread per 16-k step
   constexpr int BM = TMv / 32, BN = TNv / 32;          // MFMA blocks per wave
   auto &As = reinterpret_cast<GroupedShared<CPLX, TMv, TNv> *>(smem)->As;
   auto &Bs = reinterpret_cast<GroupedShared<CPLX, TMv, TNv> *>(smem)->Bs;
 
   const Seg seg = segs[tile.seg];
   const int i0 = tile.tm * TMv, j0 = tile.tn * TNv;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (w >> 1) * (TMv / 2), wn = (w & 1) * (TNv / 2);
   const int lr = lane & 15, lk = lane >> 4;
-  // thread mapping of the chunk being fetched, chosen per task: plain
-  // blocks always read along memory order
-  bool akf = L.a_kfast != 0, bnf = L.b_nfast != 0;
 
   v4d acc[BM][BN], acc_i[BM][BN], acc_s[BM][BN];
 #pragma unroll
@@ -225,138 +242,86 @@ __device__ __forceinline__ void grouped_tile(
       acc_s[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
     }
 
-  auto a_r = [&](int q) { return akf ? (tid >> 4) + 16 * q : tid % TMv; };
-  auto a_p = [&](int q) { return akf ? tid & 15 : tid / TMv + (256 / TMv) * q; };
-  auto b_c = [&](int q) { return bnf ? tid % TNv : (tid >> 4) + 16 * q; };
-  auto b_p = [&](int q) { return bnf ? tid / TNv + (256 / TNv) * q : tid & 15; };
-
-  // Per task: the row offsets of the A' elements and column offsets of the
-  // B' elements this thread loads.  A block whose permuted view is plain
-  // (row i, col p at i * ncols + p) needs no decomposition at all.
-  int32_t a_row[QA], b_col[QB];
-  bool a_plain = false, b_plain = false;
-  raw_t<E, CPLX> pa[QA], pb[QB];
-  // every task of this output block reads plain blocks: no descriptor reads
-  const bool seg_plain = (seg.flags & (kSegAPlain | kSegBPlain)) == (kSegAPlain | kSegBPlain);
-  auto task_rows = [&](const BlkGather &gA, const BlkGather &gB, const ExecTask &et) {
-    a_plain = seg_plain || gA.plain != 0;
-    b_plain = seg_plain || gB.plain != 0;
-    akf = a_plain || gA.fastcol != 0;
-    bnf = b_plain || gB.fastcol != 0;
-#pragma unroll
-    for (int q = 0; q < QA; ++q) {
-      const int r = i0 + a_r(q);
-      a_row[q] = (r < seg.m) ? (a_plain ? r * et.k : split_offset(r, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr)) : -1;
-    }
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      const int c = j0 + b_c(q);
-      b_col[q] = (c < seg.n) ? (b_plain ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc)) : -1;
-    }
-  };
-  auto fetch = [&](const ExecTask &et, const BlkGather &gA, const BlkGather &gB, int kk, int kend) {
-#pragma unroll
-    for (int q = 0; q < QA; ++q) {
-      const int pk = kk + a_p(q);
-      const int32_t ac = (pk < kend) ? (a_plain ? pk : split_offset(pk, gA.cdim, gA.cstr, gA.cmag, gA.csh, L.a_nc)) : -1;
-      const bool ok = (a_row[q] >= 0) && (ac >= 0);
-      const int64_t e = et.a_off + a_row[q] + ac;
-      pa[q] = ok ? ld_raw<E, CPLX>(A + e * P) : raw_t<E, CPLX>{};
-    }
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      const int pk = kk + b_p(q);
-      const int32_t br = (pk < kend) ? (b_plain ? pk * seg.n : split_offset(pk, gB.rdim, gB.rstr, gB.rmag, gB.rsh, L.b_nr)) : -1;
-      const bool ok = (b_col[q] >= 0) && (br >= 0);
-      const int64_t e = et.b_off + br + b_col[q];
-      pb[q] = ok ? ld_raw<E, CPLX>(B + e * P) : raw_t<E, CPLX>{};
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < QA; ++q) {
-      As[buf][0][a_p(q)][a_r(q)] = re_of(pa[q]);
-      if (CPLX) As[buf][P - 1][a_p(q)][a_r(q)] = im_of(pa[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-      Bs[buf][0][b_p(q)][b_c(q)] = re_of(pb[q]);
-      if (CPLX) Bs[buf][P - 1][b_p(q)][b_c(q)] = im_of(pb[q]);
-    }
-  };
-
   // ---- MFMAs on one staged step ----
-  // Work outside the output block is skipped at the MFMA's own granularity:
-  // 16 x 16 sub-blocks of the wave that lie wholly beyond m or n, and k
-  // steps of 4 beyond the step's valid extent `kv` (all wave-uniform).
+  // Work outside the output block is skipped: 16 x 16 sub-blocks of the wave
+  // that lie wholly beyond m or n, and halves of a chunk beyond its valid
+  // extent `kv`, all wave-uniform.  The fragments of half a chunk are read
+  // together, before its MFMAs: read one by one inside a guard, each MFMA
+  // waited for its own LDS round trip (with the unguarded loads below, D = 2048
+  // FP64 277 -> 249 us, D = 4096 complex128 1.17 -> 1.14 ms).
   bool mt_ok[BM], nt_ok[BN];
 #pragma unroll
   for (int mt = 0; mt < BM; ++mt) mt_ok[mt] = i0 + wm + mt * 16 < seg.m;
 #pragma unroll
   for (int nt = 0; nt < BN; ++nt) nt_ok[nt] = j0 + wn + nt * 16 < seg.n;
+  const bool wave_on = mt_ok[0] && nt_ok[0];
+  typedef double v2d __attribute__((ext_vector_type(2)));
   auto compute = [&](int buf, int kv) {
+    if (!wave_on) return;
 #pragma unroll
-    for (int ks = 0; ks < KCv; ks += 4) {
-      if (ks >= kv) break;
-      double a[BM], b[BN];
+    for (int h = 0; h < 2; ++h) {
+      if (8 * h >= kv) break;
+      v2d a[BM], ai[BM];
+      double b[2][BN], bi[2][BN];
 #pragma unroll
-      for (int mt = 0; mt < BM; ++mt) a[mt] = As[buf][0][ks + lk][wm + mt * 16 + lr];
+      for (int mt = 0; mt < BM; ++mt) {
+        a[mt] = *reinterpret_cast<const v2d *>(&As[buf][0][wm + mt * 16 + lr][4 * lk + 2 * h]);
+        if (CPLX) ai[mt] = *reinterpret_cast<const v2d *>(&As[buf][P - 1][wm + mt * 16 + lr][4 * lk + 2 * h]);
+      }
 #pragma unroll
-      for (int nt = 0; nt < BN; ++nt) b[nt] = Bs[buf][0][ks + lk][wn + nt * 16 + lr];
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int mt = 0; mt < BM; ++mt)
+        for (int nt = 0; nt < BN; ++nt) {
+          b[u][nt] = Bs[buf][0][4 * lk + 2 * h + u][wn + nt * 16 + lr];
+          if (CPLX) bi[u][nt] = Bs[buf][P - 1][4 * lk + 2 * h + u][wn + nt * 16 + lr];
+        }
 #pragma unroll
-        for (int nt = 0; nt < BN; ++nt)
-          if (mt_ok[mt] && nt_ok[nt])
-            acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
-      if (CPLX) {
-        double ai[BM], bi[BN];
+      for (int mt = 0; mt < BM; ++mt) {
+        if (mt > 0 && !mt_ok[mt]) continue;
 #pragma unroll
-        for (int mt = 0; mt < BM; ++mt) ai[mt] = As[buf][P - 1][ks + lk][wm + mt * 16 + lr];
+        for (int nt = 0; nt < BN; ++nt) {
+          if (nt > 0 && !nt_ok[nt]) continue;
 #pragma unroll
-        for (int nt = 0; nt < BN; ++nt) bi[nt] = Bs[buf][P - 1][ks + lk][wn + nt * 16 + lr];
-        // three real products per complex one (Gauss): acc = sum ar*br (above),
-        // acc_i = sum ai*bi, acc_s = sum (ar + ai)*(br + bi); after the last
-        // step re = acc - acc_i and im = acc_s - acc - acc_i
-        double as[BM], bs[BN];
-#pragma unroll
-        for (int mt = 0; mt < BM; ++mt) as[mt] = a[mt] + ai[mt];
-#pragma unroll
-        for (int nt = 0; nt < BN; ++nt) bs[nt] = b[nt] + bi[nt];
-#pragma unroll
-        for (int mt = 0; mt < BM; ++mt)
-#pragma unroll
-          for (int nt = 0; nt < BN; ++nt) {
-            if (!(mt_ok[mt] && nt_ok[nt])) continue;
-            acc_i[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[mt], bi[nt], acc_i[mt][nt], 0, 0, 0);
-            acc_s[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[mt], bs[nt], acc_s[mt][nt], 0, 0, 0);
+          for (int u = 0; u < 2; ++u) {
+            acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt][u], b[u][nt], acc[mt][nt], 0, 0, 0);
+            if (CPLX) {
+              // three real products per complex one (Gauss): acc = sum ar*br,
+              // acc_i = sum ai*bi, acc_s = sum (ar + ai)*(br + bi); after the last
+              // step re = acc - acc_i and im = acc_s - acc - acc_i
+              acc_i[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[mt][u], bi[u][nt], acc_i[mt][nt], 0, 0, 0);
+              acc_s[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt][u] + ai[mt][u], b[u][nt] + bi[u][nt],
+                                                                   acc_s[mt][nt], 0, 0, 0);
+            }
           }
+        }
       }
     }
   };
 
   // ---- pipeline over this tile's steps of the (task, k-chunk) sequence ----
-  // A step stages 16 k, never crossing a task; k beyond the task's end loads
-  // as zero.
+  // A step stages 16 k, never crossing a task.  Every load is issued without
+  // a guard (guarded or in two versions of a step, the compiler waited for all
+  // loads before issuing the last one): rows and columns past the block read its first ones (their
+  // results are never stored), and contracted indices past the task read the
+  // operand block's own elements and are staged as zero.
+  const bool seg_plain = (seg.flags & (kSegAPlain | kSegBPlain)) == (kSegAPlain | kSegBPlain);
   const bool seg_affine = (seg.flags & (kSegAColAffine | kSegBRowAffine)) == (kSegAColAffine | kSegBRowAffine);
+  raw_t<E, CPLX> pa[QA], pb[QB];
+  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks, buf = 0;
+  ExecTask et = exec[t];
+  int kv = min(KC, et.k - kk);
   if (seg_affine) {
     // Output block whose every task reads A and B blocks that are affine in
     // k: A' element (r, p) at a_off + roff(r) + p * cs, B' element (p, c) at
     // b_off + p * rs + coff(c) (plain blocks: roff = r*k, cs = 1, rs = n,
     // coff = c).  Each thread keeps one pointer per element it loads, set
     // once per task (the row / column offsets decomposed there) and advanced
-    // by 16 k per step; row and column bounds are fixed for the tile, and the
-    // k bound only matters on a task's last, partial step.
-    const int ap = tid & 15, ar0 = tid >> 4;
+    // by 16 k per step.
+    const int ap = tid & 15, ar0 = tid >> 4, apl = k_place(ap);
     const int bc = tid % TNv, bp0 = tid / TNv;
     constexpr int BPS = 256 / TNv;                     // B' rows between a thread's elements
-    bool aok[QA], bok[QB];
-    const E *aptr[QA], *bptr[QB];
+    const E *aptr[QA], *bptr[QB], *a0 = A, *b0 = B;   // a0, b0: the task's blocks
     int64_t a_adv = 0, b_adv = 0;
-#pragma unroll
-    for (int q = 0; q < QA; ++q) aok[q] = i0 + ar0 + 16 * q < seg.m;
-#pragma unroll
-    for (int q = 0; q < QB; ++q) bok[q] = j0 + bc < seg.n;
     auto setup = [&](const ExecTask &e, int kk0) {
       const BlkGather &gA = ga[e.a_blk];
       const BlkGather &gB = gb[e.b_blk];
@@ -365,115 +330,168 @@ __device__ __forceinline__ void grouped_tile(
       const int64_t rs = pb_ ? seg.n : gB.rstep;
       a_adv = KC * cs * P;
       b_adv = KC * rs * P;
+      a0 = A + e.a_off * P;
+      b0 = B + e.b_off * P;
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
-        const int r = aok[q] ? i0 + ar0 + 16 * q : 0;
+        const int r = i0 + ar0 + 16 * q < seg.m ? i0 + ar0 + 16 * q : 0;
         const int64_t roff = pa_ ? static_cast<int64_t>(r) * e.k
                                  : split_offset(r, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr);
-        aptr[q] = A + (e.a_off + roff + (ap + kk0) * cs) * P;
+        aptr[q] = a0 + (roff + (ap + kk0) * cs) * P;
       }
+      const int c = j0 + bc < seg.n ? j0 + bc : 0;
+      const int64_t coff = pb_ ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc);
 #pragma unroll
-      for (int q = 0; q < QB; ++q) {
-        const int c = bok[q] ? j0 + bc : 0;
-        const int64_t coff = pb_ ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc);
-        bptr[q] = B + (e.b_off + static_cast<int64_t>(bp0 + BPS * q + kk0) * rs + coff) * P;
-      }
+      for (int q = 0; q < QB; ++q) bptr[q] = b0 + (static_cast<int64_t>(bp0 + BPS * q + kk0) * rs + coff) * P;
     };
     auto pfetch = [&](int kvalid) {
-      const bool full = kvalid >= KC;
+      if (kvalid < KC) {   // a task's last chunk: the pointers are set anew after it
+#pragma unroll
+        for (int q = 0; q < QA; ++q) aptr[q] = ap < kvalid ? aptr[q] : a0;
+#pragma unroll
+        for (int q = 0; q < QB; ++q) bptr[q] = bp0 + BPS * q < kvalid ? bptr[q] : b0;
+      }
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
-        const bool ok = aok[q] && (full || ap < kvalid);
-        pa[q] = ok ? ld_raw<E, CPLX>(aptr[q]) : raw_t<E, CPLX>{};
+        pa[q] = ld_raw<E, CPLX>(aptr[q]);
         aptr[q] += a_adv;
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
-        const bool ok = bok[q] && (full || bp0 + BPS * q < kvalid);
-        pb[q] = ok ? ld_raw<E, CPLX>(bptr[q]) : raw_t<E, CPLX>{};
+        pb[q] = ld_raw<E, CPLX>(bptr[q]);
         bptr[q] += b_adv;
       }
     };
-    auto pstage = [&](int buf) {
+    auto pstage = [&](int buf, int kvalid) {
+      if (kvalid < KC) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) zero_unless<E, CPLX>(pa[q], ap < kvalid);
+#pragma unroll
+        for (int q = 0; q < QB; ++q) zero_unless<E, CPLX>(pb[q], bp0 + BPS * q < kvalid);
+      }
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
-        As[buf][0][ap][ar0 + 16 * q] = re_of(pa[q]);
-        if (CPLX) As[buf][P - 1][ap][ar0 + 16 * q] = im_of(pa[q]);
+        As[buf][0][ar0 + 16 * q][apl] = re_of(pa[q]);
+        if (CPLX) As[buf][P - 1][ar0 + 16 * q][apl] = im_of(pa[q]);
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
-        Bs[buf][0][bp0 + BPS * q][bc] = re_of(pb[q]);
-        if (CPLX) Bs[buf][P - 1][bp0 + BPS * q][bc] = im_of(pb[q]);
+        Bs[buf][0][k_place(bp0 + BPS * q)][bc] = re_of(pb[q]);
+        if (CPLX) Bs[buf][P - 1][k_place(bp0 + BPS * q)][bc] = im_of(pb[q]);
       }
     };
-    int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks;
-    ExecTask et = exec[t];
     setup(et, kk);
-    int kv = min(KC, et.k - kk);
     pfetch(kv);
-    pstage(0);
+    pstage(0, kv);
     __syncthreads();
-    int buf = 0;
-    while (left > 0) {
-      const int left2 = left - 1;
-      int t2 = t, kk2 = kk + KC;
-      if (kk2 >= et.k) {
-        t2 = t + 1;
-        kk2 = 0;
-      }
-      const bool has_next = left2 > 0;
-      ExecTask et2 = et;
+    for (;;) {
+      --left;
       int kv2 = 0;
-      if (has_next) {
-        if (t2 != t) {
-          et2 = exec[t2];
-          setup(et2, 0);
+      if (left > 0) {
+        kk += KC;
+        if (kk >= et.k) {
+          et = exec[++t];
+          kk = 0;
+          setup(et, 0);
         }
-        kv2 = min(KC, et2.k - kk2);
+        kv2 = min(KC, et.k - kk);
         pfetch(kv2);
       }
       compute(buf, kv);
-      if (has_next) pstage(buf ^ 1);
-      __syncthreads();
-      t = t2;
-      kk = kk2;
-      et = et2;
-      kv = kv2;
-      left = left2;
+      if (left == 0) break;
       buf ^= 1;
+      pstage(buf, kv2);
+      __syncthreads();
+      kv = kv2;
     }
   } else {
-    int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks;
-    ExecTask et = exec[t];
-    task_rows(ga[et.a_blk], gb[et.b_blk], et);
-    fetch(et, ga[et.a_blk], gb[et.b_blk], kk, min(et.k, kk + KC));
-    stage(0);
+    // Other blocks: offsets decomposed per element.  The thread mapping of a
+    // chunk follows the block's innermost memory axis, chosen per task:
+    //   A' k-contiguous -> p = tid & 15, rows (tid >> 4) + 16 q;
+    //      otherwise    -> r = tid % TM, cols tid / TM + (256 / TM) q;
+    //   B' n-contiguous -> c = tid % TN, rows tid / TN + (256 / TN) q;
+    //      otherwise    -> p = tid & 15, cols (tid >> 4) + 16 q.
+    bool akf = false, bnf = false, a_plain = false, b_plain = false;
+    auto a_r = [&](int q) { return akf ? (tid >> 4) + 16 * q : tid % TMv; };
+    auto a_p = [&](int q) { return akf ? tid & 15 : tid / TMv + (256 / TMv) * q; };
+    auto b_c = [&](int q) { return bnf ? tid % TNv : (tid >> 4) + 16 * q; };
+    auto b_p = [&](int q) { return bnf ? tid / TNv + (256 / TNv) * q : tid & 15; };
+    int32_t a_row[QA], b_col[QB];
+    auto task_rows = [&](const ExecTask &e) {
+      const BlkGather &gA = ga[e.a_blk];
+      const BlkGather &gB = gb[e.b_blk];
+      a_plain = gA.plain != 0;
+      b_plain = gB.plain != 0;
+      akf = a_plain || gA.fastcol != 0;
+      bnf = b_plain || gB.fastcol != 0;
+#pragma unroll
+      for (int q = 0; q < QA; ++q) {
+        const int r = i0 + a_r(q) < seg.m ? i0 + a_r(q) : 0;
+        a_row[q] = a_plain ? r * e.k : split_offset(r, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr);
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
+        const int c = j0 + b_c(q) < seg.n ? j0 + b_c(q) : 0;
+        b_col[q] = b_plain ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc);
+      }
+    };
+    auto fetch = [&](const ExecTask &e, int k0, int kvalid) {
+      const BlkGather &gA = ga[e.a_blk];
+      const BlkGather &gB = gb[e.b_blk];
+#pragma unroll
+      for (int q = 0; q < QA; ++q) {
+        const int pk = k0 + (a_p(q) < kvalid ? a_p(q) : 0);
+        const int32_t col = a_plain ? pk : split_offset(pk, gA.cdim, gA.cstr, gA.cmag, gA.csh, L.a_nc);
+        pa[q] = ld_raw<E, CPLX>(A + (e.a_off + a_row[q] + col) * P);
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
+        const int pk = k0 + (b_p(q) < kvalid ? b_p(q) : 0);
+        const int32_t row = b_plain ? pk * seg.n : split_offset(pk, gB.rdim, gB.rstr, gB.rmag, gB.rsh, L.b_nr);
+        pb[q] = ld_raw<E, CPLX>(B + (e.b_off + row + b_col[q]) * P);
+      }
+    };
+    auto stage = [&](int buf, int kvalid) {
+      if (kvalid < KC) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) zero_unless<E, CPLX>(pa[q], a_p(q) < kvalid);
+#pragma unroll
+        for (int q = 0; q < QB; ++q) zero_unless<E, CPLX>(pb[q], b_p(q) < kvalid);
+      }
+#pragma unroll
+      for (int q = 0; q < QA; ++q) {
+        As[buf][0][a_r(q)][k_place(a_p(q))] = re_of(pa[q]);
+        if (CPLX) As[buf][P - 1][a_r(q)][k_place(a_p(q))] = im_of(pa[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q) {
+        Bs[buf][0][k_place(b_p(q))][b_c(q)] = re_of(pb[q]);
+        if (CPLX) Bs[buf][P - 1][k_place(b_p(q))][b_c(q)] = im_of(pb[q]);
+      }
+    };
+    task_rows(et);
+    fetch(et, kk, kv);
+    stage(0, kv);
     __syncthreads();
-    int buf = 0;
-    while (left > 0) {
-      const int left2 = left - 1;
-      int t2 = t, kk2 = kk + KC;
-      if (kk2 >= et.k) {
-        t2 = t + 1;
-        kk2 = 0;
-      }
-      const bool has_next = left2 > 0;
-      ExecTask et2 = et;
-      if (has_next) {
-        if (t2 != t) {
-          et2 = exec[t2];
-          task_rows(ga[et2.a_blk], gb[et2.b_blk], et2);
+    for (;;) {
+      --left;
+      int kv2 = 0;
+      if (left > 0) {
+        kk += KC;
+        if (kk >= et.k) {
+          et = exec[++t];
+          kk = 0;
+          task_rows(et);
         }
-        fetch(et2, ga[et2.a_blk], gb[et2.b_blk], kk2, min(et2.k, kk2 + KC));
+        kv2 = min(KC, et.k - kk);
+        fetch(et, kk, kv2);
       }
-      compute(buf, min(et.k - kk, KC));
-      if (has_next) stage(buf ^ 1);
-      __syncthreads();
-      t = t2;
-      kk = kk2;
-      et = et2;
-      left = left2;
+      compute(buf, kv);
+      if (left == 0) break;
       buf ^= 1;
+      stage(buf, kv2);
+      __syncthreads();
+      kv = kv2;
     }
   }
 
@@ -567,7 +585,7 @@ __device__ __forceinline__ void narrow_tile(
     double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
   constexpr int KW = kNarrowWaves, BM = kNarrowM / 16;
-  constexpr int KS = (CPLX && sizeof(E) == 8) ? 2 : 4;   // k-steps of 4 per stage
+  constexpr int KS = sizeof(E) == 8 ? 2 : 4;   // k-steps of 4 per stage (their registers bound k_all_classes)
   constexpr int SK = 4 * KS;
   constexpr bool kLaneRuns = sizeof(E) * P <= 8;
   using R = raw_t<E, CPLX>;
@@ -829,7 +847,7 @@ __device__ __forceinline__ void reduce_slices(const ReduceItem it, const Seg &se
 // accumulates its n outputs with FP64 FMAs.  Bound by reading A and writing
 // C once.
 constexpr int RK = 16;            // k per stage
-constexpr int kRowsLoadGroup = 16;   // A loads in flight per thread
+constexpr int kRowsLoadGroup = 8;   // A loads in flight per thread
 
 template <bool CPLX, int NMAX, int RPT, typename E>
 __device__ __forceinline__ void rows_epilogue(const Seg &seg, int r0, int tid, const double (&acc)[RPT][NMAX],
@@ -1298,9 +1316,10 @@ __global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
 // one: U(1) FP64 matvec at D = 96 103 -> 32 us, D = 700 164 -> 43 us, lognormal
 // 184 -> 117 us, U(1)xU(1) complex128 D = 1500 252 -> 156 us, D = 4096 1.22 ->
 // 1.18 ms.  The register bound keeps the occupancy of the widest class alone
-// (complex: three workgroups per CU; unbounded, two, and D = 4096 took 1.35 ms).
+// (complex: three workgroups per CU; unbounded, two, and D = 4096 took 1.35 ms;
+// real: five, with D = 2048 FP64 285 -> 272 us from four; six spill).
 template <bool CPLX, bool STREAM, typename E>
-__global__ __launch_bounds__(256, CPLX ? 3 : 4) void k_all_classes(const ExecArgs<E> x) {
+__global__ __launch_bounds__(256, CPLX ? 3 : 5) void k_all_classes(const ExecArgs<E> x) {
   constexpr size_t kBytes = std::max({class_shared<CPLX, 1>(), class_shared<CPLX, 3>(), class_shared<CPLX, 4>(),
                                       class_shared<CPLX, 5>(), sizeof(PanelShared<CPLX>)});
   __shared__ __align__(16) char smem[kBytes];
