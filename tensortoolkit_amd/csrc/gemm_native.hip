@@ -99,6 +99,42 @@ __device__ __forceinline__ void st_elem(E *p, double re, double im) {
   }
 }
 
+// Offset of a linear index inside a block over one part's axes (split_offset),
+// with the descriptor's numbers read once per task: up to two axes take one
+// multiply-shift division and no further reads, more take the loop, whose
+// scalar reads of every axis are waited for at every element (they were most
+// of a step of a contraction not affine in k: a U(1) chi = 40 pair of rank-4
+// tensors over cyclic axes, complex64, 99 -> 51 us, FP64 79 -> 38 us).
+struct PartSplit {
+  const BlkGather *g;
+  int n;
+  uint64_t mag;      // of the inner of two axes; 0: one axis
+  int32_t sh, dim, outer, inner;
+};
+template <bool ROW>
+__device__ __forceinline__ PartSplit part_split(const BlkGather &g, int n) {
+  PartSplit p{&g, n, 0, 0, 1, 0, 0};
+  const int32_t *strs = ROW ? g.rstr : g.cstr;
+  if (n == 1) {
+    p.inner = strs[0];
+  } else if (n == 2) {
+    p.mag = ROW ? g.rmag[1] : g.cmag[1];
+    p.sh = ROW ? g.rsh[1] : g.csh[1];
+    p.dim = ROW ? g.rdim[1] : g.cdim[1];
+    p.outer = strs[0];
+    p.inner = strs[1];
+  }
+  return p;
+}
+template <bool ROW>
+__device__ __forceinline__ int32_t offset_of(const PartSplit &p, int32_t x) {
+  if (p.n > 2)
+    return ROW ? split_offset(x, p.g->rdim, p.g->rstr, p.g->rmag, p.g->rsh, p.n)
+               : split_offset(x, p.g->cdim, p.g->cstr, p.g->cmag, p.g->csh, p.n);
+  const int32_t q = static_cast<int32_t>((static_cast<uint64_t>(x) * p.mag) >> p.sh);
+  return q * p.outer + (x - q * p.dim) * p.inner;
+}
+
 // Epilogue of one output element: C = alpha * x + beta * old, with `old` the
 // element's earlier value, loaded by the caller beforehand (not read when
 // beta == 0).  The epilogues load every old value of a thread first, at
@@ -332,15 +368,17 @@ __device__ __forceinline__ void grouped_tile(
       b_adv = KC * rs * P;
       a0 = A + e.a_off * P;
       b0 = B + e.b_off * P;
+      PartSplit a_m{}, b_n{};
+      if (!pa_) a_m = part_split<true>(gA, L.a_nr);
+      if (!pb_) b_n = part_split<false>(gB, L.b_nc);
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
         const int r = i0 + ar0 + 16 * q < seg.m ? i0 + ar0 + 16 * q : 0;
-        const int64_t roff = pa_ ? static_cast<int64_t>(r) * e.k
-                                 : split_offset(r, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr);
+        const int64_t roff = pa_ ? static_cast<int64_t>(r) * e.k : offset_of<true>(a_m, r);
         aptr[q] = a0 + (roff + (ap + kk0) * cs) * P;
       }
       const int c = j0 + bc < seg.n ? j0 + bc : 0;
-      const int64_t coff = pb_ ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc);
+      const int64_t coff = pb_ ? c : offset_of<false>(b_n, c);
 #pragma unroll
       for (int q = 0; q < QB; ++q) bptr[q] = b0 + (static_cast<int64_t>(bp0 + BPS * q + kk0) * rs + coff) * P;
     };
@@ -417,6 +455,7 @@ __device__ __forceinline__ void grouped_tile(
     auto b_c = [&](int q) { return bnf ? tid % TNv : (tid >> 4) + 16 * q; };
     auto b_p = [&](int q) { return bnf ? tid / TNv + (256 / TNv) * q : tid & 15; };
     int32_t a_row[QA], b_col[QB];
+    PartSplit a_k{}, b_k{};
     auto task_rows = [&](const ExecTask &e) {
       const BlkGather &gA = ga[e.a_blk];
       const BlkGather &gB = gb[e.b_blk];
@@ -424,30 +463,32 @@ __device__ __forceinline__ void grouped_tile(
       b_plain = gB.plain != 0;
       akf = a_plain || gA.fastcol != 0;
       bnf = b_plain || gB.fastcol != 0;
+      a_k = part_split<false>(gA, L.a_nc);
+      b_k = part_split<true>(gB, L.b_nr);
+      const PartSplit a_m = part_split<true>(gA, L.a_nr);
+      const PartSplit b_n = part_split<false>(gB, L.b_nc);
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
         const int r = i0 + a_r(q) < seg.m ? i0 + a_r(q) : 0;
-        a_row[q] = a_plain ? r * e.k : split_offset(r, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr);
+        a_row[q] = a_plain ? r * e.k : offset_of<true>(a_m, r);
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
         const int c = j0 + b_c(q) < seg.n ? j0 + b_c(q) : 0;
-        b_col[q] = b_plain ? c : split_offset(c, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc);
+        b_col[q] = b_plain ? c : offset_of<false>(b_n, c);
       }
     };
     auto fetch = [&](const ExecTask &e, int k0, int kvalid) {
-      const BlkGather &gA = ga[e.a_blk];
-      const BlkGather &gB = gb[e.b_blk];
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
         const int pk = k0 + (a_p(q) < kvalid ? a_p(q) : 0);
-        const int32_t col = a_plain ? pk : split_offset(pk, gA.cdim, gA.cstr, gA.cmag, gA.csh, L.a_nc);
+        const int32_t col = a_plain ? pk : offset_of<false>(a_k, pk);
         pa[q] = ld_raw<E, CPLX>(A + (e.a_off + a_row[q] + col) * P);
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
         const int pk = k0 + (b_p(q) < kvalid ? b_p(q) : 0);
-        const int32_t row = b_plain ? pk * seg.n : split_offset(pk, gB.rdim, gB.rstr, gB.rmag, gB.rsh, L.b_nr);
+        const int32_t row = b_plain ? pk * seg.n : offset_of<true>(b_k, pk);
         pb[q] = ld_raw<E, CPLX>(B + (e.b_off + row + b_col[q]) * P);
       }
     };
@@ -626,38 +667,36 @@ __device__ __forceinline__ void narrow_tile(
   // per task: element pointers of this lane's rows and column at k = 0, and
   // how an index k moves them
   const E *ap[BM], *bp = nullptr;
-  const BlkGather *gA = nullptr, *gB = nullptr;
+  PartSplit a_k{}, b_k{};
   bool a_aff = false, b_aff = false;
   int cs = 1, rs = 1, cur = -1;
   auto setup = [&]() {
     cur = t;
     const ExecTask et = exec[t];
-    gA = ga + et.a_blk;
-    gB = gb + et.b_blk;
-    const bool a_plain = (seg.flags & kSegAPlain) || gA->plain != 0;
-    const bool b_plain = (seg.flags & kSegBPlain) || gB->plain != 0;
-    a_aff = (seg.flags & kSegAColAffine) || a_plain || gA->caff != 0;
-    b_aff = (seg.flags & kSegBRowAffine) || b_plain || gB->raff != 0;
-    cs = a_plain ? 1 : gA->cstep;
-    rs = b_plain ? seg.n : gB->rstep;
+    const BlkGather &gA = ga[et.a_blk];
+    const BlkGather &gB = gb[et.b_blk];
+    const bool a_plain = (seg.flags & kSegAPlain) || gA.plain != 0;
+    const bool b_plain = (seg.flags & kSegBPlain) || gB.plain != 0;
+    a_aff = (seg.flags & kSegAColAffine) || a_plain || gA.caff != 0;
+    b_aff = (seg.flags & kSegBRowAffine) || b_plain || gB.raff != 0;
+    cs = a_plain ? 1 : gA.cstep;
+    rs = b_plain ? seg.n : gB.rstep;
+    PartSplit a_m{}, b_n{};
+    if (!a_plain) a_m = part_split<true>(gA, L.a_nr);
+    if (!b_plain) b_n = part_split<false>(gB, L.b_nc);
+    if (!a_aff) a_k = part_split<false>(gA, L.a_nc);
+    if (!b_aff) b_k = part_split<true>(gB, L.b_nr);
 #pragma unroll
     for (int mt = 0; mt < BM; ++mt) {
       int r = i0 + 16 * mt + lr;
       r = r < seg.m ? r : 0;
-      const int64_t off = a_plain ? static_cast<int64_t>(r) * et.k
-                                  : split_offset(r, gA->rdim, gA->rstr, gA->rmag, gA->rsh, L.a_nr);
-      ap[mt] = A + (et.a_off + off) * P;
+      ap[mt] = A + (et.a_off + (a_plain ? static_cast<int64_t>(r) * et.k : offset_of<true>(a_m, r))) * P;
     }
     const int c = lr < seg.n ? lr : 0;
-    const int64_t off = b_plain ? c : split_offset(c, gB->cdim, gB->cstr, gB->cmag, gB->csh, L.b_nc);
-    bp = B + (et.b_off + off) * P;
+    bp = B + (et.b_off + (b_plain ? c : offset_of<false>(b_n, c))) * P;
   };
-  auto a_off = [&](int k) -> int64_t {
-    return a_aff ? static_cast<int64_t>(k) * cs : split_offset(k, gA->cdim, gA->cstr, gA->cmag, gA->csh, L.a_nc);
-  };
-  auto b_off = [&](int k) -> int64_t {
-    return b_aff ? static_cast<int64_t>(k) * rs : split_offset(k, gB->rdim, gB->rstr, gB->rmag, gB->rsh, L.b_nr);
-  };
+  auto a_off = [&](int k) -> int64_t { return a_aff ? static_cast<int64_t>(k) * cs : offset_of<false>(a_k, k); };
+  auto b_off = [&](int k) -> int64_t { return b_aff ? static_cast<int64_t>(k) * rs : offset_of<true>(b_k, k); };
   // the stage at (t, kk) into register set `s`; returns its valid extent
   auto load = [&](int s) {
     if (t != cur) setup();
@@ -927,6 +966,7 @@ __device__ __forceinline__ void rows_tile(
   int t = tile.t_begin, kk = tile.k_begin;
   ExecTask et{};
   bool a_plain = false, b_plain = false;
+  PartSplit a_k{}, b_k{};
   int32_t roff[RPT];
   int cur_task = -1;
   for (int step = 0; step < tile.n_chunks; ++step) {
@@ -937,23 +977,24 @@ __device__ __forceinline__ void rows_tile(
       const BlkGather &gB = gb[et.b_blk];
       a_plain = gA.plain != 0;
       b_plain = gB.plain != 0;
+      a_k = part_split<false>(gA, L.a_nc);
+      b_k = part_split<true>(gB, L.b_nr);
+      const PartSplit a_m = part_split<true>(gA, L.a_nr);
+      const PartSplit b_n = part_split<false>(gB, L.b_nc);
 #pragma unroll
       for (int q = 0; q < RPT; ++q) {
         const int row = r0 + tid + 256 * q;
-        roff[q] = (row < seg.m) ? (a_plain ? row * et.k : split_offset(row, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr)) : -1;
+        roff[q] = (row < seg.m) ? (a_plain ? row * et.k : offset_of<true>(a_m, row)) : -1;
       }
       __syncthreads();
-      if (tid < NMAX)
-        s_bcol[tid] = (tid < n) ? (b_plain ? tid : split_offset(tid, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc)) : -1;
+      if (tid < NMAX) s_bcol[tid] = (tid < n) ? (b_plain ? tid : offset_of<false>(b_n, tid)) : -1;
     }
-    const BlkGather &gA = ga[et.a_blk];
-    const BlkGather &gB = gb[et.b_blk];
     if (tid < RK) {
       const int p = kk + tid;
-      s_acol[tid] = (p < et.k) ? (a_plain ? p : split_offset(p, gA.cdim, gA.cstr, gA.cmag, gA.csh, L.a_nc)) : -1;
+      s_acol[tid] = (p < et.k) ? (a_plain ? p : offset_of<false>(a_k, p)) : -1;
     } else if (tid >= 64 && tid < 64 + RK) {
       const int p = kk + tid - 64;
-      s_brow[tid - 64] = (p < et.k) ? (b_plain ? p * n : split_offset(p, gB.rdim, gB.rstr, gB.rmag, gB.rsh, L.b_nr)) : -1;
+      s_brow[tid - 64] = (p < et.k) ? (b_plain ? p * n : offset_of<true>(b_k, p)) : -1;
     }
     __syncthreads();
     if (tid < RK * NMAX) {

@@ -1051,6 +1051,14 @@ qlt_status qlt_plan_build(const qlt_bsdt_desc *a, const qlt_bsdt_desc *b, int32_
         ExecTask{a_off, b_off, dt.a_pos, dt.b_pos, static_cast<int32_t>(k), 0};
   }
   const int64_t n_c = static_cast<int64_t>(segs.size());
+  for (Seg &sg : segs)
+    if (sg.cls == kTileRows4 && sg.k_total > kRows4MaxK) {
+      const int64_t was = tiles_of(sg.cls, sg.m, sg.n);
+      sg.cls = kTileRows16;
+      plan->cls_tiles[kTileRows4] -= was;
+      plan->cls_tiles[kTileRows16] += tiles_of(sg.cls, sg.m, sg.n);
+      n_tiles += tiles_of(sg.cls, sg.m, sg.n) - was;
+    }
   QLT_CHECK_ARG(n_tiles < (int64_t(1) << 31), "qlt_plan_build: more than 2^31 output tiles");
   QLT_CHECK_ARG(kmax < (int64_t(1) << 40), "qlt_plan_build: contracted extent of an output block exceeds 2^40");
   plan->n_exec = nt;

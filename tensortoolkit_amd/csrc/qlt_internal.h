@@ -166,6 +166,12 @@ constexpr int32_t kNumMfmaClasses = 4;
 constexpr int32_t kTileRows4 = 4;
 constexpr int32_t kTileRows16 = 5;
 constexpr int32_t kNumTileClasses = 6;
+// An n <= 4 block of a longer contracted extent runs with the n <= 16 class: a
+// row tile walks its 16-k steps one after the other, about 1.5 us each, where
+// an MFMA tile's waves share them (a U(1) chi = 16 pair of rank-4 tensors, FP64: 43 ->
+// 13 us).  Beyond
+// kPanelCols, so that what a row panel may take stays with the row class.
+constexpr int64_t kRows4MaxK = 64;
 
 __host__ __device__ constexpr int32_t mfma_tile_m(int32_t cls) { return (cls == 1 || cls == 3) ? 32 : 64; }
 __host__ __device__ constexpr int32_t mfma_tile_n(int32_t cls) { return (cls == 2 || cls == 3) ? 32 : 64; }
