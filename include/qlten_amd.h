@@ -346,6 +346,9 @@ qlt_status qlt_scale_segments_noalloc(int32_t dtype, int64_t n_segs, const int64
  * qlt_lanczos_extend: with j = m - 1: alphas[j] = Re c[2j], betas[j] = |w|,
  *                   V_m = w / |w| (zero when |w| = 0) if m < k_max, then
  *                   m = m + 1 (when m < k_max).  work as for qlt_basis_dot.
+ * qlt_lanczos_update_extend: qlt_basis_update by scale * c_update, then
+ *                   qlt_lanczos_extend of the updated w, with bitwise the
+ *                   same results as the two calls, in one pass over w less.
  * qlt_basis_select: x = V_{*index + offset} (no-op outside 0 .. k_max-1). */
 #define QLT_BASIS_WORK_DOUBLES(k_max) (2 * 512 * (k_max) + 1)
 qlt_status qlt_basis_dot(int32_t dtype, int64_t n, int32_t k_max, const int32_t *count, const void *V, int64_t ldv,
@@ -358,6 +361,9 @@ qlt_status qlt_basis_update_dot(int32_t dtype, int64_t n, int32_t k_max, const i
 qlt_status qlt_lanczos_extend(int32_t dtype, int64_t n, int32_t k_max, int32_t *count, const double *c,
                               const void *w, void *V, int64_t ldv, double *alphas, double *betas, double *work,
                               void *stream);
+qlt_status qlt_lanczos_update_extend(int32_t dtype, int64_t n, int32_t k_max, int32_t *count, const double *c,
+                                     double scale, const double *c_update, void *w, void *V, int64_t ldv,
+                                     double *alphas, double *betas, double *work, void *stream);
 qlt_status qlt_basis_select(int32_t dtype, int64_t n, int32_t k_max, const int32_t *index, int32_t offset,
                             const void *V, int64_t ldv, void *x, void *stream);
 

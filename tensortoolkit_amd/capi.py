@@ -164,6 +164,9 @@ _SIGS = {
                               C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int32),
     "qlt_lanczos_extend": ([C.c_int32, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                             C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p], C.c_int32),
+    "qlt_lanczos_update_extend": ([C.c_int32, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p, C.c_double, C.c_void_p,
+                                   C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p,
+                                   C.c_void_p], C.c_int32),
     "qlt_basis_select": ([C.c_int32, C.c_int64, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p, C.c_int64,
                           C.c_void_p, C.c_void_p], C.c_int32),
     "qlt_copy_blocks_2d": ([C.c_int32, C.c_int64, _i64p, _i64p, C.c_void_p, _i64p, _i64p, C.c_void_p, _i64p, _i64p,

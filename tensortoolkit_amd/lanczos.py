@@ -177,14 +177,13 @@ class KrylovArena:
         capi.check(lib.qlt_basis_select(dt, n, k, self.count.ptr, -1, self.V.ptr, n, self.x.ptr, st))
         self.hv.apply(self.x.ptr, self.w.ptr)
         # pass 1: c1 = V^H w; w -= V c1 together with pass 2's c2 = V^H w
-        # (one read of the basis for both); pass 2: w -= V c2
+        # (one read of the basis for both); pass 2: w -= V c2 together with |w|
         capi.check(lib.qlt_basis_dot(dt, n, k, self.count.ptr, self.V.ptr, n, self.w.ptr, self.c1.ptr,
                                      self.work.ptr, st))
         capi.check(lib.qlt_basis_update_dot(dt, n, k, self.count.ptr, -1.0, self.c1.ptr, self.V.ptr, n, self.w.ptr,
                                             self.c2.ptr, self.work.ptr, st))
-        capi.check(lib.qlt_basis_update(dt, n, k, self.count.ptr, -1.0, self.c2.ptr, self.V.ptr, n, self.w.ptr, st))
-        capi.check(lib.qlt_lanczos_extend(dt, n, k, self.count.ptr, self.c1.ptr, self.w.ptr, self.V.ptr, n,
-                                          self.alphas.ptr, self.betas.ptr, self.work.ptr, st))
+        capi.check(lib.qlt_lanczos_update_extend(dt, n, k, self.count.ptr, self.c1.ptr, -1.0, self.c2.ptr, self.w.ptr,
+                                                 self.V.ptr, n, self.alphas.ptr, self.betas.ptr, self.work.ptr, st))
 
     def coefficients(self):
         capi.check(capi.lib().qlt_stream_sync(self.hv.stream))
