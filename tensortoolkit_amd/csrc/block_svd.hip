@@ -132,9 +132,10 @@ __global__ void __launch_bounds__(kThreads) k_svd_norms(const SvdMat *mats, cons
 }
 
 // The matrix's squared column norms into sn[0..N), then ord[rank] = column
-// by decreasing norm (ties by column index).
+// by decreasing norm (ties by column index; a NaN norm counts as the least, so
+// that every rank is taken once and the order stays a permutation).
 __device__ void order_by_norms(const double *norms, int64_t N, double *sn, int32_t *ord) {
-  for (int64_t c = threadIdx.x; c < N; c += kThreads) sn[c] = norms[c];
+  for (int64_t c = threadIdx.x; c < N; c += kThreads) sn[c] = norms[c] >= 0.0 ? norms[c] : -1.0;
   __syncthreads();
   for (int64_t c = threadIdx.x; c < N; c += kThreads) {
     const double v = sn[c];
