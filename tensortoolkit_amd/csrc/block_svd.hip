@@ -13,9 +13,10 @@
 //      matrix G = P^H P of the panel P = [X_I X_J],
 //   2. one workgroup sums the parts in group order, skips the pair when
 //      max |G_pq| / sqrt(G_pp G_qq) < tol, and otherwise diagonalises G in
-//      LDS by cyclic two-sided Jacobi (at most kInnerSweeps sweeps),
-//      accumulating the unitary Q (G <- J^H G J, Q <- Q J per rotation),
-//   3. one workgroup per kRG-row group updates P <- P Q and the matching
+//      LDS by one sweep of cyclic two-sided Jacobi, accumulating the unitary
+//      Q (G <- J^H G J, Q <- Q J per rotation; the outer sweeps repeat the
+//      pair until its columns are orthogonal, so the solve need not finish),
+//   3. one workgroup per kUR-row group updates P <- P Q and the matching
 //      columns of V <- V Q.
 // Spreading the rows over workgroups keeps the chip busy on the few large
 // block matrices, whose pairs set the length of a round.
@@ -39,11 +40,9 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kB = 16;          // columns per Jacobi block
 constexpr int kW = 2 * kB;      // panel width
-constexpr int kRG = 64;         // rows per Gram / update workgroup
+constexpr int kRG = 64;         // rows per Gram workgroup
+constexpr int kUR = 32;         // rows per update workgroup
 constexpr int kMaxSweeps = 40;
-// Sweeps of the pair's Jacobi eigen-solve per visit: the outer sweeps repeat
-// the pair until its columns are orthogonal, so the solve need not finish.
-constexpr int kInnerSweeps = 1;
 constexpr int kMaxSortCols = 4096;   // LDS bound of the per-matrix column sort
 
 struct SvdMat {
@@ -66,7 +65,8 @@ struct SvdItem {
   int32_t k;          // pair index within a round
 };
 
-// One row group of one pair: rows g * kRG .. of X (kind 0) or of V (kind 1).
+// One row group of one pair: rows g * kRG .. of X (phase 1), or g * kUR .. of X
+// (kind 0) or V (kind 1; phase 3).
 struct SvdRowItem {
   int32_t mat;
   int32_t k;
@@ -79,15 +79,33 @@ struct SvdRowItem {
 // conditional subtraction reduces them modulo players - 1.
 __device__ __forceinline__ void circle_pair(int players, int r, int k, int &a, int &b) {
   const int m = players - 1;
-  if (k == 0) {
-    a = m;
-    b = r;
-  } else {
-    a = r + k;
-    if (a >= m) a -= m;
-    b = r - k + m;
-    if (b >= m) b -= m;
-  }
+  const int x = r + k, y = r - k + m;
+  a = k == 0 ? m : x >= m ? x - m : x;
+  b = y >= m ? y - m : y;
+}
+
+// The arithmetic of a rotation, its fused multiply-adds written out: what the
+// compiler fuses depends on the code around, and the phases of the singular
+// vectors hang on the last bits of inner products that are only rounding.
+__device__ __forceinline__ double sq_(double a) { return a * a; }
+__device__ __forceinline__ double sq_(cplx a) { return fma(a.x, a.x, a.y * a.y); }
+// e * b, and conj(e) * b
+__device__ __forceinline__ double phase_(double e, double b) { return e * b; }
+__device__ __forceinline__ cplx phase_(cplx e, cplx b) {
+  return {fma(e.x, b.x, -(e.y * b.y)), fma(e.y, b.x, e.x * b.y)};
+}
+__device__ __forceinline__ double cphase_(double e, double b) { return e * b; }
+__device__ __forceinline__ cplx cphase_(cplx e, cplx b) {
+  return {fma(e.x, b.x, e.y * b.y), fma(e.x, b.y, -(e.y * b.x))};
+}
+// c a - s b, and s a + c b
+__device__ __forceinline__ double rot_p(double c, double s, double a, double b) { return fma(c, a, -(s * b)); }
+__device__ __forceinline__ cplx rot_p(double c, double s, cplx a, cplx b) {
+  return {rot_p(c, s, a.x, b.x), rot_p(c, s, a.y, b.y)};
+}
+__device__ __forceinline__ double rot_q(double c, double s, double a, double b) { return fma(s, a, c * b); }
+__device__ __forceinline__ cplx rot_q(double c, double s, cplx a, cplx b) {
+  return {rot_q(c, s, a.x, b.x), rot_q(c, s, a.y, b.y)};
 }
 
 template <bool C>
@@ -181,29 +199,34 @@ __device__ __forceinline__ bool pair_cols(const SvdMat &mt, int32_t round, int32
   return true;
 }
 
-// Round phase 1: the partial Gram matrix P^H P of one kRG-row group of the
-// pair's panel P = [X_I X_J], stored w x w with row stride kW.
 // Stage rows rb .. re of the panel's w columns (column c = X column sCol[c])
 // into LDS as real and imaginary planes sP[part][c][row], zero beyond the
-// rows and columns.
-template <bool C, typename T>
+// rows and columns.  The loads carry no guards (past the panel they read its
+// last row or column): guarded, each was waited for before the next (a Gram
+// launch of the D = 2048 complex128 SVD 10.8 -> 9.7 us).
+template <bool C, int R, typename T>
 __device__ __forceinline__ void stage_panel(const T *base, int64_t rows, int64_t rb, int64_t re, int w,
-                                            const int32_t *sCol, double (*sP)[kW][kRG + 1]) {
-  for (int idx = threadIdx.x; idx < kW * kRG; idx += kThreads) {
-    const int c = idx / kRG, rr = idx - c * kRG;
-    const int64_t row = rb + rr;
-    T v = zero_<T>();
-    if (c < w && row < re) v = base[int64_t(sCol[c]) * rows + row];
+                                            const int32_t *sCol, double (*sP)[kW][R + 1]) {
+  constexpr int kCols = kThreads / R;   // columns per pass: consecutive threads take consecutive rows
+  const int rr = threadIdx.x % R, c0 = threadIdx.x / R;
+  const int64_t row = min<int64_t>(rb + rr, re - 1);
+  T v[kW / kCols];
+#pragma unroll
+  for (int j = 0; j < kW / kCols; ++j) v[j] = base[int64_t(sCol[min(c0 + j * kCols, w - 1)]) * rows + row];
+#pragma unroll
+  for (int j = 0; j < kW / kCols; ++j) {
+    const int c = c0 + j * kCols;
+    const bool in = c < w && rb + rr < re;
     if constexpr (C) {
-      sP[0][c][rr] = v.x;
-      sP[1][c][rr] = v.y;
+      sP[0][c][rr] = in ? v[j].x : 0.0;
+      sP[1][c][rr] = in ? v[j].y : 0.0;
     } else {
-      sP[0][c][rr] = v;
+      sP[0][c][rr] = in ? v[j] : 0.0;
     }
   }
 }
 
-// One row group's part of the pair's Gram matrix, G = P^H P over rows
+// Round phase 1: one row group's part of the pair's Gram matrix, G = P^H P over rows
 // g kRG .. (g + 1) kRG - 1, on v_mfma_f64_16x16x4f64: wave wv computes the
 // 16 x 16 tile (wv / 2, wv % 2) of the 32 x 32 result over 16 k-steps of 4
 // rows.  Complex: Re G = Pr^T Pr + Pi^T Pi, Im G = Pr^T Pi - Pi^T Pr.
@@ -216,15 +239,15 @@ __global__ void __launch_bounds__(kThreads) k_svd_gram(const SvdMat *mats, const
   __shared__ double sP[PARTS][kW][kRG + 1];
   __shared__ int32_t sCol[kW];
   const SvdRowItem it = items[blockIdx.x];
-  if (!active[it.mat]) return;
   const SvdMat mt = mats[it.mat];
+  if (!active[it.mat]) return;
   int w = 0;
   if (!pair_cols(mt, round, it.k, perm, sCol, w)) return;
   const int tid = threadIdx.x;
   const T *X = static_cast<const T *>(ws_) + mt.x_off;
   __syncthreads();
   const int64_t rb = int64_t(it.g) * kRG, re = min<int64_t>(mt.M, rb + kRG);
-  stage_panel<C>(X, mt.M, rb, re, w, sCol, sP);
+  stage_panel<C, kRG>(X, mt.M, rb, re, w, sCol, sP);
   __syncthreads();
   const int lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
   const int p0 = 16 * (wv >> 1), q0 = 16 * (wv & 1);
@@ -255,54 +278,186 @@ __global__ void __launch_bounds__(kThreads) k_svd_gram(const SvdMat *mats, const
 }
 
 // Round phase 2, one workgroup per pair: the Gram matrix as the sum of the
-// row groups' partials (in group order), the pair's convergence test, and the
-// cyclic two-sided Jacobi eigen-solve of the Gram in LDS, whose unitary Q
-// (w x w, row stride kW) phase 3 applies.  qflag = 1 when Q is to be applied.
+// row groups' partials (in group order), the pair's convergence test, and one
+// sweep of the cyclic two-sided Jacobi eigen-solve of the Gram in LDS, whose
+// unitary Q (w x w, row stride kW) phase 3 applies.  qflag = 1 when Q is to be
+// applied.
+//
+// What bounds it: the chain of each of the sweep's w - 1 rounds (read G, a
+// rotation's square roots and divisions, apply, write G, barrier), with one
+// workgroup per pair and far fewer pairs than CUs.  So everything that is
+// not on that chain is kept off it: Q has waves of its own, which share the
+// SIMDs with the chain's; a thread's column rotation is the one its lane has
+// computed, only the row rotation comes by shuffle; the entries of G a thread
+// works on are read before the rotation is known.  A visit in a U(1)xU(1) D = 2048
+// complex128 SVD: 47.6 us with G and Q in the same waves and all rotations by
+// shuffle, 37.2 with waves for Q, 29.6 with the rows of kS entries; of a round's
+// 1.0 us a rotation's square roots and divisions are 0.4.
+constexpr int kSolveThreads = 512;
+// Row stride of G and Q in LDS: even, so that the entries (p, q) and (p, p) of
+// the 16 pairs of a round, which lie along an antidiagonal and the diagonal,
+// fall into different banks.
+constexpr int kS = kW + 2;
+
+// A sweep applies, round by round, the rotations of P2 / 2 disjoint index
+// pairs, G <- J^H G J and Q <- Q J, as 2 x 2 blocks: thread (bi, bj) of the
+// waves of G takes the block of G at rows (p, q) of pair bi and columns of
+// pair bj, applies the rotation of pair bj to its columns and then that of
+// pair bi to its rows (the same operations, in the same order, as a column
+// pass followed by a row pass), and writes the result into the other G
+// buffer; thread (bi, bj) of the waves of Q rotates rows 2 bi, 2 bi + 1 of Q
+// in the columns of pair bj, in place.  Every wave computes the round's
+// rotations from the round's G, pair k in lane k (and its copies k + 16, ...),
+// so that a lane's own is that of pair bj, and a round takes one barrier: both
+// kinds of waves pass the same number of them.  w odd: the pair with index w
+// is off, and what stands in its row and column of G reaches no other.
+template <bool C, bool FORQ, typename T = typename ElemOf<C>::T>
+__device__ __forceinline__ void jacobi_sweep(T (*sG)[kW][kS], T (*sQ)[kS], int w) {
+  const int P2 = w + (w & 1);
+  const double eps = 2.220446049250313e-16;
+  const int bi = (threadIdx.x % (kSolveThreads / 2)) / (kW / 2), bj = threadIdx.x % (kW / 2);
+  const bool blk_on = bi < P2 / 2 && bj < P2 / 2;
+  const int ki = min(bi, P2 / 2 - 1), kj = min(bj, P2 / 2 - 1);   // in range: nothing of other threads is stored
+  int cur = 0;
+  for (int r = 0; r < P2 - 1; ++r) {
+    const T(*G)[kS] = sG[cur];
+    int rows[2], cols[2];
+    circle_pair(P2, r, kj, cols[0], cols[1]);
+    if (FORQ) {
+      rows[0] = 2 * ki;
+      rows[1] = 2 * ki + 1;
+    } else {
+      circle_pair(P2, r, ki, rows[0], rows[1]);
+    }
+    const double al = re_(G[cols[0]][cols[0]]), be = re_(G[cols[1]][cols[1]]);
+    const T g = G[cols[0]][cols[1]];
+    T x[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) x[a][b] = FORQ ? sQ[rows[a]][cols[b]] : G[rows[a]][cols[b]];
+    // the rotation of pair bj: c, s and the unit phase; off (identity) when
+    // the pair is orthogonal or padded.  |g| > eps sqrt(al be), squared: three
+    // square roots and three divisions per rotation.
+    const double ag2 = sq_(g);
+    const bool onj = (cols[0] < w) & (cols[1] < w) & (ag2 > 0.0) & (al > 0.0) & (be > 0.0) &
+                     (ag2 > (eps * eps) * (al * be));
+    const double ag = sqrt(ag2);
+    const double inv = 1.0 / ag;
+    const double zeta = (be - al) * (0.5 * inv);
+    const bool far = fabs(zeta) > 1e150;
+    const double num = far ? 0.5 : (zeta >= 0.0 ? 1.0 : -1.0);
+    const double den = far ? zeta : fabs(zeta) + sqrt(fma(zeta, zeta, 1.0));
+    const double t = num / den;
+    const double cj = 1.0 / sqrt(fma(t, t, 1.0));
+    const double sj = cj * t;
+    const T emj = uphase_conj_inv(g, inv);
+    double ci = 0.0, si = 0.0;
+    T emi = emj;
+    bool oni = false;
+    if (!FORQ) {
+      ci = __shfl(cj, bi);
+      si = __shfl(sj, bi);
+      emi = shfl_(emj, bi);
+      oni = __shfl(onj ? 1 : 0, bi) != 0;
+    }
+    // columns:  [x_p, x_q] <- [x_p, x_q] J,  J = [[c, s], [-s e^{-i phi}, c e^{-i phi}]]
+    if (onj) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const T xp = x[a][0], emxq = phase_(emj, x[a][1]);
+        x[a][0] = rot_p(cj, sj, xp, emxq);
+        x[a][1] = rot_q(cj, sj, xp, emxq);
+      }
+    }
+    if (FORQ) {
+      if (blk_on && onj) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          if (rows[a] >= w) continue;
+          sQ[rows[a]][cols[0]] = x[a][0];
+          sQ[rows[a]][cols[1]] = x[a][1];
+        }
+      }
+    } else {
+      // rows:  [g_p; g_q] <- J^H [g_p; g_q]; the pair's own off-diagonal entries become 0
+      if (oni) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const T gp = x[0][b], epgq = cphase_(emi, x[1][b]);
+          T np = rot_p(ci, si, gp, epgq);
+          T nq = rot_q(ci, si, gp, epgq);
+          if (cols[b] == rows[1]) np = zero_<T>();
+          if (cols[b] == rows[0]) nq = zero_<T>();
+          x[0][b] = np;
+          x[1][b] = nq;
+        }
+      }
+      if (blk_on) {
+        T(*Gn)[kS] = sG[cur ^ 1];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) Gn[rows[a]][cols[b]] = x[a][b];
+      }
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+}
+
 template <bool C>
-__global__ void __launch_bounds__(kThreads) k_svd_solve(const SvdMat *mats, const SvdItem *items, int32_t round,
-                                                         const void *part_, const int32_t *perm,
-                                                         const int32_t *active, void *q_, int32_t *qflag,
-                                                         int32_t *rotated) {
+__global__ void __launch_bounds__(kSolveThreads) k_svd_solve(const SvdMat *mats, const SvdItem *items, int32_t round,
+                                                              const void *part_, const int32_t *perm,
+                                                              const int32_t *active, void *q_, int32_t *qflag,
+                                                              int32_t *rotated) {
   using T = typename ElemOf<C>::T;
-  __shared__ T sG[2][kW][kW + 1];   // G of the current round, and the next
-  __shared__ T sQ[kW][kW + 1];
+  __shared__ __align__(16) T sG[2][kW][kS];   // G of the current round, and the next
+  __shared__ __align__(16) T sQ[kW][kS];
   __shared__ int32_t sCol[kW];
-  __shared__ double sRed[kWaves];
+  __shared__ double sRed[kSolveThreads / 64];
+  static_assert(kW == 32 && kSolveThreads == 512, "one thread per 2 x 2 block of pairs, for G and for Q");
+  constexpr int kPer = kW * kW / kSolveThreads;
 
   const SvdItem it = items[blockIdx.x];
-  if (!active[it.mat]) return;
   const SvdMat mt = mats[it.mat];
+  if (!active[it.mat]) return;
   const int tid = threadIdx.x;
   int w = 0;
   if (!pair_cols(mt, round, it.k, perm, sCol, w)) return;
   int32_t *flag = qflag + mt.pair0 + it.k;
   const T *part = static_cast<const T *>(part_) + (mt.gram0 + int64_t(it.k) * mt.ng) * (kW * kW);
-  for (int e = tid; e < w * w; e += kThreads) {
-    const int p = e / w, q = e - p * w;
-    T s = zero_<T>();
-    for (int g = 0; g < mt.ng; ++g) s = add_(s, part[int64_t(g) * (kW * kW) + p * kW + q]);
-    sG[0][p][q] = s;
+  T sum[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) sum[u] = zero_<T>();
+  for (int g = 0; g < mt.ng; ++g)   // entries past w x w: whatever the slot holds, not used
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) sum[u] = add_(sum[u], part[int64_t(g) * (kW * kW) + tid + u * kSolveThreads]);
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int e = tid + u * kSolveThreads, p = e / kW, q = e % kW;
+    sG[0][p][q] = sum[u];
+    sQ[p][q] = (p == q) ? one_<T>() : zero_<T>();
   }
   __syncthreads();
 
   // ---- convergence test of the pair ----
   double off = 0.0;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int e = tid + u * kThreads;
-    if (e < w * w) {
-      const int p = e / w, q = e - p * w;
-      if (p < q) {
-        const double dp = re_(sG[0][p][p]), dq = re_(sG[0][q][q]);
-        if (dp > 0.0 && dq > 0.0) off = fmax(off, abs2_(sG[0][p][q]) / (dp * dq));
-      }
+  for (int u = 0; u < kPer; ++u) {
+    const int e = tid + u * kSolveThreads, p = e / kW, q = e % kW;
+    if (p < q && q < w) {
+      const double dp = re_(sG[0][p][p]), dq = re_(sG[0][q][q]);
+      if (dp > 0.0 && dq > 0.0) off = fmax(off, abs2_(sG[0][p][q]) / (dp * dq));
     }
   }
   off = wave_max(off);
   if ((tid & 63) == 0) sRed[tid >> 6] = off;
   __syncthreads();
   const double tol = fmax(16.0, static_cast<double>(mt.M)) * 2.220446049250313e-16;
-  const double offmax = fmax(fmax(sRed[0], sRed[1]), fmax(sRed[2], sRed[3]));
+  double offmax = sRed[0];
+#pragma unroll
+  for (int v = 1; v < kSolveThreads / 64; ++v) offmax = fmax(offmax, sRed[v]);
   if (offmax < tol * tol) {
     if (tid == 0) *flag = 0;
     return;
@@ -312,200 +467,90 @@ __global__ void __launch_bounds__(kThreads) k_svd_solve(const SvdMat *mats, cons
     *flag = 1;
   }
 
-  // ---- Jacobi diagonalisation of G in LDS ----
-  // A round applies the rotations of P2 / 2 disjoint index pairs,
-  // G <- J^H G J and Q <- Q J, as 2 x 2 blocks: thread (bi, bj) takes the
-  // block of G at rows (p, q) of pair bi and columns of pair bj, applies the
-  // rotation of pair bj to its columns and then that of pair bi to its rows
-  // (the same operations, in the same order, as a column pass followed by a
-  // row pass), and writes the result into the other G buffer; it also
-  // rotates rows 2 bi, 2 bi + 1 of Q in the columns of pair bj, in place.
-  // Every wave computes the round's rotations from the round's G, pair k in
-  // lane k (and its copies k + 16, ...), and each lane takes those of pairs
-  // bi and bj by shuffle, so a round takes one barrier.
-  for (int e = tid; e < w * w; e += kThreads) {
-    const int p = e / w, q = e - p * w;
-    sQ[p][q] = (p == q) ? one_<T>() : zero_<T>();
-  }
-  const int P2 = w + (w & 1);
-  const double eps = 2.220446049250313e-16;
-  static_assert(kW == 32 && kThreads == 256, "one thread per 2 x 2 block of pairs");
-  const int bi = tid / (kW / 2), bj = tid % (kW / 2);
-  const bool blk_on = bi < P2 / 2 && bj < P2 / 2;
-  // rotation of pair k of round r from the round's G: indexes, c, s and the
-  // unit phase; false (identity) when the pair is orthogonal or padded
-  auto rotation = [&](const T (*G)[kW + 1], int r, int k, int &p, int &q, double &c, double &sn, T &em) {
-    circle_pair(P2, r, k, p, q);
-    c = 1.0;
-    sn = 0.0;
-    em = one_<T>();
-    if (p >= w || q >= w) return false;
-    const double al = re_(G[p][p]), be = re_(G[q][q]);
-    const T g = G[p][q];
-    // |g| > eps sqrt(al be), squared: three square roots and three divisions
-    // per rotation, the round's latency chain
-    const double ag2 = abs2_(g);
-    if (!(ag2 > 0.0 && al > 0.0 && be > 0.0 && ag2 > (eps * eps) * (al * be))) return false;
-    const double ag = sqrt(ag2);
-    const double inv = 1.0 / ag;
-    const double zeta = (be - al) * (0.5 * inv);
-    double t;
-    if (fabs(zeta) > 1e150) t = 0.5 / zeta;
-    else t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-    c = 1.0 / sqrt(1.0 + t * t);
-    sn = c * t;
-    em = uphase_conj_inv(g, inv);
-    return true;
-  };
-  __syncthreads();
-  int cur = 0;
-  for (int sweep = 0; sweep < kInnerSweeps; ++sweep) {
-    int any = 0;
-    for (int r = 0; r < P2 - 1; ++r) {
-      const T(*G)[kW + 1] = sG[cur];
-      const int kr = (tid & 63) % (kW / 2);
-      int rp = 0, rq = 0;
-      double rc = 1.0, rs = 0.0;
-      T rem = one_<T>();
-      const bool ron = kr < P2 / 2 && rotation(G, r, kr, rp, rq, rc, rs, rem);
-      any |= ron ? 1 : 0;
-      const int pi = __shfl(rp, bi), qi = __shfl(rq, bi), pj = __shfl(rp, bj), qj = __shfl(rq, bj);
-      const bool oni = __shfl(ron ? 1 : 0, bi) != 0, onj = __shfl(ron ? 1 : 0, bj) != 0;
-      const double ci = __shfl(rc, bi), si = __shfl(rs, bi), cj = __shfl(rc, bj), sj = __shfl(rs, bj);
-      const T emi = shfl_(rem, bi), emj = shfl_(rem, bj);
-      if (blk_on) {
-        T(*Gn)[kW + 1] = sG[cur ^ 1];
-        const int rows[2] = {pi, qi}, cols[2] = {pj, qj};
-        T x[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) x[a][b] = (rows[a] < w && cols[b] < w) ? G[rows[a]][cols[b]] : zero_<T>();
-        // columns:  [x_p, x_q] <- [x_p, x_q] J,  J = [[c, s], [-s e^{-i phi}, c e^{-i phi}]]
-        if (onj) {
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-            const T xp = x[a][0], emxq = mul_(emj, x[a][1]);
-            x[a][0] = sub_(scl_(cj, xp), scl_(sj, emxq));
-            x[a][1] = add_(scl_(sj, xp), scl_(cj, emxq));
-          }
-        }
-        // rows:  [g_p; g_q] <- J^H [g_p; g_q]; the pair's own off-diagonal entries become 0
-        if (oni) {
-          const T ep = conj_(emi);
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const T gp = x[0][b], epgq = mul_(ep, x[1][b]);
-            T np = sub_(scl_(ci, gp), scl_(si, epgq));
-            T nq = add_(scl_(si, gp), scl_(ci, epgq));
-            if (cols[b] == qi) np = zero_<T>();
-            if (cols[b] == pi) nq = zero_<T>();
-            x[0][b] = np;
-            x[1][b] = nq;
-          }
-        }
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            if (rows[a] < w && cols[b] < w) Gn[rows[a]][cols[b]] = x[a][b];
-        // Q: rows 2 bi, 2 bi + 1, columns of pair bj
-        if (onj) {
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-            const int i = 2 * bi + a;
-            if (i >= w) continue;
-            const T xp = sQ[i][pj], emxq = mul_(emj, sQ[i][qj]);
-            sQ[i][pj] = sub_(scl_(cj, xp), scl_(sj, emxq));
-            sQ[i][qj] = add_(scl_(sj, xp), scl_(cj, emxq));
-          }
-        }
-      }
-      __syncthreads();
-      cur ^= 1;
-    }
-    if (!__syncthreads_or(any)) break;
-  }
+  if (__builtin_amdgcn_readfirstlane(tid) < kSolveThreads / 2) jacobi_sweep<C, false>(sG, sQ, w);
+  else jacobi_sweep<C, true>(sG, sQ, w);
   T *Q = static_cast<T *>(q_) + int64_t(mt.pair0 + it.k) * (kW * kW);
-  for (int e = tid; e < w * w; e += kThreads) {
-    const int p = e / w, q = e - p * w;
-    Q[p * kW + q] = sQ[p][q];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int e = tid + u * kSolveThreads, p = e / kW, q = e % kW;
+    if (p < w && q < w) Q[e] = sQ[p][q];
   }
 }
 
-// Round phase 3: P <- P Q on one kRG-row group of the pair's columns of X
-// (kind 0) or of V (kind 1).
-// P <- P Q (and V <- V Q) for one row group of the pair, on
-// v_mfma_f64_16x16x4f64: wave wv computes rows 16 wv .. 16 wv + 15 of the
-// kRG-row group, in two 16-column tiles, over k-steps of 4 of the pair's w
-// columns.  Complex: Re = Pr Qr - Pi Qi, Im = Pr Qi + Pi Qr.
+// Round phase 3: P <- P Q for one group of kUR rows of the pair's columns of X
+// (kind 0) or of V (kind 1), on v_mfma_f64_16x16x4f64 over k-steps of 4 of the
+// pair's w columns: wave wv computes rows 16 (wv % 2) .. + 15 of columns
+// 16 (wv / 2) .. + 15.  Complex: Re = Pr Qr - Pi Qi, Im = Pr Qi + Pi Qr.  The
+// product is formed as Q^T P^T, whose accumulators hold consecutive rows in
+// consecutive lanes, so that a store covers 256 bytes of each of 4 columns;
+// as P Q, 64 bytes of each of 16, the stores took 6 of 16 us.  In a U(1)xU(1) D =
+// 2048 complex128 SVD with guarded loads 17.7 us, unguarded 14.9, now 12.9; 4.5
+// of it is a launch that finds nothing to do.
 template <bool C>
 __global__ void __launch_bounds__(kThreads) k_svd_update(const SvdMat *mats, const SvdRowItem *items, int32_t round,
                                                           void *ws_, const int32_t *perm, const int32_t *active,
                                                           const void *q_, const int32_t *qflag) {
   using T = typename ElemOf<C>::T;
   constexpr int PARTS = C ? 2 : 1;
-  __shared__ double sP[PARTS][kW][kRG + 1];
+  __shared__ double sP[PARTS][kW][kUR + 1];
   __shared__ double sQ[PARTS][kW][kW];
   __shared__ int32_t sCol[kW];
   const SvdRowItem it = items[blockIdx.x];
-  if (!active[it.mat]) return;
   const SvdMat mt = mats[it.mat];
+  if (!active[it.mat]) return;
   int w = 0;
   if (!pair_cols(mt, round, it.k, perm, sCol, w)) return;
   if (!qflag[mt.pair0 + it.k]) return;
   const int tid = threadIdx.x;
   const T *Q = static_cast<const T *>(q_) + int64_t(mt.pair0 + it.k) * (kW * kW);
-  for (int e = tid; e < kW * kW; e += kThreads) {
-    const int p = e / kW, q = e - p * kW;
-    const T v = (p < w && q < w) ? Q[p * kW + q] : zero_<T>();
-    if constexpr (C) {
-      sQ[0][p][q] = v.x;
-      sQ[1][p][q] = v.y;
-    } else {
-      sQ[0][p][q] = v;
-    }
-  }
+  T qv[kW * kW / kThreads];   // past w x w: whatever the slot holds, staged as zero
+#pragma unroll
+  for (int u = 0; u < kW * kW / kThreads; ++u) qv[u] = Q[tid + u * kThreads];
   T *base = static_cast<T *>(ws_) + (it.kind ? mt.v_off : mt.x_off);
   const int64_t rows = it.kind ? mt.N : mt.M;
-  const int64_t rb = int64_t(it.g) * kRG, re = min<int64_t>(rows, rb + kRG);
+  const int64_t rb = int64_t(it.g) * kUR, re = min<int64_t>(rows, rb + kUR);
   __syncthreads();
-  stage_panel<C>(base, rows, rb, re, w, sCol, sP);
+  stage_panel<C, kUR>(base, rows, rb, re, w, sCol, sP);
+#pragma unroll
+  for (int u = 0; u < kW * kW / kThreads; ++u) {
+    const int e = tid + u * kThreads, p = e / kW, q = e % kW;
+    const bool in = p < w && q < w;
+    if constexpr (C) {
+      sQ[0][p][q] = in ? qv[u].x : 0.0;
+      sQ[1][p][q] = in ? qv[u].y : 0.0;
+    } else {
+      sQ[0][p][q] = in ? qv[u] : 0.0;
+    }
+  }
   __syncthreads();
   const int lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
   typedef double v4d __attribute__((ext_vector_type(4)));
-  v4d acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-  v4d acc_i[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-  if (rb + 16 * wv < re) {
-    for (int ks = 0; ks < w; ks += 4) {
-      const double ar = sP[0][ks + lk][16 * wv + lr];
-      const double ai = C ? sP[PARTS - 1][ks + lk][16 * wv + lr] : 0.0;
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const double br = sQ[0][ks + lk][16 * nt + lr];
-        acc[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, acc[nt], 0, 0, 0);
-        if constexpr (C) {
-          const double bi = sQ[1][ks + lk][16 * nt + lr];
-          acc[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, acc[nt], 0, 0, 0);
-          acc_i[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, acc_i[nt], 0, 0, 0);
-          acc_i[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, acc_i[nt], 0, 0, 0);
-        }
-      }
+  static_assert(kUR == 32 && kW == 32 && kWaves == 4, "one 16 x 16 tile per wave");
+  const int r0 = 16 * (wv & 1), j0 = 16 * (wv >> 1);
+  v4d acc = {0.0, 0.0, 0.0, 0.0}, acc_i = {0.0, 0.0, 0.0, 0.0};
+  if (rb + r0 >= re || j0 >= w) return;
+#pragma unroll 2
+  for (int ks = 0; ks < w; ks += 4) {
+    const double ar = sP[0][ks + lk][r0 + lr], br = sQ[0][ks + lk][j0 + lr];
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar, acc, 0, 0, 0);
+    if constexpr (C) {
+      const double ai = sP[1][ks + lk][r0 + lr], bi = sQ[1][ks + lk][j0 + lr];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, -ai, acc, 0, 0, 0);
+      acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(bi, ar, acc_i, 0, 0, 0);
+      acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ai, acc_i, 0, 0, 0);
     }
   }
   // every read of the rows is done (they sit in LDS): write the new columns
+  const int64_t row = rb + r0 + lr;
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int64_t row = rb + 16 * wv + 4 * v + lk;
-      const int j = 16 * nt + lr;
-      if (row < re && j < w) {
-        T *dst = base + int64_t(sCol[j]) * rows + row;
-        if constexpr (C) *dst = cplx{acc[nt][v], acc_i[nt][v]};
-        else *dst = acc[nt][v];
-      }
+  for (int v = 0; v < 4; ++v) {
+    const int j = j0 + 4 * v + lk;
+    if (row < re && j < w) {
+      T *dst = base + int64_t(sCol[j]) * rows + row;
+      if constexpr (C) *dst = cplx{acc[v], acc_i[v]};
+      else *dst = acc[v];
     }
+  }
 }
 
 // Singular values and vectors, grid (element groups, matrices): the columns
@@ -593,14 +638,12 @@ qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, co
     max_elems = std::max(max_elems, mt.M * mt.N);
     if (mt.N >= 2) {
       max_players = std::max(max_players, mt.P);
-      const int32_t ngv = static_cast<int32_t>((mt.N + kRG - 1) / kRG);
+      const int32_t nux = static_cast<int32_t>((mt.M + kUR - 1) / kUR), nuv = static_cast<int32_t>((mt.N + kUR - 1) / kUR);
       for (int32_t k = 0; k < mt.P / 2; ++k) {
         items.push_back(SvdItem{static_cast<int32_t>(i), k});
-        for (int32_t g = 0; g < mt.ng; ++g) {
-          gitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 0});
-          uitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 0});
-        }
-        for (int32_t g = 0; g < ngv; ++g) uitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 1});
+        for (int32_t g = 0; g < mt.ng; ++g) gitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 0});
+        for (int32_t g = 0; g < nux; ++g) uitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 0});
+        for (int32_t g = 0; g < nuv; ++g) uitems.push_back(SvdRowItem{static_cast<int32_t>(i), k, g, 1});
       }
       pair_slots += mt.P / 2;
       gram_slots += int64_t(mt.P / 2) * mt.ng;
@@ -657,7 +700,7 @@ qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, co
     for (int32_t r = 0; r < max_players - 1; ++r) {
       hipLaunchKernelGGL(k_svd_gram<C>, dim3(static_cast<unsigned>(gitems.size())), dim3(kThreads), 0, st, dm, gi,
                          r, d_ws.p, perm, active, d_part.p);
-      hipLaunchKernelGGL(k_svd_solve<C>, dim3(static_cast<unsigned>(items.size())), dim3(kThreads), 0, st, dm,
+      hipLaunchKernelGGL(k_svd_solve<C>, dim3(static_cast<unsigned>(items.size())), dim3(kSolveThreads), 0, st, dm,
                          static_cast<const SvdItem *>(d_items.p), r, d_part.p, perm, active, d_q.p, qflag, rotated);
       hipLaunchKernelGGL(k_svd_update<C>, dim3(static_cast<unsigned>(uitems.size())), dim3(kThreads), 0, st, dm, ui,
                          r, d_ws.p, perm, active, d_q.p, qflag);
