@@ -176,24 +176,33 @@ __global__ __launch_bounds__(256) void k_emit(const uint64_t *ha, int64_t na, co
 // plus tasks of equal key before t.  Grid (256 tasks, chunk of kRankChunk keys
 // to compare them with).  Quadratic, but spread over the chip: up to
 // kRankMaxTasks it is faster than the single-workgroup radix sort (43 us at
-// 4860 tasks, 170 us at 45 000).
-constexpr int kRankChunk = 1024;
+// 4860 tasks, 170 us at 45 000).  What bounds it is the LDS latency of the keys
+// (one address for the whole wave), so the comparisons run in groups whose
+// keys are read together, with no test of the position but in the chunk on the
+// diagonal: 52 -> 7.6 us at 4600 tasks, 54 -> 11.9 at 11 500 (chunks of 1024
+// and a loop over each side of the position before).
+constexpr int kRankChunk = 256;
 constexpr int64_t kRankMaxTasks = 32768;
 __global__ __launch_bounds__(256) void k_rank(const uint64_t *key, int64_t n, int32_t *rank) {
-  __shared__ uint64_t sk[kRankChunk];
-  const int64_t base = int64_t(blockIdx.y) * kRankChunk;
-  const int len = static_cast<int>(n - base < kRankChunk ? n - base : kRankChunk);
-  for (int j = threadIdx.x; j < len; j += 256) sk[j] = key[base + j];
+  __shared__ __align__(16) uint64_t sk[kRankChunk];
+  static_assert(kRankChunk == 256, "a chunk per workgroup of tasks: one key per thread");
+  const int tid = threadIdx.x;
+  const int64_t base = int64_t(blockIdx.y) * kRankChunk, t = int64_t(blockIdx.x) * 256 + tid;
+  sk[tid] = base + tid < n ? key[base + tid] : ~uint64_t(0);   // past the end: never smaller
+  const uint64_t mine = t < n ? key[t] : 0;
   __syncthreads();
-  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= n) return;
-  const uint64_t mine = key[t];
-  // keys before position t count when equal, too
-  const int before = t <= base ? 0 : (t - base < len ? static_cast<int>(t - base) : len);
   int32_t r = 0;
-  for (int j = 0; j < before; ++j) r += sk[j] <= mine ? 1 : 0;
-  for (int j = before; j < len; ++j) r += sk[j] < mine ? 1 : 0;
-  if (r != 0) atomicAdd(&rank[t], r);
+  if (blockIdx.y < blockIdx.x) {   // keys before position t count when equal, too
+#pragma unroll 16
+    for (int j = 0; j < kRankChunk; ++j) r += sk[j] <= mine ? 1 : 0;
+  } else if (blockIdx.y > blockIdx.x) {
+#pragma unroll 16
+    for (int j = 0; j < kRankChunk; ++j) r += sk[j] < mine ? 1 : 0;
+  } else {
+#pragma unroll 16
+    for (int j = 0; j < kRankChunk; ++j) r += sk[j] < mine + (j < tid ? 1 : 0) ? 1 : 0;
+  }
+  if (t < n && r != 0) atomicAdd(&rank[t], r);
 }
 __global__ void k_place(const uint64_t *key, const int32_t *rank, int64_t n, uint64_t *sk, int32_t *sv) {
   const int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
