@@ -38,6 +38,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
+constexpr int kSolveThreads = 512;   // of the Gram and solve workgroups
 constexpr int kB = 16;          // columns per Jacobi block
 constexpr int kW = 2 * kB;      // panel width
 constexpr int kRG = 64;         // rows per Gram workgroup
@@ -204,10 +205,10 @@ __device__ __forceinline__ bool pair_cols(const SvdMat &mt, int32_t round, int32
 // rows and columns.  The loads carry no guards (past the panel they read its
 // last row or column): guarded, each was waited for before the next (a Gram
 // launch of the D = 2048 complex128 SVD 10.8 -> 9.7 us).
-template <bool C, int R, typename T>
+template <bool C, int R, int NT, typename T>
 __device__ __forceinline__ void stage_panel(const T *base, int64_t rows, int64_t rb, int64_t re, int w,
                                             const int32_t *sCol, double (*sP)[kW][R + 1]) {
-  constexpr int kCols = kThreads / R;   // columns per pass: consecutive threads take consecutive rows
+  constexpr int kCols = NT / R;   // columns per pass: consecutive threads take consecutive rows
   const int rr = threadIdx.x % R, c0 = threadIdx.x / R;
   const int64_t row = min<int64_t>(rb + rr, re - 1);
   T v[kW / kCols];
@@ -230,51 +231,63 @@ __device__ __forceinline__ void stage_panel(const T *base, int64_t rows, int64_t
 // g kRG .. (g + 1) kRG - 1, on v_mfma_f64_16x16x4f64: wave wv computes the
 // 16 x 16 tile (wv / 2, wv % 2) of the 32 x 32 result over 16 k-steps of 4
 // rows.  Complex: Re G = Pr^T Pr + Pi^T Pi, Im G = Pr^T Pi - Pi^T Pr.
+template <bool C, int NT>
+__device__ __forceinline__ void gram_tile(const SvdMat &mt, int32_t g, const void *ws_, int w, const int32_t *sCol,
+                                          double (*sP)[kW][kRG + 1], v4d &acc, v4d &acc_i) {
+  using T = typename ElemOf<C>::T;
+  const int tid = threadIdx.x;
+  const T *X = static_cast<const T *>(ws_) + mt.x_off;
+  const int64_t rb = int64_t(g) * kRG, re = min<int64_t>(mt.M, rb + kRG);
+  stage_panel<C, kRG, NT>(X, mt.M, rb, re, w, sCol, sP);
+  __syncthreads();
+  const int lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  const int p0 = 16 * (wv >> 1), q0 = 16 * (wv & 1);
+  acc = acc_i = v4d{0.0, 0.0, 0.0, 0.0};
+  if (p0 >= w || q0 >= w) return;   // waves past the four tiles have p0 >= kW
+#pragma unroll 4
+  for (int ks = 0; ks < kRG; ks += 4) {
+    const double ar = sP[0][p0 + lr][ks + lk], br = sP[0][q0 + lr][ks + lk];
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, acc, 0, 0, 0);
+    if constexpr (C) {
+      const double ai = sP[1][p0 + lr][ks + lk], bi = sP[1][q0 + lr][ks + lk];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, acc, 0, 0, 0);
+      acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, acc_i, 0, 0, 0);
+      acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, br, acc_i, 0, 0, 0);
+    }
+  }
+}
+
+// The thread's 4 entries of its wave's tile, put(p, q, value).
+template <bool C, typename F>
+__device__ __forceinline__ void each_gram_entry(int w, const v4d &acc, const v4d &acc_i, F put) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int p = 16 * (wv >> 1) + 4 * v + lk, q = 16 * (wv & 1) + lr;
+    if (p < w && q < w) {
+      if constexpr (C) put(p, q, cplx{acc[v], acc_i[v]});
+      else put(p, q, acc[v]);
+    }
+  }
+}
+
 template <bool C>
 __global__ void __launch_bounds__(kThreads) k_svd_gram(const SvdMat *mats, const SvdRowItem *items, int32_t round,
                                                         const void *ws_, const int32_t *perm, const int32_t *active,
                                                         void *part_) {
   using T = typename ElemOf<C>::T;
-  constexpr int PARTS = C ? 2 : 1;
-  __shared__ double sP[PARTS][kW][kRG + 1];
+  __shared__ double sP[C ? 2 : 1][kW][kRG + 1];
   __shared__ int32_t sCol[kW];
   const SvdRowItem it = items[blockIdx.x];
   const SvdMat mt = mats[it.mat];
   if (!active[it.mat]) return;
   int w = 0;
   if (!pair_cols(mt, round, it.k, perm, sCol, w)) return;
-  const int tid = threadIdx.x;
-  const T *X = static_cast<const T *>(ws_) + mt.x_off;
   __syncthreads();
-  const int64_t rb = int64_t(it.g) * kRG, re = min<int64_t>(mt.M, rb + kRG);
-  stage_panel<C, kRG>(X, mt.M, rb, re, w, sCol, sP);
-  __syncthreads();
-  const int lane = tid & 63, wv = tid >> 6, lr = lane & 15, lk = lane >> 4;
-  const int p0 = 16 * (wv >> 1), q0 = 16 * (wv & 1);
-  typedef double v4d __attribute__((ext_vector_type(4)));
-  v4d acc = {0.0, 0.0, 0.0, 0.0}, acc_i = {0.0, 0.0, 0.0, 0.0};
-  if (p0 < w && q0 < w) {
-#pragma unroll 4
-    for (int ks = 0; ks < kRG; ks += 4) {
-      const double ar = sP[0][p0 + lr][ks + lk], br = sP[0][q0 + lr][ks + lk];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, acc, 0, 0, 0);
-      if constexpr (C) {
-        const double ai = sP[1][p0 + lr][ks + lk], bi = sP[1][q0 + lr][ks + lk];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, acc, 0, 0, 0);
-        acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, acc_i, 0, 0, 0);
-        acc_i = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, br, acc_i, 0, 0, 0);
-      }
-    }
-  }
+  v4d acc, acc_i;
+  gram_tile<C, kThreads>(mt, it.g, ws_, w, sCol, sP, acc, acc_i);
   T *part = static_cast<T *>(part_) + (mt.gram0 + int64_t(it.k) * mt.ng + it.g) * (kW * kW);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int p = p0 + 4 * v + lk, q = q0 + lr;
-    if (p < w && q < w) {
-      if constexpr (C) part[p * kW + q] = cplx{acc[v], acc_i[v]};
-      else part[p * kW + q] = acc[v];
-    }
-  }
+  each_gram_entry<C>(w, acc, acc_i, [&](int p, int q, T v) { part[p * kW + q] = v; });
 }
 
 // Round phase 2, one workgroup per pair: the Gram matrix as the sum of the
@@ -289,11 +302,17 @@ __global__ void __launch_bounds__(kThreads) k_svd_gram(const SvdMat *mats, const
 // not on that chain is kept off it: Q has waves of its own, which share the
 // SIMDs with the chain's; a thread's column rotation is the one its lane has
 // computed, only the row rotation comes by shuffle; the entries of G a thread
-// works on are read before the rotation is known.  A visit in a U(1)xU(1) D = 2048
+// works on are read before the rotation is known.
+// GRAM: the workgroup forms the pair's Gram itself, phase 1 and 2 in one
+// launch, for calls whose matrices have one row group each (a 33 x 32 matrix,
+// complex128: 853 -> 653 us, FP64 706 -> 595); with more groups the last
+// workgroup of a pair to write its part would have to go on, and the
+// device-wide fences of all of them took 72 us a round in the D = 2048 SVD where
+// the two launches take 39.
+// A visit in a U(1)xU(1) D = 2048
 // complex128 SVD: 47.6 us with G and Q in the same waves and all rotations by
 // shuffle, 37.2 with waves for Q, 29.6 with the rows of kS entries; of a round's
 // 1.0 us a rotation's square roots and divisions are 0.4.
-constexpr int kSolveThreads = 512;
 // Row stride of G and Q in LDS: even, so that the entries (p, q) and (p, p) of
 // the 16 pairs of a round, which lie along an antidiagonal and the diagonal,
 // fall into different banks.
@@ -406,16 +425,21 @@ __device__ __forceinline__ void jacobi_sweep(T (*sG)[kW][kS], T (*sQ)[kS], int w
   }
 }
 
-template <bool C>
+template <bool C, bool GRAM>
 __global__ void __launch_bounds__(kSolveThreads) k_svd_solve(const SvdMat *mats, const SvdItem *items, int32_t round,
-                                                              const void *part_, const int32_t *perm,
+                                                              const void *ws_, const void *part_, const int32_t *perm,
                                                               const int32_t *active, void *q_, int32_t *qflag,
                                                               int32_t *rotated) {
   using T = typename ElemOf<C>::T;
-  __shared__ __align__(16) T sG[2][kW][kS];   // G of the current round, and the next
-  __shared__ __align__(16) T sQ[kW][kS];
+  constexpr int PARTS = C ? 2 : 1;
+  // G (of the current round, and the next) and Q; before them the panel
+  constexpr size_t kG = 2 * kW * kS * sizeof(T), kQ = kW * kS * sizeof(T);
+  static_assert(PARTS * kW * (kRG + 1) * sizeof(double) <= kG + kQ, "the panel fits in the place of G and Q");
+  __shared__ __align__(16) char smem[kG + kQ];
   __shared__ int32_t sCol[kW];
   __shared__ double sRed[kSolveThreads / 64];
+  auto *sG = reinterpret_cast<T(*)[kW][kS]>(smem);
+  auto *sQ = reinterpret_cast<T(*)[kS]>(smem + kG);
   static_assert(kW == 32 && kSolveThreads == 512, "one thread per 2 x 2 block of pairs, for G and for Q");
   constexpr int kPer = kW * kW / kSolveThreads;
 
@@ -426,17 +450,29 @@ __global__ void __launch_bounds__(kSolveThreads) k_svd_solve(const SvdMat *mats,
   int w = 0;
   if (!pair_cols(mt, round, it.k, perm, sCol, w)) return;
   int32_t *flag = qflag + mt.pair0 + it.k;
-  const T *part = static_cast<const T *>(part_) + (mt.gram0 + int64_t(it.k) * mt.ng) * (kW * kW);
-  T sum[kPer];
+  if constexpr (GRAM) {
+    __syncthreads();
+    v4d acc, acc_i;
+    gram_tile<C, kSolveThreads>(mt, 0, ws_, w, sCol, reinterpret_cast<double(*)[kW][kRG + 1]>(smem), acc, acc_i);
+    __syncthreads();   // the panel is read: G and Q take its place
+    each_gram_entry<C>(w, acc, acc_i, [&](int p, int q, T v) { sG[0][p][q] = add_(zero_<T>(), v); });
+  } else {
+    const T *part = static_cast<const T *>(part_) + (mt.gram0 + int64_t(it.k) * mt.ng) * (kW * kW);
+    T sum[kPer];
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) sum[u] = zero_<T>();
-  for (int g = 0; g < mt.ng; ++g)   // entries past w x w: whatever the slot holds, not used
+    for (int u = 0; u < kPer; ++u) sum[u] = zero_<T>();
+    for (int g = 0; g < mt.ng; ++g)   // entries past w x w: whatever the slot holds, not used
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) sum[u] = add_(sum[u], part[int64_t(g) * (kW * kW) + tid + u * kSolveThreads]);
+      for (int u = 0; u < kPer; ++u) sum[u] = add_(sum[u], part[int64_t(g) * (kW * kW) + tid + u * kSolveThreads]);
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int e = tid + u * kSolveThreads;
+      sG[0][e / kW][e % kW] = sum[u];
+    }
+  }
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
     const int e = tid + u * kSolveThreads, p = e / kW, q = e % kW;
-    sG[0][p][q] = sum[u];
     sQ[p][q] = (p == q) ? one_<T>() : zero_<T>();
   }
   __syncthreads();
@@ -510,7 +546,7 @@ __global__ void __launch_bounds__(kThreads) k_svd_update(const SvdMat *mats, con
   const int64_t rows = it.kind ? mt.N : mt.M;
   const int64_t rb = int64_t(it.g) * kUR, re = min<int64_t>(rows, rb + kUR);
   __syncthreads();
-  stage_panel<C, kUR>(base, rows, rb, re, w, sCol, sP);
+  stage_panel<C, kUR, kThreads>(base, rows, rb, re, w, sCol, sP);
 #pragma unroll
   for (int u = 0; u < kW * kW / kThreads; ++u) {
     const int e = tid + u * kThreads, p = e / kW, q = e % kW;
@@ -529,7 +565,6 @@ __global__ void __launch_bounds__(kThreads) k_svd_update(const SvdMat *mats, con
   const int r0 = 16 * (wv & 1), j0 = 16 * (wv >> 1);
   v4d acc = {0.0, 0.0, 0.0, 0.0}, acc_i = {0.0, 0.0, 0.0, 0.0};
   if (rb + r0 >= re || j0 >= w) return;
-#pragma unroll 2
   for (int ks = 0; ks < w; ks += 4) {
     const double ar = sP[0][ks + lk][r0 + lr], br = sQ[0][ks + lk][j0 + lr];
     acc = __builtin_amdgcn_mfma_f64_16x16x4f64(br, ar, acc, 0, 0, 0);
@@ -689,7 +724,8 @@ qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, co
   std::vector<int32_t> h_active(mats.size()), h_rot(mats.size(), 0);
   for (size_t i = 0; i < mats.size(); ++i) h_active[i] = mats[i].N >= 2;
   int32_t sweeps = 0;
-  bool any = !items.empty();
+  bool any = !items.empty(), one_group = true;   // one row group per matrix of more than one column
+  for (const SvdMat &mt : mats) one_group = one_group && (mt.N < 2 || mt.ng == 1);
   while (any && sweeps < kMaxSweeps) {
     QLT_HIP(hipMemcpyAsync(active, h_active.data(), sizeof(int32_t) * mats.size(), hipMemcpyHostToDevice, st));
     std::fill(h_rot.begin(), h_rot.end(), 0);
@@ -698,10 +734,13 @@ qlt_status svd_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, co
     hipLaunchKernelGGL(k_svd_sort, dim3(static_cast<unsigned>(n_mats)), dim3(kThreads), 0, st, dm, norms, perm,
                        active, 0);
     for (int32_t r = 0; r < max_players - 1; ++r) {
-      hipLaunchKernelGGL(k_svd_gram<C>, dim3(static_cast<unsigned>(gitems.size())), dim3(kThreads), 0, st, dm, gi,
-                         r, d_ws.p, perm, active, d_part.p);
-      hipLaunchKernelGGL(k_svd_solve<C>, dim3(static_cast<unsigned>(items.size())), dim3(kSolveThreads), 0, st, dm,
-                         static_cast<const SvdItem *>(d_items.p), r, d_part.p, perm, active, d_q.p, qflag, rotated);
+      if (!one_group)
+        hipLaunchKernelGGL(k_svd_gram<C>, dim3(static_cast<unsigned>(gitems.size())), dim3(kThreads), 0, st, dm, gi, r,
+                           d_ws.p, perm, active, d_part.p);
+      hipLaunchKernelGGL((one_group ? k_svd_solve<C, true> : k_svd_solve<C, false>),
+                         dim3(static_cast<unsigned>(items.size())), dim3(kSolveThreads), 0, st, dm,
+                         static_cast<const SvdItem *>(d_items.p), r, d_ws.p, d_part.p, perm, active, d_q.p, qflag,
+                         rotated);
       hipLaunchKernelGGL(k_svd_update<C>, dim3(static_cast<unsigned>(uitems.size())), dim3(kThreads), 0, st, dm, ui,
                          r, d_ws.p, perm, active, d_q.p, qflag);
     }
