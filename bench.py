@@ -565,9 +565,9 @@ def main() -> int:
     roofline = kernel_roofline(r["kernel"], mv.name)
 
     def contraction_roofline(res):
-        """The heaviest contraction as a whole: its tile-class kernels run
-        concurrently on the class streams, so the unit that reaches the MFMA
-        bound together is the contraction (flops over its event-timed launch)."""
+        """The heaviest contraction as a whole: its tile classes run in one
+        launch, so the unit that reaches the MFMA bound together is the
+        contraction (flops over its event-timed launch)."""
         ms = float(res["per_launch_ms"][dom])
         tf = runner.flops[dom] / (ms * 1e-3) / 1e12
         return {"unit_of_work": f"contraction {dom} (all tile classes)", "ms_per_launch": round(ms, 5),

@@ -195,10 +195,10 @@ qlt_status qlt_set_split_min_mean_k(double min_mean_k);
 double qlt_get_split_min_mean_k(void);
 
 /* Row panels (default on, 1), read when a plan is built: the narrow output
- * blocks (n <= 4) that share their coordinates on A's saved axes, and
- * together read at most 4 contracted columns of A', run as one unit that
- * reads each A element once for all of them.  0 keeps every such block on
- * the per-block row kernel.  The values are bitwise the same either way
+ * blocks (n <= 4, contracted extent <= 64) that share their coordinates on A's
+ * saved axes, and together read at most 4 contracted columns of A', run as one
+ * unit that reads each A element once for all of them.  0 keeps every such block
+ * on the per-block row kernel.  The values are bitwise the same either way
  * (same sums in the same order).  An execution-strategy knob with no
  * reference counterpart (the reference runs one BLAS call per task,
  * global_operations.h:919-978). */
@@ -213,8 +213,8 @@ int32_t qlt_get_row_panels(void);
  * 1: 32x64, 2: 64x32, 3: 32x32; -1: the built-in rule, which takes 32 in a
  * dimension when that pads at most 9/10 as much as 64).  slice_target[c] is the
  * workgroup count that k-slicing of tile class c aims at (0: the built-in
- * 512 for the MFMA classes 0-3, 2048 for classes 4 and 5, the narrow-output
- * row classes).  A plan keeps
+ * 512 for the MFMA classes 0-3, 2048 for classes 4 and 5, the narrow
+ * outputs).  A plan keeps
  * the tuning in effect when it was built. */
 #define QLT_TUNE_BUCKETS 16
 #define QLT_TILE_CLASSES 6
