@@ -234,8 +234,12 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 // way at D = 2048 FP64), 8-deep complex steps at four workgroups per CU (1.14
 // ms either way at D = 4096), B' fragments loaded past LDS (249 -> 308 us), and
 // 64 x 64 tiles (303 -> 376 us).
-// The staged chunk, double-buffered, real and imaginary planes: A' by rows (18
-// doubles apart), B' by k (TN + 4 doubles apart), contracted index p at place
+// The staged chunk, real and imaginary planes, in one buffer (the next chunk
+// waits in registers): with two a step takes one barrier less, but twice the LDS,
+// and was slower at the same number of workgroups per CU (D = 2048 FP64 matvec 255
+// -> 246 us with its data in the cache, D = 4096 complex128 1.146 -> 1.119 ms; at
+// four complex workgroups per CU, which one buffer leaves room for, the registers
+// spill: 1.139 ms).  A' by rows (18 doubles apart), B' by k (TN + 4 doubles apart), contracted index p at place
 // k_place(p).  Lane (lr, lk) finds the indices lk, 4 + lk, 8 + lk, 12 + lk of the four
 // MFMA steps at places 4 lk .. 4 lk + 3: A' is read in 16-byte pieces, and both
 // strides keep a wave's reads and the k-contiguous / n-contiguous writes free
@@ -246,8 +250,8 @@ __device__ __forceinline__ int k_place(int p) { return ((p & 3) << 2) | (p >> 2)
 template <bool CPLX, int TMv, int TNv>
 struct GroupedShared {
   static constexpr int P = CPLX ? 2 : 1;
-  double As[2][P][TMv][KC + 2];
-  double Bs[2][P][KC][TNv + 4];
+  double As[P][TMv][KC + 2];
+  double Bs[P][KC][TNv + 4];
 };
 template <bool CPLX, int TMv, int TNv, typename E>
 __device__ __forceinline__ void grouped_tile(
@@ -292,7 +296,7 @@ __device__ __forceinline__ void grouped_tile(
   for (int nt = 0; nt < BN; ++nt) nt_ok[nt] = j0 + wn + nt * 16 < seg.n;
   const bool wave_on = mt_ok[0] && nt_ok[0];
   typedef double v2d __attribute__((ext_vector_type(2)));
-  auto compute = [&](int buf, int kv) {
+  auto compute = [&](int kv) {
     if (!wave_on) return;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -301,15 +305,15 @@ __device__ __forceinline__ void grouped_tile(
       double b[2][BN], bi[2][BN];
 #pragma unroll
       for (int mt = 0; mt < BM; ++mt) {
-        a[mt] = *reinterpret_cast<const v2d *>(&As[buf][0][wm + mt * 16 + lr][4 * lk + 2 * h]);
-        if (CPLX) ai[mt] = *reinterpret_cast<const v2d *>(&As[buf][P - 1][wm + mt * 16 + lr][4 * lk + 2 * h]);
+        a[mt] = *reinterpret_cast<const v2d *>(&As[0][wm + mt * 16 + lr][4 * lk + 2 * h]);
+        if (CPLX) ai[mt] = *reinterpret_cast<const v2d *>(&As[P - 1][wm + mt * 16 + lr][4 * lk + 2 * h]);
       }
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int nt = 0; nt < BN; ++nt) {
-          b[u][nt] = Bs[buf][0][4 * lk + 2 * h + u][wn + nt * 16 + lr];
-          if (CPLX) bi[u][nt] = Bs[buf][P - 1][4 * lk + 2 * h + u][wn + nt * 16 + lr];
+          b[u][nt] = Bs[0][4 * lk + 2 * h + u][wn + nt * 16 + lr];
+          if (CPLX) bi[u][nt] = Bs[P - 1][4 * lk + 2 * h + u][wn + nt * 16 + lr];
         }
 #pragma unroll
       for (int mt = 0; mt < BM; ++mt) {
@@ -343,7 +347,7 @@ __device__ __forceinline__ void grouped_tile(
   const bool seg_plain = (seg.flags & (kSegAPlain | kSegBPlain)) == (kSegAPlain | kSegBPlain);
   const bool seg_affine = (seg.flags & (kSegAColAffine | kSegBRowAffine)) == (kSegAColAffine | kSegBRowAffine);
   raw_t<E, CPLX> pa[QA], pb[QB];
-  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks, buf = 0;
+  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks;
   ExecTask et = exec[t];
   int kv = min(KC, et.k - kk);
   if (seg_affine) {
@@ -400,7 +404,7 @@ __device__ __forceinline__ void grouped_tile(
         bptr[q] += b_adv;
       }
     };
-    auto pstage = [&](int buf, int kvalid) {
+    auto pstage = [&](int kvalid) {
       if (kvalid < KC) {
 #pragma unroll
         for (int q = 0; q < QA; ++q) zero_unless<E, CPLX>(pa[q], ap < kvalid);
@@ -409,18 +413,18 @@ __device__ __forceinline__ void grouped_tile(
       }
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
-        As[buf][0][ar0 + 16 * q][apl] = re_of(pa[q]);
-        if (CPLX) As[buf][P - 1][ar0 + 16 * q][apl] = im_of(pa[q]);
+        As[0][ar0 + 16 * q][apl] = re_of(pa[q]);
+        if (CPLX) As[P - 1][ar0 + 16 * q][apl] = im_of(pa[q]);
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
-        Bs[buf][0][k_place(bp0 + BPS * q)][bc] = re_of(pb[q]);
-        if (CPLX) Bs[buf][P - 1][k_place(bp0 + BPS * q)][bc] = im_of(pb[q]);
+        Bs[0][k_place(bp0 + BPS * q)][bc] = re_of(pb[q]);
+        if (CPLX) Bs[P - 1][k_place(bp0 + BPS * q)][bc] = im_of(pb[q]);
       }
     };
     setup(et, kk);
     pfetch(kv);
-    pstage(0, kv);
+    pstage(kv);
     __syncthreads();
     for (;;) {
       --left;
@@ -435,10 +439,10 @@ __device__ __forceinline__ void grouped_tile(
         kv2 = min(KC, et.k - kk);
         pfetch(kv2);
       }
-      compute(buf, kv);
+      compute(kv);
       if (left == 0) break;
-      buf ^= 1;
-      pstage(buf, kv2);
+      __syncthreads();
+      pstage(kv2);
       __syncthreads();
       kv = kv2;
     }
@@ -492,7 +496,7 @@ __device__ __forceinline__ void grouped_tile(
         pb[q] = ld_raw<E, CPLX>(B + (e.b_off + row + b_col[q]) * P);
       }
     };
-    auto stage = [&](int buf, int kvalid) {
+    auto stage = [&](int kvalid) {
       if (kvalid < KC) {
 #pragma unroll
         for (int q = 0; q < QA; ++q) zero_unless<E, CPLX>(pa[q], a_p(q) < kvalid);
@@ -501,18 +505,18 @@ __device__ __forceinline__ void grouped_tile(
       }
 #pragma unroll
       for (int q = 0; q < QA; ++q) {
-        As[buf][0][a_r(q)][k_place(a_p(q))] = re_of(pa[q]);
-        if (CPLX) As[buf][P - 1][a_r(q)][k_place(a_p(q))] = im_of(pa[q]);
+        As[0][a_r(q)][k_place(a_p(q))] = re_of(pa[q]);
+        if (CPLX) As[P - 1][a_r(q)][k_place(a_p(q))] = im_of(pa[q]);
       }
 #pragma unroll
       for (int q = 0; q < QB; ++q) {
-        Bs[buf][0][k_place(b_p(q))][b_c(q)] = re_of(pb[q]);
-        if (CPLX) Bs[buf][P - 1][k_place(b_p(q))][b_c(q)] = im_of(pb[q]);
+        Bs[0][k_place(b_p(q))][b_c(q)] = re_of(pb[q]);
+        if (CPLX) Bs[P - 1][k_place(b_p(q))][b_c(q)] = im_of(pb[q]);
       }
     };
     task_rows(et);
     fetch(et, kk, kv);
-    stage(0, kv);
+    stage(kv);
     __syncthreads();
     for (;;) {
       --left;
@@ -527,10 +531,10 @@ __device__ __forceinline__ void grouped_tile(
         kv2 = min(KC, et.k - kk);
         fetch(et, kk, kv2);
       }
-      compute(buf, kv);
+      compute(kv);
       if (left == 0) break;
-      buf ^= 1;
-      stage(buf, kv2);
+      __syncthreads();
+      stage(kv2);
       __syncthreads();
       kv = kv2;
     }
