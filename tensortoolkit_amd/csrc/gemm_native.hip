@@ -239,8 +239,8 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 // and was slower at the same number of workgroups per CU (D = 2048 FP64 matvec 255
 // -> 246 us with its data in the cache, D = 4096 complex128 1.146 -> 1.119 ms; at
 // four complex workgroups per CU, which one buffer leaves room for, the registers
-// spill: 1.139 ms).  A' by rows (18 doubles apart), B' by k (TN + 4 doubles apart), contracted index p at place
-// k_place(p).  Lane (lr, lk) finds the indices lk, 4 + lk, 8 + lk, 12 + lk of the four
+// spill: 1.139 ms).  A' by rows (18 doubles apart), B' by k (TN + 4 doubles apart),
+// contracted index p at place k_place(p).  Lane (lr, lk) finds the indices lk, 4 + lk, 8 + lk, 12 + lk of the four
 // MFMA steps at places 4 lk .. 4 lk + 3: A' is read in 16-byte pieces, and both
 // strides keep a wave's reads and the k-contiguous / n-contiguous writes free
 // of bank conflicts (with both operands by k and rows one double more than a
