@@ -658,7 +658,7 @@ __device__ __forceinline__ void narrow_tile(
         kk = 0;
       }
       if (n == 0) break;
-      const int here = (tk - kk + KC - 1) / KC;
+      const int here = chunks_from(kk, tk);
       if (n < here) {
         kk += KC * n;
         break;
@@ -710,11 +710,12 @@ __device__ __forceinline__ void narrow_tile(
       if constexpr (kLaneRuns) {
         a_run = a_aff && cs == 1;
         b_run = b_aff && rs == 1;
+        const int64_t off = run_offset(kk + KS * lk, P);
         if (a_run) {
-          ld_run<E, CPLX, KS>(ap[0] + (kk + KS * lk) * P, a[s][0]);
-          if (m1_ok) ld_run<E, CPLX, KS>(ap[1] + (kk + KS * lk) * P, a[s][1]);
+          ld_run<E, CPLX, KS>(ap[0] + off, a[s][0]);
+          if (m1_ok) ld_run<E, CPLX, KS>(ap[1] + off, a[s][1]);
         }
-        if (b_run) ld_run<E, CPLX, KS>(bp + (kk + KS * lk) * P, b[s]);
+        if (b_run) ld_run<E, CPLX, KS>(bp + off, b[s]);
       }
       if (!a_run) {
 #pragma unroll

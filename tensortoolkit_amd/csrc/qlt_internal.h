@@ -221,6 +221,13 @@ __host__ __device__ constexpr int64_t tiles_of(int32_t cls, int64_t m, int64_t n
 // k extent of one pipeline step of the MFMA kernels; a task of contracted
 // extent k takes ceil(k / kKChunk) steps.
 constexpr int32_t kKChunk = 16;
+// A block holds up to 2^31 - 1 elements and so does its contracted extent:
+// stored reals up to contracted index k of an operand contiguous in it
+// (`parts`: 2 for complex elements) pass 2^31, and a sum rounded up to whole
+// chunks before it is divided would, too.
+__host__ __device__ constexpr int64_t run_offset(int32_t k, int32_t parts) { return static_cast<int64_t>(k) * parts; }
+// Chunks from index k (0 <= k < extent) to the end of a task.
+__host__ __device__ constexpr int32_t chunks_from(int32_t k, int32_t extent) { return (extent - k - 1) / kKChunk + 1; }
 
 // One output tile of the grouped kernel, or one k-slice of it.  A k-slice
 // covers `n_chunks` consecutive steps of the output block's (task, k-chunk)
