@@ -79,7 +79,7 @@ qlt_status time_workload(int32_t n_items, const qlt_tune_item *items, int32_t dt
         (*weights)[{bm, bn}] += static_cast<double>(sg.m) * sg.n * static_cast<double>(sg.k_total);
       }
     if (cls_tiles != nullptr)
-      for (int c = 0; c < kNumTileClasses; ++c) cls_tiles[c] += p->cls_tiles[c];
+      for (int c = 0; c < kNumTileClasses; ++c) cls_tiles[tuning_class(c)] += p->cls_tiles[c];
   }
   const double alpha[2] = {1.0, 0.0}, beta[2] = {0.0, 0.0};
   auto run_all = [&]() -> qlt_status {
@@ -155,7 +155,7 @@ qlt_status qlt_autotune(int32_t n_items, const qlt_tune_item *items, int32_t dty
   const qlt_tuning entry = tuning_snapshot();
 
   std::map<Bucket, double> weights;
-  int64_t cls_tiles[kNumTileClasses] = {0, 0, 0, 0, 0, 0};
+  int64_t cls_tiles[QLT_TILE_CLASSES] = {};
   double base_ms = 0.0;
   QLT_TRY(time_workload(n_items, items, dtype, mode, reps, st, &base_ms, &weights, cls_tiles));
   int32_t trials = 1;
@@ -194,7 +194,7 @@ qlt_status qlt_autotune(int32_t n_items, const qlt_tune_item *items, int32_t dty
     }
   }
   const int32_t targets[] = {512, 1024, 2048, 4096, -1};
-  for (int c = 0; c < kNumTileClasses; ++c) {
+  for (int c = 0; c < QLT_TILE_CLASSES; ++c) {
     if (cls_tiles[c] == 0) continue;
     for (int32_t tg : targets) {
       const int32_t now = cur.slice_target[c] == 0 ? 2048 : cur.slice_target[c];

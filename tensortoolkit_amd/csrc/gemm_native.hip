@@ -573,21 +573,25 @@ __device__ __forceinline__ void grouped_tile(
   tile_epilogue<CPLX, BM, BN, E>(seg, i0 + wm + lk, j0 + wn + lr, acc, acc_i, C, alpha_r, alpha_i, beta_r, beta_i);
 }
 
-// Narrow outputs (4 < n <= 16): one workgroup per 32 x 16 tile (two MFMA
-// blocks of 16 x 16) or k-slice of it, its four waves taking every fourth
-// 16-k chunk of the tile's (task, chunk) sequence and meeting in LDS at the
-// end (sums in wave order).  The operand fragments are loaded from global
-// memory straight into the registers the MFMA reads (lane lr = lane % 16 holds
-// A' row / B' column lr, lk = lane / 16 the contracted index), so no wave waits
-// for another inside the loop, and the loads of one stage are issued before
+// Narrow outputs (n <= 16): 32 x 16 tiles of two MFMA blocks of 16 x 16.  KW = 4: a
+// workgroup takes one tile or k-slice of it, its four waves every fourth
+// 16-k chunk of the tile's (task, chunk) sequence, and they meet in LDS at the
+// end (sums in wave order).  KW = 1: a workgroup takes four tiles, a wave each,
+// which walks all of its tile's chunks.  The operand fragments are loaded from
+// global memory straight into the registers the MFMA reads (lane lr = lane % 16
+// holds A' row / B' column lr, lk = lane / 16 the contracted index), so no wave
+// waits for another inside the loop, and the loads of one stage are issued before
 // the MFMAs of the previous one (two register sets).
-//   What bounds it is latency: few tiles, each a long chain of chunks.  A row
-// kernel with one thread per row and an LDS chunk of B' per step walked the
-// chain alone, about 1 us per 16 k: a complex64 contraction onto n <= 16
-// outputs 143 -> 27 us, the n <= 16 tiles of a lognormal FP64 matvec 46 -> 15 us
-// per contraction.  The same unstaged form for n > 16 is slower than the LDS
-// tiles (D = 4096 complex128 matvec 1.23 -> 1.41 ms): there the fragments'
-// uncoalesced lines bound it, so it stays with this class.
+//   What bounds it is latency: with KW = 4 of few tiles, each a long chain of
+// chunks, which a kernel with one thread per row and an LDS chunk of B' per step
+// walked alone, about 1 us per 16 k: a complex64 contraction onto n <= 16 outputs
+// 143 -> 27 us, the n <= 16 tiles of a lognormal FP64 matvec 46 -> 15 us per
+// contraction.  With KW = 1 of many tiles of few chunks: the chain of a tile's
+// records, its loads and its stores, against the waves in flight (complex: two k-steps
+// a stage instead of four for them; n = 8, k = 16, m = 10^6, complex64: 150 us with KW = 4, 77
+// with four, 69 with two; one thread per row 82).  The same unstaged form for n > 16
+// is slower than the LDS tiles (D = 4096 complex128 matvec 1.23 -> 1.41 ms): there the
+// fragments' uncoalesced lines bound it, so it stays with these classes.
 //   Full stages of the types of at most 8 bytes per element give lane (lr, lk)
 // the KS consecutive contracted indices KS lk .. KS lk + KS - 1, so that an
 // operand contiguous in k is read in 16-byte pieces; complex128 and a task's
@@ -622,22 +626,27 @@ __device__ __forceinline__ void ld_run(const E *p, raw_t<E, CPLX> (&x)[KS]) {
   }
 }
 
-template <bool CPLX, typename E>
+template <bool CPLX, int KW, typename E>
 __device__ __forceinline__ void narrow_tile(
     char *smem, const Tile tile, const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
     const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb, const GatherLayout &L,
     const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part,
     double alpha_r, double alpha_i, double beta_r, double beta_i) {
   constexpr int P = CPLX ? 2 : 1;
-  constexpr int KW = kNarrowWaves, BM = kNarrowM / 16;
-  constexpr int KS = sizeof(E) == 8 ? 2 : 4;   // k-steps of 4 per stage (their registers bound k_all_classes)
+  constexpr int BM = kNarrowM / 16;
+  constexpr int kTileRows = kNarrowM * (kNarrowWaves / KW);   // of the workgroup
+  // k-steps of 4 per stage: their registers bound k_all_classes (KW = 4) and the waves in flight (KW = 1)
+  constexpr int KS = sizeof(E) == 8 || (CPLX && KW == 1) ? 2 : 4;
   constexpr int SK = 4 * KS;
   constexpr bool kLaneRuns = sizeof(E) * P <= 8;
   using R = raw_t<E, CPLX>;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const Seg seg = segs[tile.seg];
-  const int i0 = tile.tm * kNarrowM;
+  const int wk = KW > 1 ? w : 0;                              // the wave's place in its tile's chunks
+  const int r0 = KW > 1 ? 0 : kNarrowM * w;                   // its rows' place in the workgroup's
+  const int i0 = tile.tm * kTileRows + r0;
+  if (KW == 1 && i0 >= seg.m) return;
   const bool m1_ok = i0 + 16 < seg.m;
   v4d acc[P][BM];
 #pragma unroll
@@ -647,7 +656,7 @@ __device__ __forceinline__ void narrow_tile(
   R a[2][BM][KS], b[2][KS];
 
   // position: task t (k extent tk), contracted index kk, chunks left
-  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks - w;
+  int t = tile.t_begin, kk = tile.k_begin, left = tile.n_chunks - wk;
   int tk = 0;
   // moves n chunks forward from chunk start kk (which may equal or pass tk)
   auto skip = [&](int n) {
@@ -710,12 +719,11 @@ __device__ __forceinline__ void narrow_tile(
       if constexpr (kLaneRuns) {
         a_run = a_aff && cs == 1;
         b_run = b_aff && rs == 1;
-        const int64_t off = run_offset(kk + KS * lk, P);
         if (a_run) {
-          ld_run<E, CPLX, KS>(ap[0] + off, a[s][0]);
-          if (m1_ok) ld_run<E, CPLX, KS>(ap[1] + off, a[s][1]);
+          ld_run<E, CPLX, KS>(ap[0] + run_offset(kk + KS * lk, P), a[s][0]);
+          if (m1_ok) ld_run<E, CPLX, KS>(ap[1] + run_offset(kk + KS * lk, P), a[s][1]);
         }
-        if (b_run) ld_run<E, CPLX, KS>(bp + off, b[s]);
+        if (b_run) ld_run<E, CPLX, KS>(bp + run_offset(kk + KS * lk, P), b[s]);
       }
       if (!a_run) {
 #pragma unroll
@@ -782,7 +790,7 @@ __device__ __forceinline__ void narrow_tile(
   };
   if (left > 0) {
     tk = exec[t].k;
-    skip(w);
+    skip(wk);
     int kv0 = load(0);
     for (;;) {
       bool more = advance(kv0);
@@ -795,6 +803,40 @@ __device__ __forceinline__ void narrow_tile(
       compute(1, kv1);
       if (!more) break;
     }
+  }
+
+  if constexpr (KW == 1) {
+    // element v of a lane is row 4 v + lk of its MFMA block; a k-slice stores its
+    // unscaled partial sum, row-major over the workgroup's rows
+    double *pp = tile.part >= 0 ? part + static_cast<int64_t>(tile.part) * (kTileRows * kNarrowN * P) : nullptr;
+    const bool use_beta = pp == nullptr && (beta_r != 0.0 || beta_i != 0.0);
+    R old[BM][4];
+#pragma unroll
+    for (int mt = 0; mt < BM; ++mt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        old[mt][v] = R{};
+        if (use_beta) {
+          const int row = i0 + 16 * mt + 4 * v + lk;
+          const bool ok = row < seg.m && lr < seg.n;
+          old[mt][v] = ld_raw<E, CPLX>(C + P * (seg.c_off + (ok ? static_cast<int64_t>(row) * seg.n + lr : 0)));
+        }
+      }
+#pragma unroll
+    for (int mt = 0; mt < BM; ++mt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int lrow = 16 * mt + 4 * v + lk;
+        const double xr = acc[0][mt][v], xi = CPLX ? acc[P - 1][mt][v] : 0.0;
+        if (pp != nullptr) {
+          pp[(r0 + lrow) * kNarrowN + lr] = xr;
+          if (CPLX) pp[kTileRows * kNarrowN + (r0 + lrow) * kNarrowN + lr] = xi;
+        } else if (i0 + lrow < seg.m && lr < seg.n) {
+          st_scaled<E, CPLX>(C + P * (seg.c_off + static_cast<int64_t>(i0 + lrow) * seg.n + lr), xr, xi, old[mt][v],
+                             use_beta, alpha_r, alpha_i, beta_r, beta_i);
+        }
+      }
+    return;
   }
 
   // wave w takes the accumulator element v = w of every lane, from all waves
@@ -1320,7 +1362,7 @@ struct ExecArgs {
 
 // Order of the classes in k_all_classes: the few narrow-output tiles, whose
 // chains of contracted indices are the longest, start first.
-constexpr int32_t kLaunchOrder[kNumTileClasses - 1] = {kTileRows16, kTileRows4, 1, 3, kNumTileClasses};
+constexpr int32_t kLaunchOrder[] = {kTileNarrow, kTileRows4, 1, 3, kNumTileClasses};
 
 // Workgroup `b` of `n` of class CLS.
 template <bool CPLX, int CLS, typename E>
@@ -1330,9 +1372,12 @@ __device__ __forceinline__ void class_block(char *smem, const ExecArgs<E> &x, in
   if constexpr (CLS == kTileRows4)
     rows_tile<CPLX, 4, 4, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar,
                              x.ai, x.br, x.bi);
-  else if constexpr (CLS == kTileRows16)
-    narrow_tile<CPLX, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar, x.ai,
-                         x.br, x.bi);
+  else if constexpr (CLS == kTileNarrowRows)
+    narrow_tile<CPLX, 1, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar,
+                            x.ai, x.br, x.bi);
+  else if constexpr (CLS == kTileNarrow)
+    narrow_tile<CPLX, kNarrowWaves, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C,
+                                       part, x.ar, x.ai, x.br, x.bi);
   else
     grouped_tile<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS), E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C,
                                           part, x.ar, x.ai, x.br, x.bi);
@@ -1340,7 +1385,8 @@ __device__ __forceinline__ void class_block(char *smem, const ExecArgs<E> &x, in
 template <bool CPLX, int CLS>
 constexpr size_t class_shared() {
   if constexpr (CLS == kTileRows4) return sizeof(RowsShared<CPLX, 4>);
-  else if constexpr (CLS == kTileRows16) return sizeof(NarrowShared<CPLX>);
+  else if constexpr (CLS == kTileNarrow) return sizeof(NarrowShared<CPLX>);
+  else if constexpr (CLS == kTileNarrowRows) return 16;
   else return sizeof(GroupedShared<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS)>);
 }
 
@@ -1367,15 +1413,15 @@ __global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
 template <bool CPLX, bool STREAM, typename E>
 __global__ __launch_bounds__(256, CPLX ? 3 : 5) void k_all_classes(const ExecArgs<E> x) {
   constexpr size_t kBytes = std::max({class_shared<CPLX, 1>(), class_shared<CPLX, 3>(), class_shared<CPLX, 4>(),
-                                      class_shared<CPLX, 5>(), sizeof(PanelShared<CPLX>)});
+                                      class_shared<CPLX, 6>(), sizeof(PanelShared<CPLX>)});
   __shared__ __align__(16) char smem[kBytes];
   const int b = static_cast<int>(blockIdx.x);
-  if (b < x.block0[4]) class_block<CPLX, 5, E>(smem, x, b - x.block0[5], x.count[5]);
+  if (b < x.block0[4]) class_block<CPLX, 6, E>(smem, x, b - x.block0[6], x.count[6]);
   else if (b < x.block0[1]) class_block<CPLX, 4, E>(smem, x, b - x.block0[4], x.count[4]);
   else if (b < x.block0[3]) class_block<CPLX, 1, E>(smem, x, b - x.block0[1], x.count[1]);
-  else if (b < x.block0[6]) class_block<CPLX, 3, E>(smem, x, b - x.block0[3], x.count[3]);
+  else if (b < x.block0[7]) class_block<CPLX, 3, E>(smem, x, b - x.block0[3], x.count[3]);
   else
-    panel_tile<CPLX, STREAM, E>(smem, x.ptiles[b - x.block0[6]], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai,
+    panel_tile<CPLX, STREAM, E>(smem, x.ptiles[b - x.block0[7]], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai,
                                 x.br, x.bi);
 }
 // The k-slice sums of reduction items first, first + 1, ...
@@ -1390,6 +1436,7 @@ __global__ __launch_bounds__(256) void k_reduce(const ExecArgs<E> x, int first) 
     case 2: reduce_slices<CPLX, 64, 32, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
     case 3: reduce_slices<CPLX, 32, 32, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
     case kTileRows4: reduce_rows<CPLX, 4, 4, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
+    case kTileNarrowRows: reduce_slices<CPLX, kNarrowM * kNarrowWaves, kNarrowN, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
     default: reduce_slices<CPLX, kNarrowM, kNarrowN, E>(it, seg, part, x.C, x.ar, x.ai, x.br, x.bi); break;
   }
 }
@@ -1425,18 +1472,21 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
       }
     if (runs(kPanelId) && plan->panel_mkn > best) dom = kPanelId;
   }
-  // one launch for all classes; a probed class, and the 64-row classes that
-  // k_all_classes leaves out, take a launch per class on the class streams
-  const bool fused = dom < 0 && n_cls >= 2 && !runs(0) && !runs(2) &&
-                     plan->n_tiles + plan->n_ptiles < (int64_t(1) << 31);
+  // One stream, and one launch for the classes that k_all_classes holds; a
+  // probed class, and the 64-row classes, take a launch per class on the class
+  // streams.  The kTileNarrowRows class fills the chip by itself and has a launch of
+  // its own before the others'.  A launch holds less than 2^32 threads.
+  const bool one_stream = dom < 0 && !runs(0) && !runs(2);
+  const bool fused = one_stream && n_cls - (runs(kTileNarrowRows) ? 1 : 0) >= 2 &&
+                     plan->n_tiles + plan->n_ptiles < (int64_t(1) << 24);
   std::unique_ptr<ClassStreams> own;
   ClassStreams *cs = shared;
-  if (cs == nullptr && n_cls >= 2 && !fused) {
+  if (cs == nullptr && n_cls >= 2 && !one_stream) {
     own = std::make_unique<ClassStreams>(st);
     cs = own.get();
   }
   auto stream_of = [&](int32_t cls) {
-    if (cls == kPanelId) cls = kTileRows4;
+    if (cls == kPanelId || one_stream) cls = kTileRows4;
     return cs != nullptr ? cs->get(cls) : st;
   };
   auto probe_in = [&](int32_t cls) {
@@ -1449,7 +1499,7 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     static const char *const kNames[kNumTileClasses + 1] = {
         "k_grouped_gemm_f64<64x64>", "k_grouped_gemm_f64<32x64>", "k_grouped_gemm_f64<64x32>",
         "k_grouped_gemm_f64<32x32>", "k_rows_f64<n<=4>",          "k_rows_f64<n<=16>",
-        "k_panel_rows"};
+        "k_rows_f64<n<=16>",          "k_panel_rows"};
     char name[64];
     static const char *const kTypes[4] = {"f64", "c128", "f32", "c64"};
     std::snprintf(name, sizeof(name), "%s %s", kNames[cls], kTypes[dtype & 3]);
@@ -1509,13 +1559,6 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     // 0.83 GB W contraction 0.169 -> 0.148 ms with the hint, a small one
     // 0.028 -> 0.032 ms)
     const bool stream_a = plan->panel_elems * static_cast<double>(sizeof(E) * (CX ? 2 : 1)) > kPanelStreamBytes;
-    if (fused) {
-      const hipStream_t ls = stream_of(kTileRows4);
-      if (stream_a) hipLaunchKernelGGL((k_all_classes<CX, true, E>), grid_of(blocks), block, 0, ls, x);
-      else hipLaunchKernelGGL((k_all_classes<CX, false, E>), grid_of(blocks), block, 0, ls, x);
-      if (n_red > 0) hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(n_red), block, 0, ls, x, static_cast<int>(first_red));
-      return;
-    }
     auto one = [&](auto cls_tag) {
       constexpr int CLS = decltype(cls_tag)::value;
       if (!runs(CLS)) return;
@@ -1525,15 +1568,23 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
       probe_out(CLS);
       // k-sliced tiles: the slices wrote partial sums; one workgroup per sliced
       // tile adds them and applies alpha / beta
-      if (plan->cls_red[CLS] > 0)
+      if (!fused && plan->cls_red[CLS] > 0)
         hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(plan->cls_red[CLS]), block, 0, ls, x, red0[CLS]);
     };
+    one(std::integral_constant<int, kTileNarrowRows>{});
+    if (fused) {
+      const hipStream_t ls = stream_of(kTileRows4);
+      if (stream_a) hipLaunchKernelGGL((k_all_classes<CX, true, E>), grid_of(blocks), block, 0, ls, x);
+      else hipLaunchKernelGGL((k_all_classes<CX, false, E>), grid_of(blocks), block, 0, ls, x);
+      if (n_red > 0) hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(n_red), block, 0, ls, x, static_cast<int>(first_red));
+      return;
+    }
     one(std::integral_constant<int, 0>{});
     one(std::integral_constant<int, 1>{});
     one(std::integral_constant<int, 2>{});
     one(std::integral_constant<int, 3>{});
-    one(std::integral_constant<int, 4>{});
-    one(std::integral_constant<int, 5>{});
+    one(std::integral_constant<int, kTileRows4>{});
+    one(std::integral_constant<int, kTileNarrow>{});
     // row panels, after the n <= 4 row class on its stream
     if (runs(kPanelId)) {
       const hipStream_t ls = stream_of(kPanelId);

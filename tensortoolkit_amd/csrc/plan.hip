@@ -609,6 +609,62 @@ qlt_status build_panels(qlt_plan *plan, HostBuild &hb, std::vector<char> &in_pan
   return QLT_OK;
 }
 
+// Beyond kPanelCols, so that what a row panel may take stays with the row class.
+constexpr int64_t kRows4MaxK = 64;
+
+// Class of every n <= 16 output block, from measurements of single blocks of m
+// rows in FP64, complex128 and complex64 with A in either memory order, and of
+// blocks of many short tasks (us; k: contracted extent).
+//   4 < n <= 16: a chain of steps shared by four waves (kTileNarrow) while the
+// 32-row tiles are too few to fill the chip, else a tile per wave
+// (kTileNarrowRows): shared, waves without a step idle and all four meet in LDS.
+// The line is 1024 tiles for each 16-k step, 2048 for each of more than four that
+// are not short (shared | a wave each, n = 8, complex128: k = 16, m = 10^4 5.0 | 6.5, m =
+// 10^5 17.8 | 13.2, m = 10^6 163 | 96; k = 64, m = 10^5 29.9 | 31.4; k = 128, m = 3 10^5
+// 150 | 157, m = 10^6 474 | 458; complex64, k = 16, m = 10^6 150 | 69).
+//   n <= 4, k <= 64: the row class, in which row panels look for their members.
+//   n <= 4, k > 64: the row class walks its steps one after the other (a U(1)
+// chi = 16 pair of rank-4 tensors, FP64: 43 us, as kTileNarrow 13), but reads A
+// once in whole lines when k is not A's innermost axis or the tasks are short,
+// and is the faster one when its 1024-row tiles are many (n = 1, rows | kTileNarrow:
+// k = 128, k not innermost, complex64, m = 10^5 43 | 43, m = 10^6 181 | 391; k
+// innermost, FP64, m = 10^6 1089 | 223; 100 tasks of k = 1, FP64, m = 3000 25 | 14,
+// m = 30 000 32 | 46, m = 10^5 43 | 127; 40 tasks of k = 4, m = 30 000 28 | 24).
+constexpr int64_t kShortK = 4;
+constexpr int64_t kNarrowTilesPerStep = 1024;
+constexpr int64_t kRowsTilesStream = 256;   // tiles
+constexpr int64_t kRowsStepsShort = 1536;   // tiles times steps
+void choose_narrow_classes(qlt_plan *plan, const std::vector<BlkShape> &a) {
+  const int64_t rows4 = plan->cls_tiles[kTileRows4], tiles32 = plan->cls_tiles[kTileNarrow];
+  for (Seg &sg : plan->h_segs) {
+    const bool long_rows = sg.cls == kTileRows4 && sg.k_total > kRows4MaxK;
+    const bool many_tiles = sg.cls == kTileNarrow && tiles32 >= kNarrowTilesPerStep;
+    if (!long_rows && !many_tiles) continue;
+    int64_t steps = 0;
+    bool all_short = true, streams = true;   // streams: no longer task has k innermost in A
+    for (int32_t t = sg.t0; t < sg.t1; ++t) {
+      const ExecTask &e = plan->h_exec[static_cast<size_t>(t)];
+      const BlkShape &ga = a[static_cast<size_t>(e.a_blk)];
+      steps += chunks_from(0, e.k);
+      if (e.k > kShortK) {
+        all_short = false;
+        if (ga.plain || ga.fastcol) streams = false;
+      }
+    }
+    int32_t to = sg.cls;
+    if (long_rows) {
+      const bool rows = (all_short && rows4 * steps >= kRowsStepsShort) || (streams && rows4 >= kRowsTilesStream);
+      if (!rows) to = kTileNarrow;
+    } else if (tiles32 >= kNarrowTilesPerStep * steps * (steps > 4 && !all_short ? 2 : 1)) {
+      to = kTileNarrowRows;
+    }
+    if (to == sg.cls) continue;
+    plan->cls_tiles[sg.cls] -= tiles_of(sg.cls, sg.m, sg.n);
+    sg.cls = to;
+    plan->cls_tiles[sg.cls] += tiles_of(sg.cls, sg.m, sg.n);
+  }
+}
+
 // k-slicing of long tiles (MFMA and row classes alike).  Per class, a step budget Q = max(kMinSliceChunks,
 // ceil(total steps / T)) is set, T = kSliceTargetWGsMfma (MFMA classes) or kSliceTargetWGs (row classes)
 // unless tuned (qlt_tuning); a tile of w > Q steps is cut into
@@ -660,7 +716,7 @@ qlt_status build_tiles(qlt_plan *plan, HostBuild &hb) {
     const int64_t target = plan->slice_target[cls] > 0 ? plan->slice_target[cls]
                                                        : (is_mfma_class(cls) ? kSliceTargetWGsMfma : kSliceTargetWGs);
     const int64_t q =
-        std::max(cls == kTileRows16 ? kMinSliceChunksNarrow : kMinSliceChunks, (total + target - 1) / target);
+        std::max(cls == kTileNarrow ? kMinSliceChunksNarrow : kMinSliceChunks, (total + target - 1) / target);
     cl.clear();
     cl.reserve(static_cast<size_t>(count));
     int64_t parts = 0;
@@ -854,7 +910,7 @@ qlt_status qlt_plan_build(const qlt_bsdt_desc *a, const qlt_bsdt_desc *b, int32_
   plan->device = current_device();
   plan->c_rank = c_rank;
   plan->c_is_scalar = args.c_is_scalar;
-  for (int c = 0; c < kNumTileClasses; ++c) plan->slice_target[c] = tun.slice_target[c];
+  for (int c = 0; c < kNumTileClasses; ++c) plan->slice_target[c] = tun.slice_target[tuning_class(c)];
   plan->n_a_blks = a->n_blks;
   plan->n_b_blks = b->n_blks;
   {
@@ -1025,7 +1081,6 @@ qlt_status qlt_plan_build(const qlt_bsdt_desc *a, const qlt_bsdt_desc *b, int32_
       sg.flags = kSegAPlain | kSegBPlain | kSegAColAffine | kSegBRowAffine;
       segs.push_back(sg);
       c_raw += m * n;
-      n_tiles += tiles_of(sg.cls, m, n);
       plan->cls_tiles[sg.cls] += tiles_of(sg.cls, m, n);
       // The reference keeps no block for a rank-0 output; its raw size is 1.
       if (!args.c_is_scalar) {
@@ -1060,14 +1115,9 @@ qlt_status qlt_plan_build(const qlt_bsdt_desc *a, const qlt_bsdt_desc *b, int32_
         ExecTask{a_off, b_off, dt.a_pos, dt.b_pos, static_cast<int32_t>(k), 0};
   }
   const int64_t n_c = static_cast<int64_t>(segs.size());
-  for (Seg &sg : segs)
-    if (sg.cls == kTileRows4 && sg.k_total > kRows4MaxK) {
-      const int64_t was = tiles_of(sg.cls, sg.m, sg.n);
-      sg.cls = kTileRows16;
-      plan->cls_tiles[kTileRows4] -= was;
-      plan->cls_tiles[kTileRows16] += tiles_of(sg.cls, sg.m, sg.n);
-      n_tiles += tiles_of(sg.cls, sg.m, sg.n) - was;
-    }
+  choose_narrow_classes(plan.get(), hb.a);
+  n_tiles = 0;
+  for (int c = 0; c < kNumTileClasses; ++c) n_tiles += plan->cls_tiles[c];
   QLT_CHECK_ARG(n_tiles < (int64_t(1) << 31), "qlt_plan_build: more than 2^31 output tiles");
   QLT_CHECK_ARG(kmax < (int64_t(1) << 40), "qlt_plan_build: contracted extent of an output block exceeds 2^40");
   plan->n_exec = nt;

@@ -126,7 +126,7 @@ struct Seg {
   int32_t t0;      // first ExecTask
   int32_t t1;      // one past the last ExecTask
   int64_t k_total; // sum of k over the segment's tasks
-  int32_t cls;     // tile class of the segment (kTileMfma, kTileRows4, kTileRows16)
+  int32_t cls;     // tile class of the segment
   int32_t flags;   // kSegAPlain | kSegBPlain when every task's A (B) block is plain
 };
 constexpr int32_t kSegAPlain = 1;
@@ -159,19 +159,18 @@ __host__ __device__ inline void magic_of(uint32_t d, uint64_t &mag, int32_t &sh)
 // Tile classes.  Classes 0..3: MFMA output tiles of 64x64, 32x64, 64x32 and
 // 32x32 (rows x cols), chosen per output block to limit padding.
 // kTileRows4: narrow outputs (n <= 4) on a row-streaming path, 1024 output
-// rows per workgroup (4 per thread).  kTileRows16: n <= 16, MFMA tiles of 32
-// rows with the contracted extent spread over the workgroup's waves.
+// rows per workgroup (4 per thread).  n <= 16: MFMA tiles of 32 rows, of which
+// a workgroup takes one, its contracted extent spread over the four waves
+// (kTileNarrow), or four, one per wave (kTileNarrowRows).  choose_narrow_class
+// (plan.hip) says which of the three a narrow block takes.
 constexpr int32_t kTileMfma = 0;       // 64 x 64 (first MFMA class)
 constexpr int32_t kNumMfmaClasses = 4;
 constexpr int32_t kTileRows4 = 4;
-constexpr int32_t kTileRows16 = 5;
-constexpr int32_t kNumTileClasses = 6;
-// An n <= 4 block of a longer contracted extent runs with the n <= 16 class: a
-// row tile walks its 16-k steps one after the other, about 1.5 us each, where
-// an MFMA tile's waves share them (a U(1) chi = 16 pair of rank-4 tensors, FP64: 43 ->
-// 13 us).  Beyond
-// kPanelCols, so that what a row panel may take stays with the row class.
-constexpr int64_t kRows4MaxK = 64;
+constexpr int32_t kTileNarrowRows = 5;
+constexpr int32_t kTileNarrow = 6;
+constexpr int32_t kNumTileClasses = 7;
+// The entry of qlt_tuning that holds a class's slice target: both n <= 16 classes share one.
+constexpr int32_t tuning_class(int32_t cls) { return cls == kTileNarrow ? kTileNarrowRows : cls; }
 
 __host__ __device__ constexpr int32_t mfma_tile_m(int32_t cls) { return (cls == 1 || cls == 3) ? 32 : 64; }
 __host__ __device__ constexpr int32_t mfma_tile_n(int32_t cls) { return (cls == 2 || cls == 3) ? 32 : 64; }
@@ -196,7 +195,7 @@ __host__ __device__ constexpr bool prefer_32(int64_t x) {
 // columns when that cuts the padded width by >= 10%, else 64.  m is kept in
 // the signature for the tuning table's buckets.
 __host__ __device__ constexpr int32_t tile_class_of(int64_t m, int64_t n) {
-  return (void)m, n <= 4 ? kTileRows4 : (n <= 16 ? kTileRows16 : 1 + (prefer_32(n) ? 2 : 0));
+  return (void)m, n <= 4 ? kTileRows4 : (n <= 16 ? kTileNarrow : 1 + (prefer_32(n) ? 2 : 0));
 }
 // Tile class of an output block under a tuning table (qlt_tuning): the
 // narrow-output row classes are fixed; an MFMA-class block takes the table
@@ -211,7 +210,9 @@ __host__ __device__ inline int32_t tuned_tile_class(int64_t m, int64_t n,
   const int8_t t = table[bm - 1][bn - 1];
   return (t >= 0 && t < kNumMfmaClasses) ? t : c;
 }
-__host__ __device__ constexpr int32_t rows_per_tile(int32_t cls) { return cls == kTileRows4 ? 1024 : 32; }
+__host__ __device__ constexpr int32_t rows_per_tile(int32_t cls) {
+  return cls == kTileRows4 ? 1024 : cls == kTileNarrowRows ? 128 : 32;
+}
 __host__ __device__ constexpr int64_t tiles_of(int32_t cls, int64_t m, int64_t n) {
   return is_mfma_class(cls)
              ? ((m + mfma_tile_m(cls) - 1) / mfma_tile_m(cls)) * ((n + mfma_tile_n(cls) - 1) / mfma_tile_n(cls))
@@ -388,19 +389,19 @@ struct qlt_plan {
   std::vector<qlt::ExecTask> h_exec;    // host mirror of the execution list
   // k-slicing workgroup target per tile class in effect at build time
   // (0: the built-in target, -1: unsliced)
-  int32_t slice_target[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};
-  int64_t cls_tiles[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};  // tiles per class, class-major in d_tiles
-  double cls_mkn[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};     // sum of m*k*n over the class's tasks
-  double cls_elems[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};   // distinct A + B block elements + C elements
+  int32_t slice_target[qlt::kNumTileClasses] = {};
+  int64_t cls_tiles[qlt::kNumTileClasses] = {};  // tiles per class, class-major in d_tiles
+  double cls_mkn[qlt::kNumTileClasses] = {};     // sum of m*k*n over the class's tasks
+  double cls_elems[qlt::kNumTileClasses] = {};   // distinct A + B block elements + C elements
   double mfma_elems = 0.0;              // the same over all MFMA classes together (blocks counted once)
   // ---- k-slicing of long MFMA tiles (native path) ----
   qlt::ReduceItem *d_red = nullptr;     // class-major reduction items
-  int64_t cls_red[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};
+  int64_t cls_red[qlt::kNumTileClasses] = {};
   // k-slice partial sums, sized for complex128; each tile class owns the
   // region starting at cls_part_off[cls] doubles (the classes run concurrently)
   double *d_part = nullptr;
   size_t part_doubles = 0;
-  int64_t cls_part_off[qlt::kNumTileClasses] = {0, 0, 0, 0, 0, 0};
+  int64_t cls_part_off[qlt::kNumTileClasses] = {};
   // ---- row panels (output blocks of the n <= 4 row class sharing A rows) ----
   bool panels_enabled = true;           // qlt_set_row_panels in effect at build time
   int64_t n_ptiles = 0;
