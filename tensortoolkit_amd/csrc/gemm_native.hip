@@ -104,7 +104,9 @@ __device__ __forceinline__ void st_elem(E *p, double re, double im) {
 // multiply-shift division and no further reads, more take the loop, whose
 // scalar reads of every axis are waited for at every element (they were most
 // of a step of a contraction not affine in k: a U(1) chi = 40 pair of rank-4
-// tensors over cyclic axes, complex64, 99 -> 51 us, FP64 79 -> 38 us).
+// tensors over cyclic axes, complex64, 99 -> 51 us, FP64 79 -> 38 us).  The row
+// class, where 16 threads take the offsets of a step, keeps the plain form: these
+// numbers cost it 16 registers and a wave per SIMD.
 struct PartSplit {
   const BlkGather *g;
   int n;
@@ -933,7 +935,11 @@ __device__ __forceinline__ void reduce_slices(const ReduceItem it, const Seg &se
 // accumulates its n outputs with FP64 FMAs.  Bound by reading A and writing
 // C once.
 constexpr int RK = 16;            // k per stage
-constexpr int kRowsLoadGroup = 8;   // A loads in flight per thread
+// A loads in flight per thread.  A row of 16 contiguous k is one memory line, which
+// a step touches once per group: eight loads at a time instead of sixteen cost
+// up to half of the time (n = 4, k = 16, m = 10^6, FP64: 141 -> 230 us, with the vector
+// loads that k_row_class avoids).
+constexpr int kRowsLoadGroup = 16;
 
 template <bool CPLX, int NMAX, int RPT, typename E>
 __device__ __forceinline__ void rows_epilogue(const Seg &seg, int r0, int tid, const double (&acc)[RPT][NMAX],
@@ -1013,7 +1019,6 @@ __device__ __forceinline__ void rows_tile(
   int t = tile.t_begin, kk = tile.k_begin;
   ExecTask et{};
   bool a_plain = false, b_plain = false;
-  PartSplit a_k{}, b_k{};
   int32_t roff[RPT];
   int cur_task = -1;
   for (int step = 0; step < tile.n_chunks; ++step) {
@@ -1024,24 +1029,23 @@ __device__ __forceinline__ void rows_tile(
       const BlkGather &gB = gb[et.b_blk];
       a_plain = gA.plain != 0;
       b_plain = gB.plain != 0;
-      a_k = part_split<false>(gA, L.a_nc);
-      b_k = part_split<true>(gB, L.b_nr);
-      const PartSplit a_m = part_split<true>(gA, L.a_nr);
-      const PartSplit b_n = part_split<false>(gB, L.b_nc);
 #pragma unroll
       for (int q = 0; q < RPT; ++q) {
         const int row = r0 + tid + 256 * q;
-        roff[q] = (row < seg.m) ? (a_plain ? row * et.k : offset_of<true>(a_m, row)) : -1;
+        roff[q] = (row < seg.m) ? (a_plain ? row * et.k : split_offset(row, gA.rdim, gA.rstr, gA.rmag, gA.rsh, L.a_nr)) : -1;
       }
       __syncthreads();
-      if (tid < NMAX) s_bcol[tid] = (tid < n) ? (b_plain ? tid : offset_of<false>(b_n, tid)) : -1;
+      if (tid < NMAX)
+        s_bcol[tid] = (tid < n) ? (b_plain ? tid : split_offset(tid, gB.cdim, gB.cstr, gB.cmag, gB.csh, L.b_nc)) : -1;
     }
+    const BlkGather &gA = ga[et.a_blk];
+    const BlkGather &gB = gb[et.b_blk];
     if (tid < RK) {
       const int p = kk + tid;
-      s_acol[tid] = (p < et.k) ? (a_plain ? p : offset_of<false>(a_k, p)) : -1;
+      s_acol[tid] = (p < et.k) ? (a_plain ? p : split_offset(p, gA.cdim, gA.cstr, gA.cmag, gA.csh, L.a_nc)) : -1;
     } else if (tid >= 64 && tid < 64 + RK) {
       const int p = kk + tid - 64;
-      s_brow[tid - 64] = (p < et.k) ? (b_plain ? p * n : offset_of<true>(b_k, p)) : -1;
+      s_brow[tid - 64] = (p < et.k) ? (b_plain ? p * n : split_offset(p, gB.rdim, gB.rstr, gB.rmag, gB.rsh, L.b_nr)) : -1;
     }
     __syncthreads();
     if (tid < RK * NMAX) {
@@ -1366,21 +1370,22 @@ constexpr int32_t kLaunchOrder[] = {kTileNarrow, kTileRows4, 1, 3, kNumTileClass
 
 // Workgroup `b` of `n` of class CLS.
 template <bool CPLX, int CLS, typename E>
-__device__ __forceinline__ void class_block(char *smem, const ExecArgs<E> &x, int b, int n) {
-  const Tile *tiles = x.tiles + x.tile0[CLS];
-  double *part = x.part + x.part_off[CLS];
+__device__ __forceinline__ void class_block(char *smem, const ExecArgs<E> &x, int b, int n,
+                                            const Tile *__restrict__ tiles, const Seg *__restrict__ segs,
+                                            const ExecTask *__restrict__ exec, const BlkGather *__restrict__ ga,
+                                            const BlkGather *__restrict__ gb, const E *__restrict__ A,
+                                            const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part) {
+  const Tile tile = tiles[x.tile0[CLS] + xcd_tile(b, n)];
+  double *const cp = part + x.part_off[CLS];
   if constexpr (CLS == kTileRows4)
-    rows_tile<CPLX, 4, 4, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar,
-                             x.ai, x.br, x.bi);
+    rows_tile<CPLX, 4, 4, E>(smem, tile, segs, exec, ga, gb, x.L, A, B, C, cp, x.ar, x.ai, x.br, x.bi);
   else if constexpr (CLS == kTileNarrowRows)
-    narrow_tile<CPLX, 1, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C, part, x.ar,
-                            x.ai, x.br, x.bi);
+    narrow_tile<CPLX, 1, E>(smem, tile, segs, exec, ga, gb, x.L, A, B, C, cp, x.ar, x.ai, x.br, x.bi);
   else if constexpr (CLS == kTileNarrow)
-    narrow_tile<CPLX, kNarrowWaves, E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C,
-                                       part, x.ar, x.ai, x.br, x.bi);
+    narrow_tile<CPLX, kNarrowWaves, E>(smem, tile, segs, exec, ga, gb, x.L, A, B, C, cp, x.ar, x.ai, x.br, x.bi);
   else
-    grouped_tile<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS), E>(smem, tiles[xcd_tile(b, n)], x.segs, x.exec, x.ga, x.gb, x.L, x.A, x.B, x.C,
-                                          part, x.ar, x.ai, x.br, x.bi);
+    grouped_tile<CPLX, mfma_tile_m(CLS), mfma_tile_n(CLS), E>(smem, tile, segs, exec, ga, gb, x.L, A, B, C, cp, x.ar,
+                                                              x.ai, x.br, x.bi);
 }
 template <bool CPLX, int CLS>
 constexpr size_t class_shared() {
@@ -1393,7 +1398,22 @@ constexpr size_t class_shared() {
 template <bool CPLX, int CLS, typename E>
 __global__ __launch_bounds__(256) void k_class(const ExecArgs<E> x) {
   __shared__ __align__(16) char smem[class_shared<CPLX, CLS>()];
-  class_block<CPLX, CLS, E>(smem, x, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  class_block<CPLX, CLS, E>(smem, x, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), x.tiles, x.segs, x.exec,
+                            x.ga, x.gb, x.A, x.B, x.C, x.part);
+}
+// The row classes, whose pointers are restrict-qualified arguments of their
+// own: read from a struct they may alias the output as far as the compiler
+// knows, and the per-task descriptors came by vector loads, each waited for,
+// instead of scalar ones (n = 4, k = 5, m = 1000 in FP64: 7.0 -> 5.3 us).
+template <bool CPLX, int CLS, typename E>
+__global__ __launch_bounds__(256) void k_row_class(const ExecArgs<E> x, const Tile *__restrict__ tiles,
+                                                   const Seg *__restrict__ segs, const ExecTask *__restrict__ exec,
+                                                   const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb,
+                                                   const E *__restrict__ A, const E *__restrict__ B,
+                                                   E *__restrict__ C, double *__restrict__ part) {
+  __shared__ __align__(16) char smem[class_shared<CPLX, CLS>()];
+  class_block<CPLX, CLS, E>(smem, x, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), tiles, segs, exec, ga,
+                            gb, A, B, C, part);
 }
 template <bool CPLX, bool STREAM, typename E>
 __global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
@@ -1409,20 +1429,32 @@ __global__ __launch_bounds__(256) void k_panel_rows(const ExecArgs<E> x) {
 // 184 -> 117 us, U(1)xU(1) complex128 D = 1500 252 -> 156 us, D = 4096 1.22 ->
 // 1.18 ms.  The register bound keeps the occupancy of the widest class alone
 // (complex: three workgroups per CU; unbounded, two, and D = 4096 took 1.35 ms;
-// real: five, with D = 2048 FP64 285 -> 272 us from four; six spill).
+// real: five, with D = 2048 FP64 285 -> 272 us from four; six spill).  The
+// row and grouped classes read through the restrict-qualified arguments, as in
+// k_row_class (D = 2048 FP64 matvec 273.9 -> 273.3 us, D = 4096 complex128
+// 1.116 -> 1.101 ms); the n <= 16 tiles, a chain of few loads, through the struct
+// (complex64 accumulate 49.7 us, 51.3 with scalar loads on the chain).
 template <bool CPLX, bool STREAM, typename E>
-__global__ __launch_bounds__(256, CPLX ? 3 : 5) void k_all_classes(const ExecArgs<E> x) {
+__global__ __launch_bounds__(256, CPLX ? 3 : 5) void k_all_classes(
+    const ExecArgs<E> x, const Tile *__restrict__ tiles, const Seg *__restrict__ segs,
+    const ExecTask *__restrict__ exec, const BlkGather *__restrict__ ga, const BlkGather *__restrict__ gb,
+    const E *__restrict__ A, const E *__restrict__ B, E *__restrict__ C, double *__restrict__ part) {
   constexpr size_t kBytes = std::max({class_shared<CPLX, 1>(), class_shared<CPLX, 3>(), class_shared<CPLX, 4>(),
                                       class_shared<CPLX, 6>(), sizeof(PanelShared<CPLX>)});
   __shared__ __align__(16) char smem[kBytes];
   const int b = static_cast<int>(blockIdx.x);
-  if (b < x.block0[4]) class_block<CPLX, 6, E>(smem, x, b - x.block0[6], x.count[6]);
-  else if (b < x.block0[1]) class_block<CPLX, 4, E>(smem, x, b - x.block0[4], x.count[4]);
-  else if (b < x.block0[3]) class_block<CPLX, 1, E>(smem, x, b - x.block0[1], x.count[1]);
-  else if (b < x.block0[7]) class_block<CPLX, 3, E>(smem, x, b - x.block0[3], x.count[3]);
+  if (b < x.block0[4])
+    class_block<CPLX, 6, E>(smem, x, b - x.block0[6], x.count[6], x.tiles, x.segs, x.exec, x.ga, x.gb, x.A, x.B, x.C,
+                            x.part);
+  else if (b < x.block0[1])
+    class_block<CPLX, 4, E>(smem, x, b - x.block0[4], x.count[4], tiles, segs, exec, ga, gb, A, B, C, part);
+  else if (b < x.block0[3])
+    class_block<CPLX, 1, E>(smem, x, b - x.block0[1], x.count[1], tiles, segs, exec, ga, gb, A, B, C, part);
+  else if (b < x.block0[7])
+    class_block<CPLX, 3, E>(smem, x, b - x.block0[3], x.count[3], tiles, segs, exec, ga, gb, A, B, C, part);
   else
-    panel_tile<CPLX, STREAM, E>(smem, x.ptiles[b - x.block0[7]], x.pouts, x.pterms, x.segs, x.A, x.B, x.C, x.ar, x.ai,
-                                x.br, x.bi);
+    panel_tile<CPLX, STREAM, E>(smem, x.ptiles[b - x.block0[7]], x.pouts, x.pterms, segs, A, B, C, x.ar, x.ai, x.br,
+                                x.bi);
 }
 // The k-slice sums of reduction items first, first + 1, ...
 template <bool CPLX, typename E>
@@ -1564,7 +1596,10 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
       if (!runs(CLS)) return;
       const hipStream_t ls = stream_of(CLS);
       probe_in(CLS);
-      hipLaunchKernelGGL((k_class<CX, CLS, E>), grid_of(plan->cls_tiles[CLS]), block, 0, ls, x);
+      if constexpr (CLS == kTileRows4)
+        hipLaunchKernelGGL((k_row_class<CX, CLS, E>), grid_of(plan->cls_tiles[CLS]), block, 0, ls, x, x.tiles, x.segs,
+                           x.exec, x.ga, x.gb, x.A, x.B, x.C, x.part);
+      else hipLaunchKernelGGL((k_class<CX, CLS, E>), grid_of(plan->cls_tiles[CLS]), block, 0, ls, x);
       probe_out(CLS);
       // k-sliced tiles: the slices wrote partial sums; one workgroup per sliced
       // tile adds them and applies alpha / beta
@@ -1574,8 +1609,9 @@ qlt_status launch_native_classes(const qlt_plan *plan, int32_t dtype, const void
     one(std::integral_constant<int, kTileNarrowRows>{});
     if (fused) {
       const hipStream_t ls = stream_of(kTileRows4);
-      if (stream_a) hipLaunchKernelGGL((k_all_classes<CX, true, E>), grid_of(blocks), block, 0, ls, x);
-      else hipLaunchKernelGGL((k_all_classes<CX, false, E>), grid_of(blocks), block, 0, ls, x);
+      const auto kernel = stream_a ? k_all_classes<CX, true, E> : k_all_classes<CX, false, E>;
+      hipLaunchKernelGGL(kernel, grid_of(blocks), block, 0, ls, x, x.tiles, x.segs, x.exec, x.ga, x.gb, x.A, x.B, x.C,
+                         x.part);
       if (n_red > 0) hipLaunchKernelGGL((k_reduce<CX, E>), grid_of(n_red), block, 0, ls, x, static_cast<int>(first_red));
       return;
     }
