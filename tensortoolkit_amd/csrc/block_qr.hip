@@ -44,24 +44,30 @@ constexpr int kNB = 16;   // columns per block: one MFMA tile
 struct QrMat {
   int64_t m, n, k;
   int64_t w_off;      // W: m x n, row-major (column-major in k_qr_generic)
-  int64_t v_off;      // block b's reflectors at v_off + b m kNB: m x kNB row-major, rows from b kNB on
-                      // (k_qr_generic: Q, column-major m x k)
+  int64_t v_off;      // block b's kc = min(kNB, k - b kNB) reflectors at v_off + b m kNB: m x kc row-major,
+                      // rows from b kNB on (k_qr_generic: Q, column-major m x k)
   int64_t t_off;      // block b's T at t_off + b kNB kNB (k_qr_generic: tau)
   int64_t a_off, q_off, r_off;
   int32_t blocked;    // 0: the matrix is k_qr_generic's
   int32_t pad;
 };
 
+// Reflectors of block b of a matrix with k of them.
+__device__ __forceinline__ int block_cols(int64_t k, int64_t b) {
+  return static_cast<int>(k - b * kNB < kNB ? k - b * kNB : kNB);
+}
+
 // X <- (I - V op(T) V^H) X for rows r0 .. m - 1 and `nc` columns of X, op(T) =
-// T^H (`CONJT`, applying the adjoint) or T.  V and T are block-reflector
+// T^H (`CONJT`, applying the adjoint) or T.  V (kc columns) and T are block-reflector
 // storage (QrMat), X is row-major with leading dimension ld.
 //   P = V^H X: the rows are the contracted extent; wave w takes k-steps w,
 //   w + W, ... of 4 rows and the waves' partial 16 x 16 sums meet in LDS;
 //   Z = op(T) P, one element per thread;
 //   X -= V Z: wave w takes row blocks w, w + W, ...
-template <bool C, int NW, bool CONJT, typename T>
-__device__ void apply_block(const T *__restrict__ V, const T *__restrict__ Tm, T *X, int64_t ld, int64_t r0, int64_t m,
-                            int nc, T (*sPart)[kNB][kNB + 1], T (*sZ)[kNB + 1], T (*sT)[kNB + 1]) {
+template <bool C, int NW, bool CONJT, bool FULL, typename T>
+__device__ __forceinline__ void apply_cols(const T *__restrict__ V, int cols, const T *__restrict__ Tm, T *X, int64_t ld, int64_t r0,
+                            int64_t m, int nc, T (*sPart)[kNB][kNB + 1], T (*sZ)[kNB + 1], T (*sT)[kNB + 1]) {
+  const int kc = FULL ? kNB : cols;   // a whole block's row stride is a constant
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lk = lane >> 4;
   const int64_t mm = m - r0;
   const int steps = static_cast<int>((mm + 3) / 4);
@@ -74,7 +80,7 @@ __device__ void apply_block(const T *__restrict__ V, const T *__restrict__ Tm, T
     for (int u = 0; u < U; ++u) {
       const int64_t r = r0 + 4 * int64_t(s0 + NW * u) + lk;
       const bool ok = r < m;
-      va[u] = ok ? V[r * kNB + lr] : zero_<T>();
+      va[u] = (ok && lr < kc) ? V[r * kc + lr] : zero_<T>();
       xa[u] = (ok && lr < nc) ? X[r * ld + lr] : zero_<T>();
     }
 #pragma unroll
@@ -121,7 +127,7 @@ __device__ void apply_block(const T *__restrict__ V, const T *__restrict__ Tm, T
     const int64_t rv = r0 + 16 * int64_t(rb) + lr;
     T va[kNB / 4], old[4];
 #pragma unroll
-    for (int s = 0; s < kNB / 4; ++s) va[s] = rv < m ? V[rv * kNB + 4 * s + lk] : zero_<T>();
+    for (int s = 0; s < kNB / 4; ++s) va[s] = (rv < m && 4 * s + lk < kc) ? V[rv * kc + 4 * s + lk] : zero_<T>();
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int64_t r = r0 + 16 * int64_t(rb) + 4 * v + lk;
@@ -148,6 +154,13 @@ __device__ void apply_block(const T *__restrict__ V, const T *__restrict__ Tm, T
       }
     }
   }
+}
+
+template <bool C, int NW, bool CONJT, typename T>
+__device__ __forceinline__ void apply_block(const T *V, int kc, const T *Tm, T *X, int64_t ld, int64_t r0, int64_t m,
+                                            int nc, T (*sPart)[kNB][kNB + 1], T (*sZ)[kNB + 1], T (*sT)[kNB + 1]) {
+  if (kc == kNB) apply_cols<C, NW, CONJT, true>(V, kc, Tm, X, ld, r0, m, nc, sPart, sZ, sT);
+  else apply_cols<C, NW, CONJT, false>(V, kc, Tm, X, ld, r0, m, nc, sPart, sZ, sT);
 }
 
 // Sums over the wave of 16 values per lane: lane l returns the sum of value
@@ -259,7 +272,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
     src = A;
   } else {
     auto *sPart = reinterpret_cast<T (*)[kNB][kNB + 1]>(smem);
-    apply_block<C, NW, true>(static_cast<const T *>(ws_) + mt.v_off + int64_t(b) * m * kNB,
+    apply_block<C, NW, true>(static_cast<const T *>(ws_) + mt.v_off + int64_t(b) * m * kNB, block_cols(k, b),
                              static_cast<const T *>(ws_) + mt.t_off + int64_t(b) * kNB * kNB, W + j0, n,
                              int64_t(b) * kNB, m, nc, sPart, sPart[NW], sPart[NW + 1]);
     if (tile != int64_t(b) + 1 || j0 >= k) return;
@@ -270,7 +283,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
   // A wave's 64 rows pass through LDS so that memory is read and written in
   // runs of kStageCols elements.
   const int64_t mp = m - j0;
-  const int kc = static_cast<int>(k - j0 < kNB ? k - j0 : kNB);
+  const int kc = block_cols(k, tile);
   T x[kNB][RPT];
   auto *sStage = reinterpret_cast<T (*)[kStageCols + 1]>(smem) + 64 * w;
   constexpr int kRowsPerLoad = 64 / kStageCols;
@@ -386,7 +399,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
 #pragma unroll
       for (int q = 0; q < 64; q += kRowsPerLoad) {
         const int64_t i = base + q + srow;
-        if (i < mp) V[(j0 + i) * kNB + c0 + scol] = sStage[q + srow][scol];
+        if (i < mp && c0 + scol < kc) V[(j0 + i) * kc + c0 + scol] = sStage[q + srow][scol];
       }
       wave_lds_sync();
     }
@@ -436,14 +449,14 @@ __global__ void __launch_bounds__(64 * NW) k_qr_q(const QrMat *mats, const void 
   const int nc = static_cast<int>(k - j0 < kNB ? k - j0 : kNB);
   for (int64_t b = blockIdx.y; b >= 0; --b) {
     __syncthreads();
-    apply_block<C, NW, false>(static_cast<const T *>(ws_) + mt.v_off + b * m * kNB,
+    apply_block<C, NW, false>(static_cast<const T *>(ws_) + mt.v_off + b * m * kNB, block_cols(k, b),
                               static_cast<const T *>(ws_) + mt.t_off + b * kNB * kNB, Q + j0, k, b * kNB, m, nc, sPart,
                               sPart[NW], sPart[NW + 1]);
   }
 }
 
-// Matrices with more rows than a panel in registers takes: one workgroup per
-// matrix, unblocked.
+// Matrices with more rows than a panel in registers takes, and small ones: one
+// workgroup per matrix, unblocked.
 template <typename T>
 __device__ __forceinline__ double block_sum(double v, double *red) {
   v = wave_sum(v);
@@ -567,9 +580,30 @@ __global__ void __launch_bounds__(kThreads) k_qr_generic(const QrMat *mats, cons
   }
 }
 
-// Rows a panel in registers takes: 512 threads of 4 (FP64) or 3 (complex) rows.
+// Rows a panel takes: 512 threads of 4 (FP64) or 3 (complex) rows.  Three complex
+// rows do not fit the 256 registers of a thread (111 spill to scratch): 1025 to 1536
+// complex rows run slower than the registers would allow, and still faster than
+// unblocked (one 1200 x 600 matrix 813 -> 6.2 ms, one of 1025 x 17 561 -> 333 us).
 template <bool C>
 constexpr int64_t kMaxBlockedRows = C ? 1536 : 2048;
+
+// Small matrices go to k_qr_generic when the whole call is of them, or when they
+// are many: one workgroup walks their few short columns faster than the launches of
+// the blocked form come and go, and more of them fit a compute unit (us, generic |
+// blocked: one 2 x 2 FP64 28 | 44, one 8 x 8 45 | 45, one 4 x 64 57 | 48, one 1024 x 4
+// 75 | 68; 3000 of 4 x 4 65 | 185, of 12 x 12 184 | 198, of 16 x 16 251 | 205, of 1500 x 1
+// 468 | 908, of 256 x 8 603 | 476; complex128, one 10 x 10 58 | 62, one 1024 x 4 80 | 102, 300 of
+// 12 x 12 81 | 111, of 8 x 64 166 | 131, 3000 of 24 x 24 615 | 1075, of 32 x 32 1248 | 1096).  A
+// few among larger ones are not worth a launch of their own (about 30 us).
+template <bool C>
+constexpr int64_t kManySmall = C ? 256 : 512;
+template <bool C>
+bool small_matrix(int64_t m, int64_t n, int64_t k, int64_t n_mats) {
+  if (C && n_mats >= 1024 && m <= 24 && n <= 24) return true;
+  if (k > 24 || m * k * k > (C ? 16384 : 9216)) return false;
+  if (n_mats < kManySmall<C>) return n <= (C ? 128 : 512) && k * k * n <= (C ? 1000 : 512);
+  return k * k * n <= (C ? 2048 : 1800);
+}
 
 template <bool C>
 qlt_status qr_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, const void *a, const int64_t *a_offsets,
@@ -578,18 +612,25 @@ qlt_status qr_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, con
   std::vector<QrMat> mats(static_cast<size_t>(n_mats));
   int64_t ws = 0, max_rows = 0, max_blocks = 0, max_tiles = 0;
   bool any_generic = false;
+  int64_t n_small = 0;
   for (int64_t i = 0; i < n_mats; ++i) {
     QrMat &mt = mats[static_cast<size_t>(i)];
     mt.m = rows[i];
     mt.n = cols[i];
     mt.k = std::min(rows[i], cols[i]);
-    mt.blocked = mt.m <= kMaxBlockedRows<C> && (mt.n + kNB - 1) / kNB <= 65535;
+    mt.blocked = !small_matrix<C>(mt.m, mt.n, mt.k, n_mats);
+    n_small += !mt.blocked;
+  }
+  const bool small_apart = n_small == n_mats || n_small >= kManySmall<C>;
+  for (int64_t i = 0; i < n_mats; ++i) {
+    QrMat &mt = mats[static_cast<size_t>(i)];
+    mt.blocked = (mt.blocked || !small_apart) && mt.m <= kMaxBlockedRows<C> && (mt.n + kNB - 1) / kNB <= 65535;
     mt.pad = 0;
     const int64_t nb = (mt.k + kNB - 1) / kNB;
     mt.w_off = ws;
     ws += mt.m * mt.n;
     mt.v_off = ws;
-    ws += mt.blocked ? nb * mt.m * kNB : mt.m * mt.k;
+    ws += mt.m * mt.k;
     mt.t_off = ws;
     ws += mt.blocked ? nb * kNB * kNB : mt.k;
     mt.a_off = a_offsets[i];
