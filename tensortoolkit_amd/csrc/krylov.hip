@@ -151,9 +151,14 @@ __device__ __forceinline__ double sweep(int64_t n, int i0, int m, const double *
 // The narrowest sweep over the vectors left: loads and sums of vectors past
 // the count are not free (2 products of 10^6 complex elements in a sweep of 8:
 // 15.7 us, of 2: 12.2).
+// An update in FP64 by up to half as many vectors again as kSweep takes them in
+// halves for the same reason: by 17 vectors of 3 * 10^6 elements 92.9 -> 87.8 us,
+// by 20 of 2 * 10^5 7.5 -> 6.6 (complex, and more vectors: no difference).
 template <bool CPLX, bool UPDATE, bool DOT, bool NORM>
 __device__ __forceinline__ double sweep_of(int64_t n, int i0, int m, const double *s_c, const double *__restrict__ V,
                                            int64_t ldv, double *__restrict__ w, double *work, double (*s_red)[4]) {
+  if (UPDATE && !DOT && !CPLX && m > kSweep && m <= kSweep + kSweep / 2)
+    return sweep<CPLX, kSweep / 2, UPDATE, DOT, NORM>(n, i0, m, s_c, V, ldv, w, work, s_red);
   if (m - i0 <= kSweep / 8)
     return sweep<CPLX, kSweep / 8, UPDATE, DOT, NORM>(n, i0, m, s_c, V, ldv, w, work, s_red);
   if (m - i0 <= kSweep / 4)
@@ -240,7 +245,7 @@ __global__ __launch_bounds__(256) void k_basis_update_dot(int64_t n, int32_t k_m
   if (m <= kSweep) {
     sweep_of<CPLX, true, true, false>(n, 0, m, s_c, V, ldv, w, work, s_red);
   } else {
-    sweep<CPLX, kSweep, true, false, false>(n, 0, m, s_c, V, ldv, w, nullptr, nullptr);
+    sweep_of<CPLX, true, false, false>(n, 0, m, s_c, V, ldv, w, nullptr, nullptr);
     dot_sweeps<CPLX>(n, m, V, ldv, w, work, s_red);
   }
 }
