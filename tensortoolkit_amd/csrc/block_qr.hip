@@ -44,12 +44,10 @@ constexpr int kNB = 16;   // columns per block: one MFMA tile
 struct QrMat {
   int64_t m, n, k;
   int64_t w_off;      // W: m x n, row-major (column-major in k_qr_generic)
-  int64_t v_off;      // block b's kc = min(kNB, k - b kNB) reflectors at v_off + b m kNB: m x kc row-major,
-                      // rows from b kNB on (k_qr_generic: Q, column-major m x k)
+  int64_t v_off;      // block b's reflectors at v_off + b m kNB: m x v_cols row-major, rows from b kNB on
+                      // (k_qr_generic: Q, column-major m x k)
   int64_t t_off;      // block b's T at t_off + b kNB kNB (k_qr_generic: tau)
   int64_t a_off, q_off, r_off;
-  int32_t blocked;    // 0: the matrix is k_qr_generic's
-  int32_t pad;
 };
 
 // Reflectors of block b of a matrix with k of them.
@@ -57,17 +55,25 @@ __device__ __forceinline__ int block_cols(int64_t k, int64_t b) {
   return static_cast<int>(k - b * kNB < kNB ? k - b * kNB : kNB);
 }
 
+// Row stride of block b's reflectors: with PAD the last block, too, takes kNB
+// columns (zeros past k), and the stride is a constant.  Padding is faster (U(1)
+// D = 1024, FP64: 656 us, 672 without) and costs a matrix of few columns a multiple
+// of its size in scratch, so qr_impl takes it where that is little.
+template <bool PAD>
+__device__ __forceinline__ int v_cols(int64_t k, int64_t b) {
+  return PAD ? kNB : block_cols(k, b);
+}
+
 // X <- (I - V op(T) V^H) X for rows r0 .. m - 1 and `nc` columns of X, op(T) =
-// T^H (`CONJT`, applying the adjoint) or T.  V (kc columns) and T are block-reflector
+// T^H (`CONJT`, applying the adjoint) or T.  V (row stride ldv) and T are block-reflector
 // storage (QrMat), X is row-major with leading dimension ld.
 //   P = V^H X: the rows are the contracted extent; wave w takes k-steps w,
 //   w + W, ... of 4 rows and the waves' partial 16 x 16 sums meet in LDS;
 //   Z = op(T) P, one element per thread;
 //   X -= V Z: wave w takes row blocks w, w + W, ...
-template <bool C, int NW, bool CONJT, bool FULL, typename T>
-__device__ __forceinline__ void apply_cols(const T *__restrict__ V, int cols, const T *__restrict__ Tm, T *X, int64_t ld, int64_t r0,
+template <bool C, int NW, bool CONJT, bool PAD, typename T>
+__device__ void apply_block(const T *__restrict__ V, int ldv, const T *__restrict__ Tm, T *X, int64_t ld, int64_t r0,
                             int64_t m, int nc, T (*sPart)[kNB][kNB + 1], T (*sZ)[kNB + 1], T (*sT)[kNB + 1]) {
-  const int kc = FULL ? kNB : cols;   // a whole block's row stride is a constant
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lk = lane >> 4;
   const int64_t mm = m - r0;
   const int steps = static_cast<int>((mm + 3) / 4);
@@ -80,7 +86,7 @@ __device__ __forceinline__ void apply_cols(const T *__restrict__ V, int cols, co
     for (int u = 0; u < U; ++u) {
       const int64_t r = r0 + 4 * int64_t(s0 + NW * u) + lk;
       const bool ok = r < m;
-      va[u] = (ok && lr < kc) ? V[r * kc + lr] : zero_<T>();
+      va[u] = (ok && (PAD || lr < ldv)) ? V[r * ldv + lr] : zero_<T>();
       xa[u] = (ok && lr < nc) ? X[r * ld + lr] : zero_<T>();
     }
 #pragma unroll
@@ -127,7 +133,8 @@ __device__ __forceinline__ void apply_cols(const T *__restrict__ V, int cols, co
     const int64_t rv = r0 + 16 * int64_t(rb) + lr;
     T va[kNB / 4], old[4];
 #pragma unroll
-    for (int s = 0; s < kNB / 4; ++s) va[s] = (rv < m && 4 * s + lk < kc) ? V[rv * kc + 4 * s + lk] : zero_<T>();
+    for (int s = 0; s < kNB / 4; ++s)
+      va[s] = (rv < m && (PAD || 4 * s + lk < ldv)) ? V[rv * ldv + 4 * s + lk] : zero_<T>();
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int64_t r = r0 + 16 * int64_t(rb) + 4 * v + lk;
@@ -154,13 +161,6 @@ __device__ __forceinline__ void apply_cols(const T *__restrict__ V, int cols, co
       }
     }
   }
-}
-
-template <bool C, int NW, bool CONJT, typename T>
-__device__ __forceinline__ void apply_block(const T *V, int kc, const T *Tm, T *X, int64_t ld, int64_t r0, int64_t m,
-                                            int nc, T (*sPart)[kNB][kNB + 1], T (*sZ)[kNB + 1], T (*sT)[kNB + 1]) {
-  if (kc == kNB) apply_cols<C, NW, CONJT, true>(V, kc, Tm, X, ld, r0, m, nc, sPart, sZ, sT);
-  else apply_cols<C, NW, CONJT, false>(V, kc, Tm, X, ld, r0, m, nc, sPart, sZ, sT);
 }
 
 // Sums over the wave of 16 values per lane: lane l returns the sum of value
@@ -243,7 +243,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Launch b of the factorisation, grid (matrices, column tiles b + 1 ..).
 // FIRST (b = -1): the tiles are copied from the input into W, and tile 0 is
 // factored.  Rows up to 64 NW RPT.
-template <bool C, int NW, int RPT, bool FIRST>
+template <bool C, int NW, int RPT, bool FIRST, bool PAD>
 __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t b, const void *a_, void *ws_) {
   using T = typename ElemOf<C>::T;
   constexpr int TH = 64 * NW;
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
   const int64_t m = mt.m, n = mt.n, k = mt.k;
   const int64_t tile = FIRST ? int64_t(blockIdx.y) : int64_t(b) + 1 + blockIdx.y;
   const int64_t j0 = tile * kNB;
-  if (!mt.blocked || j0 >= n || int64_t(b) * kNB >= k) return;
+  if (j0 >= n || int64_t(b) * kNB >= k) return;
   const int nc = static_cast<int>(n - j0 < kNB ? n - j0 : kNB);
   T *W = static_cast<T *>(ws_) + mt.w_off;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
     src = A;
   } else {
     auto *sPart = reinterpret_cast<T (*)[kNB][kNB + 1]>(smem);
-    apply_block<C, NW, true>(static_cast<const T *>(ws_) + mt.v_off + int64_t(b) * m * kNB, block_cols(k, b),
+    apply_block<C, NW, true, PAD>(static_cast<const T *>(ws_) + mt.v_off + int64_t(b) * m * kNB, v_cols<PAD>(k, b),
                              static_cast<const T *>(ws_) + mt.t_off + int64_t(b) * kNB * kNB, W + j0, n,
                              int64_t(b) * kNB, m, nc, sPart, sPart[NW], sPart[NW + 1]);
     if (tile != int64_t(b) + 1 || j0 >= k) return;
@@ -384,6 +384,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
   }
   const int64_t pb = FIRST ? 0 : int64_t(b) + 1;
   T *V = static_cast<T *>(ws_) + mt.v_off + pb * m * kNB;
+  const int ldv = v_cols<PAD>(k, pb);
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
     const int64_t base = 64 * w + int64_t(TH) * r;
@@ -399,7 +400,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
 #pragma unroll
       for (int q = 0; q < 64; q += kRowsPerLoad) {
         const int64_t i = base + q + srow;
-        if (i < mp && c0 + scol < kc) V[(j0 + i) * kc + c0 + scol] = sStage[q + srow][scol];
+        if (i < mp && (PAD || c0 + scol < kc)) V[(j0 + i) * ldv + c0 + scol] = sStage[q + srow][scol];
       }
       wave_lds_sync();
     }
@@ -427,7 +428,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_step(const QrMat *mats, int32_t 
 // R and Q, grid (matrices, column tiles): columns j0 .. of R, and the same
 // columns of Q = H_0 ... H_{k-1} I, the blocks applied from the tile's own
 // one back to the first (a later block acts on rows where the tile is zero).
-template <bool C, int NW>
+template <bool C, int NW, bool PAD>
 __global__ void __launch_bounds__(64 * NW) k_qr_q(const QrMat *mats, const void *ws_, void *q_, void *r_) {
   using T = typename ElemOf<C>::T;
   constexpr int TH = 64 * NW;
@@ -435,7 +436,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_q(const QrMat *mats, const void 
   const QrMat mt = mats[blockIdx.x];
   const int64_t m = mt.m, n = mt.n, k = mt.k;
   const int64_t j0 = int64_t(blockIdx.y) * kNB;
-  if (!mt.blocked || j0 >= n) return;
+  if (j0 >= n) return;
   const int c = threadIdx.x % kNB;
   const T *W = static_cast<const T *>(ws_) + mt.w_off;
   T *R = static_cast<T *>(r_) + mt.r_off;
@@ -449,7 +450,7 @@ __global__ void __launch_bounds__(64 * NW) k_qr_q(const QrMat *mats, const void 
   const int nc = static_cast<int>(k - j0 < kNB ? k - j0 : kNB);
   for (int64_t b = blockIdx.y; b >= 0; --b) {
     __syncthreads();
-    apply_block<C, NW, false>(static_cast<const T *>(ws_) + mt.v_off + b * m * kNB, block_cols(k, b),
+    apply_block<C, NW, false, PAD>(static_cast<const T *>(ws_) + mt.v_off + b * m * kNB, v_cols<PAD>(k, b),
                               static_cast<const T *>(ws_) + mt.t_off + b * kNB * kNB, Q + j0, k, b * kNB, m, nc, sPart,
                               sPart[NW], sPart[NW + 1]);
   }
@@ -473,7 +474,6 @@ __global__ void __launch_bounds__(kThreads) k_qr_generic(const QrMat *mats, cons
   __shared__ double sRed[kWaves];
   __shared__ T sTau, sScale;
   const QrMat mt = mats[blockIdx.x];
-  if (mt.blocked) return;
   const T *A = static_cast<const T *>(a_) + mt.a_off;
   T *Wm = static_cast<T *>(ws_) + mt.w_off;
   T *Qw = static_cast<T *>(ws_) + mt.v_off;
@@ -591,15 +591,16 @@ constexpr int64_t kMaxBlockedRows = C ? 1536 : 2048;
 // are many: one workgroup walks their few short columns faster than the launches of
 // the blocked form come and go, and more of them fit a compute unit (us, generic |
 // blocked: one 2 x 2 FP64 28 | 44, one 8 x 8 45 | 45, one 4 x 64 57 | 48, one 1024 x 4
-// 75 | 68; 3000 of 4 x 4 65 | 185, of 12 x 12 184 | 198, of 16 x 16 251 | 205, of 1500 x 1
-// 468 | 908, of 256 x 8 603 | 476; complex128, one 10 x 10 58 | 62, one 1024 x 4 80 | 102, 300 of
-// 12 x 12 81 | 111, of 8 x 64 166 | 131, 3000 of 24 x 24 615 | 1075, of 32 x 32 1248 | 1096).  A
-// few among larger ones are not worth a launch of their own (about 30 us).
+// 75 | 68; 3000 of 4 x 4 65 | 185, of 12 x 12 184 | 198, of 16 x 16 251 | 205, of
+// 1500 x 1 468 | 908, of 256 x 8 603 | 476; complex128, one 10 x 10 58 | 62, one
+// 1024 x 4 80 | 102, 300 of 12 x 12 81 | 111, of 8 x 64 166 | 131, 1000 of 16 x 16
+// 159 | 186, 3000 of 24 x 24 615 | 1075, of 32 x 32 1248 | 1096).  A few among larger
+// ones are not worth a launch of their own (about 30 us).
 template <bool C>
 constexpr int64_t kManySmall = C ? 256 : 512;
 template <bool C>
 bool small_matrix(int64_t m, int64_t n, int64_t k, int64_t n_mats) {
-  if (C && n_mats >= 1024 && m <= 24 && n <= 24) return true;
+  if (C && n_mats >= 512 && m <= 24 && n <= 24) return true;
   if (k > 24 || m * k * k > (C ? 16384 : 9216)) return false;
   if (n_mats < kManySmall<C>) return n <= (C ? 128 : 512) && k * k * n <= (C ? 1000 : 512);
   return k * k * n <= (C ? 2048 : 1800);
@@ -609,39 +610,45 @@ template <bool C>
 qlt_status qr_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, const void *a, const int64_t *a_offsets,
                    void *q, const int64_t *q_offsets, void *r, const int64_t *r_offsets, hipStream_t st) {
   const size_t esz = C ? 16 : 8;
-  std::vector<QrMat> mats(static_cast<size_t>(n_mats));
-  int64_t ws = 0, max_rows = 0, max_blocks = 0, max_tiles = 0;
-  bool any_generic = false;
   int64_t n_small = 0;
+  for (int64_t i = 0; i < n_mats; ++i) n_small += small_matrix<C>(rows[i], cols[i], std::min(rows[i], cols[i]), n_mats);
+  const bool all_small = n_small == n_mats, small_apart = all_small || n_small >= kManySmall<C>;
+  const auto is_blocked = [&](int64_t m, int64_t n, int64_t k) {
+    return !all_small && m <= kMaxBlockedRows<C> && (n + kNB - 1) / kNB <= 65535 &&
+           !(small_apart && small_matrix<C>(m, n, k, n_mats));
+  };
+  int64_t n_blocked = 0, compact = 0, padding = 0;   // elements of scratch
+  for (int64_t i = 0; i < n_mats && !all_small; ++i) {
+    const int64_t m = rows[i], n = cols[i], k = std::min(m, n);
+    compact += m * (n + k);
+    if (!is_blocked(m, n, k)) continue;
+    ++n_blocked;
+    padding += m * ((k + kNB - 1) / kNB * kNB - k);
+  }
+  const bool pad = padding <= compact / 4;
+  // the blocked matrices, then k_qr_generic's
+  std::vector<QrMat> mats(static_cast<size_t>(n_mats));
+  int64_t ws = 0, max_rows = 0, max_blocks = 0, max_tiles = 0, at_blocked = 0, at_generic = n_blocked;
   for (int64_t i = 0; i < n_mats; ++i) {
-    QrMat &mt = mats[static_cast<size_t>(i)];
+    const bool blocked = is_blocked(rows[i], cols[i], std::min(rows[i], cols[i]));
+    QrMat &mt = mats[static_cast<size_t>(blocked ? at_blocked++ : at_generic++)];
     mt.m = rows[i];
     mt.n = cols[i];
     mt.k = std::min(rows[i], cols[i]);
-    mt.blocked = !small_matrix<C>(mt.m, mt.n, mt.k, n_mats);
-    n_small += !mt.blocked;
-  }
-  const bool small_apart = n_small == n_mats || n_small >= kManySmall<C>;
-  for (int64_t i = 0; i < n_mats; ++i) {
-    QrMat &mt = mats[static_cast<size_t>(i)];
-    mt.blocked = (mt.blocked || !small_apart) && mt.m <= kMaxBlockedRows<C> && (mt.n + kNB - 1) / kNB <= 65535;
-    mt.pad = 0;
     const int64_t nb = (mt.k + kNB - 1) / kNB;
     mt.w_off = ws;
     ws += mt.m * mt.n;
     mt.v_off = ws;
-    ws += mt.m * mt.k;
+    ws += mt.m * (blocked && pad ? nb * kNB : mt.k);
     mt.t_off = ws;
-    ws += mt.blocked ? nb * kNB * kNB : mt.k;
+    ws += blocked ? nb * kNB * kNB : mt.k;
     mt.a_off = a_offsets[i];
     mt.q_off = q_offsets[i];
     mt.r_off = r_offsets[i];
-    if (mt.blocked) {
+    if (blocked) {
       max_rows = std::max(max_rows, mt.m);
       max_blocks = std::max(max_blocks, nb);
       max_tiles = std::max(max_tiles, (mt.n + kNB - 1) / kNB);
-    } else {
-      any_generic = true;
     }
   }
   DevBuf d_ws, d_mats;
@@ -649,24 +656,32 @@ qlt_status qr_impl(int64_t n_mats, const int64_t *rows, const int64_t *cols, con
   QLT_HIP(hipMalloc(&d_mats.p, sizeof(QrMat) * mats.size()));
   QLT_HIP(hipMemcpyAsync(d_mats.p, mats.data(), sizeof(QrMat) * mats.size(), hipMemcpyHostToDevice, st));
   const auto *dm = static_cast<const QrMat *>(d_mats.p);
-  const unsigned gm = static_cast<unsigned>(n_mats);
-  if (any_generic) hipLaunchKernelGGL(k_qr_generic<C>, dim3(gm), dim3(kThreads), 0, st, dm, a, d_ws.p, q, r);
-  auto blocked = [&](auto nw_tag, auto rpt_tag) {
+  const unsigned gm = static_cast<unsigned>(n_blocked);
+  if (n_blocked < n_mats)
+    hipLaunchKernelGGL(k_qr_generic<C>, dim3(static_cast<unsigned>(n_mats - n_blocked)), dim3(kThreads), 0, st,
+                       dm + n_blocked, a, d_ws.p, q, r);
+  auto launch_pad = [&](auto nw_tag, auto rpt_tag, auto pad_tag) {
     constexpr int NW = decltype(nw_tag)::value, RPT = decltype(rpt_tag)::value;
-    hipLaunchKernelGGL((k_qr_step<C, NW, RPT, true>), dim3(gm, static_cast<unsigned>(max_tiles)), dim3(64 * NW), 0, st,
+    constexpr bool PAD = decltype(pad_tag)::value;
+    hipLaunchKernelGGL((k_qr_step<C, NW, RPT, true, PAD>), dim3(gm, static_cast<unsigned>(max_tiles)), dim3(64 * NW), 0, st,
                        dm, -1, a, d_ws.p);
     for (int64_t b = 0; b + 1 < max_tiles && b < max_blocks; ++b)
-      hipLaunchKernelGGL((k_qr_step<C, NW, RPT, false>), dim3(gm, static_cast<unsigned>(max_tiles - b - 1)),
+      hipLaunchKernelGGL((k_qr_step<C, NW, RPT, false, PAD>), dim3(gm, static_cast<unsigned>(max_tiles - b - 1)),
                          dim3(64 * NW), 0, st, dm, static_cast<int32_t>(b), a, d_ws.p);
+    hipLaunchKernelGGL((k_qr_q<C, 4, PAD>), dim3(gm, static_cast<unsigned>(max_tiles)), dim3(256), 0, st, dm, d_ws.p, q,
+                       r);
+  };
+  auto launch = [&](auto nw_tag, auto rpt_tag) {
+    if (pad) launch_pad(nw_tag, rpt_tag, std::true_type{});
+    else launch_pad(nw_tag, rpt_tag, std::false_type{});
   };
   using std::integral_constant;
   if (max_tiles > 0) {
     // the fewest waves whose registers hold the tallest panel: a column costs
     // every wave its own reduction
-    if (max_rows <= 512) blocked(integral_constant<int, 4>{}, integral_constant<int, 2>{});
-    else if (max_rows <= 1024) blocked(integral_constant<int, 8>{}, integral_constant<int, 2>{});
-    else blocked(integral_constant<int, 8>{}, integral_constant<int, C ? 3 : 4>{});
-    hipLaunchKernelGGL((k_qr_q<C, 4>), dim3(gm, static_cast<unsigned>(max_tiles)), dim3(256), 0, st, dm, d_ws.p, q, r);
+    if (max_rows <= 512) launch(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+    else if (max_rows <= 1024) launch(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+    else launch(integral_constant<int, 8>{}, integral_constant<int, C ? 3 : 4>{});
   }
   QLT_HIP(hipGetLastError());
   QLT_HIP(hipStreamSynchronize(st));
