@@ -15,8 +15,10 @@ tuned and built-in chains measure within run-to-run spread of each other).
 
 The JSON line reports the split-BF16 path (``value``) next to the native
 FP64 path; the roofline of the dominant kernel (the library's kernel probe
-records HIP events around that one kernel launch, on its launch stream,
-in every timed step); the error of the step's output against the FP64 CPU
+records HIP events around that one kernel launch, on its launch stream, in
+steps of their own after the timed ones; a native tile class, which shares
+one launch with the others in the timed steps, has a launch of its own
+there); the error of the step's output against the FP64 CPU
 oracle; and the CPU baseline: the oracle (the reference algorithm restated
 in C, OpenBLAS zgemm per task) on a bounded sample.
 """
@@ -281,6 +283,8 @@ def kernel_roofline(kernel: dict, workload: str) -> dict:
     traffic, src = profile_traffic(kernel["name"], workload)
     out = {"kernel": kernel["name"], "ms_per_launch": round(kernel["ms"], 5),
            "algorithmic_flops": kernel["flops"], "algorithmic_bytes": kernel["bytes"]}
+    if not split and not split_i8:
+        out["launch"] = "the tile class in a launch of its own; the timed steps run all tile classes in one"
     if rows:
         gbs = kernel["bytes"] / secs / 1e9
         out.update(bound="hbm", achieved=round(gbs, 1), peak=PEAK_HBM_GBS, unit="GB/s",

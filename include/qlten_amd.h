@@ -195,7 +195,7 @@ qlt_status qlt_set_split_min_mean_k(double min_mean_k);
 double qlt_get_split_min_mean_k(void);
 
 /* Row panels (default on, 1), read when a plan is built: the narrow output
- * blocks (n <= 4, contracted extent <= 64) that share their coordinates on A's
+ * blocks (n <= 4) that share their coordinates on A's
  * saved axes, and together read at most 4 contracted columns of A', run as one
  * unit that reads each A element once for all of them.  0 keeps every such block
  * on the per-block row kernel.  The values are bitwise the same either way
@@ -213,9 +213,10 @@ int32_t qlt_get_row_panels(void);
  * 1: 32x64, 2: 64x32, 3: 32x32; -1: the built-in rule, which takes 32 in a
  * dimension when that pads at most 9/10 as much as 64).  slice_target[c] is the
  * workgroup count that k-slicing of tile class c aims at (0: the built-in
- * 512 for the MFMA classes 0-3, 2048 for classes 4 and 5, the narrow
- * outputs).  A plan keeps
- * the tuning in effect when it was built. */
+ * 512 for classes 0-3, 2048 for the narrow outputs, of which class 4 is one
+ * thread per row of n <= 4 columns and class 5 the 16-column MFMA tiles,
+ * whether one wave or four take a tile).  A plan keeps the tuning in effect
+ * when it was built. */
 #define QLT_TUNE_BUCKETS 16
 #define QLT_TILE_CLASSES 6
 typedef struct {
@@ -257,9 +258,10 @@ qlt_status qlt_autotune(int32_t n_items, const qlt_tune_item *items, int32_t dty
  * With both events non-null (hipEvent_t created on the current device),
  * every later qlt_contract_execute outside graph capture records
  * `start_event` on its stream just before the launch of its dominant kernel
- * (the tile-class kernel, or the split GEMM, with the most algorithmic
- * flops) and `stop_event` just after it.  qlt_kernel_probe_last returns that
- * kernel's name, its algorithmic flops (sum of c*m*k*n, c = 2 real or 8
+ * (the tile class, or the split GEMM, with the most algorithmic flops) and
+ * `stop_event` just after it.  For that the tile classes, which otherwise
+ * share one launch, get a launch each; qlt_kernel_probe_last returns the name
+ * of the class's, its algorithmic flops (sum of c*m*k*n, c = 2 real or 8
  * complex) and its compulsory bytes (distinct A and B blocks it reads plus
  * the C elements it writes).  Null events disarm the probe.  Process-wide;
  * meant for one measuring thread. */

@@ -161,7 +161,7 @@ __host__ __device__ inline void magic_of(uint32_t d, uint64_t &mag, int32_t &sh)
 // kTileRows4: narrow outputs (n <= 4) on a row-streaming path, 1024 output
 // rows per workgroup (4 per thread).  n <= 16: MFMA tiles of 32 rows, of which
 // a workgroup takes one, its contracted extent spread over the four waves
-// (kTileNarrow), or four, one per wave (kTileNarrowRows).  choose_narrow_class
+// (kTileNarrow), or four, one per wave (kTileNarrowRows).  choose_narrow_classes
 // (plan.hip) says which of the three a narrow block takes.
 constexpr int32_t kTileMfma = 0;       // 64 x 64 (first MFMA class)
 constexpr int32_t kNumMfmaClasses = 4;
